@@ -250,8 +250,15 @@ def rows_served(K: int, batch: int) -> bool:
     return ROWS_BATCH[0] <= batch <= ROWS_BATCH[1] and 1024 <= K <= 6144 and K % 512 == 0
 
 
+def _only_matmuls_read(graph: Graph, tensor: str, planned: set) -> bool:
+    """Whether ``tensor`` has readers and every one is a matmul of the partition being compiled (node ids ``planned``) that takes
+    it as its activation: then nothing misses the tensor when its producer leaves it as Q8_1 blocks alone."""
+    readers = graph.tensors[tensor].consumers
+    return bool(readers) and all(c.op == "gemm" and c.inputs[0].tensorName == tensor and c.id in planned for c in readers)
+
+
 def _group_plan(graph: Graph, grp: list, batch: int, device_scalars: bool, q8_of: dict, attn_exact: bool = True,
-                raw_of: dict | None = None) -> KernelPlan:
+                raw_of: dict | None = None, planned: set = frozenset()) -> KernelPlan:
     """The fused op spec and slot list for a multi-node group (see fusedPartition)."""
     ops = tuple(n.op for n in grp)
     bpart = f" batch={batch}" if batch != 1 else ""
@@ -279,7 +286,7 @@ def _group_plan(graph: Graph, grp: list, batch: int, device_scalars: bool, q8_of
             aux = sw.outputs[0].tensorName + ".q8_1"
             q8_of[sw.outputs[0].tensorName] = aux
             return KernelPlan(spec + " q8out=1", name, args + [aux], [1, 1, 1], grp, {aux: batch * (N // 32) * 36})
-        if rows_served(N, batch) and K in (1024, 2048) and all(c.op == "gemm" for c in graph.tensors[sw.outputs[0].tensorName].consumers):
+        if rows_served(N, batch) and K in (1024, 2048) and _only_matmuls_read(graph, sw.outputs[0].tensorName, planned):
             # a few sequences: the activation is only ever read by the down projection, which takes it as Q8_1
             aux = sw.outputs[0].tensorName + ".q8_1"
             q8_of[sw.outputs[0].tensorName] = aux
@@ -348,10 +355,11 @@ def compilePartition(graph: Graph, ordered: Partition, batch: int = 1, device_sc
     q8_of: dict[str, str] = {}
     raw_of: dict[str, tuple] = {}       # output of a gdn_delta_rule node in slab form -> (its raw block, its norm weight)
     in_conv_group = {n.outputs[0].tensorName for grp in ordered if len(grp) == 6 for n in grp if n.op == "conv1d_decode"}
+    planned = {n.id for grp in ordered for n in grp}
     plans = []
     for grp in ordered:
         if len(grp) != 1:
-            plans.append(_group_plan(graph, grp, batch, device_scalars, q8_of, attn_exact, raw_of))
+            plans.append(_group_plan(graph, grp, batch, device_scalars, q8_of, attn_exact, raw_of, planned))
             continue
         n = grp[0]
         args = [i.tensorName for i in n.inputs] + [o.tensorName for o in n.outputs]

@@ -1,6 +1,7 @@
 """Host logic without a GPU: the decode graph has the reference's shape (node count, op sequence,
 slot order per op), the runner orders it correctly, and the CPU checker runs a tiny model."""
 import numpy as np
+import pytest
 
 from bunker_amd import model, runner, synth_model
 from bunker_amd.model import REFERENCE, SYNTH, TINY
@@ -169,6 +170,58 @@ def test_fused_partition_groups_and_specs():
     # residual of the fused matmul + cast + add is the add's other input
     down = next(p for p in plans if p.spec.startswith("gemv_fused K=6144"))
     assert g.t(down.args[2]).producer.op == "add" and g.t(down.args[3]).producer.op == "add"
+
+
+def _mlp_graph(batch, tail):
+    """norm + gate + up + swiglu at H = 1024, INTER = 3584, and what ``tail(graph, swiglu output)`` puts behind it."""
+    from bunker_amd.graph import Graph, row_major
+    H, F = 1024, 3584
+    g = Graph()
+    x = g.input("x", row_major([batch, H], "bf16"))
+    nw = g.input("nw", row_major([H], "bf16"), "weight")
+    wg, wu = (g.input(n, row_major([F, H], "q4_k"), "weight") for n in ("Wg", "Wu"))
+    n = g.node("rmsnorm", [(x, "x"), (nw, "w")], [("out", row_major([batch, H], "bf16"))], [1, 1, 1], {"N": H})
+    gu = [g.node("gemm", [(g.out(n), "x"), (w, "w")], [("out", row_major([batch, F], "f32"))], [1, 1, 1], {"N": F, "K": H}) for w in (wg, wu)]
+    sw = g.node("swiglu", [(g.out(gu[0]), "g"), (g.out(gu[1]), "u")], [("out", row_major([batch, F], "bf16"))], [1, 1, 1], {"N": F})
+    tail(g, g.out(sw))
+    return g, g.out(sw)
+
+
+def _down(g, act, name="Wd", weight=None):
+    from bunker_amd.graph import row_major
+    batch, F = g.t(act).type.shape
+    w = weight or g.input(name, row_major([1024, F], "q4_k"), "weight")
+    return g.node("gemm", [(act, "x"), (w, "w")], [("out", row_major([batch, 1024], "f32"))], [1, 1, 1], {"N": 1024, "K": F})
+
+
+@pytest.mark.parametrize("batch", [2, 5, 7])
+def test_the_swiglu_result_is_left_out_only_when_matmuls_of_the_partition_read_all_of_it(batch):
+    """q8only=1 writes no bf16 activation.  Without a reader (the graph ends there), with a reader that is no matmul, with one that
+    takes it as its weight, and with one outside of the partition being compiled, the bf16 tensor has to be written."""
+    from bunker_amd.graph import row_major
+
+    def plan(tail, drop=()):
+        g, act = _mlp_graph(batch, tail)
+        part = [grp for grp in runner.fusedPartition(g) if not any(n.id in drop for n in grp)]
+        plans = runner.compilePartition(g, runner.topoOrder(g, part), batch)
+        return next(p for p in plans if "swiglu=1" in p.spec), plans, act
+
+    def weight_of_another(g, act):
+        y = g.input("y", row_major([batch, 3584], "bf16"))
+        _down(g, y.name, weight=g.t(act))
+
+    bf16_readers = {
+        "none": (lambda g, act: None, ()),
+        "cast": (lambda g, act: (_down(g, act), g.node("cast", [(act, "x")], [("out", row_major([batch, 3584], "bf16"))], [1, 1, 1], {"N": 3584})), ()),
+        "weight": (weight_of_another, ()),
+        "outside": (lambda g, act: (_down(g, act, "Wd0"), _down(g, act, "Wd1")), (5,)),
+    }
+    for what, (tail, drop) in bf16_readers.items():
+        sw, _, act = plan(tail, drop)
+        assert "q8only" not in sw.spec and sw.args[-1] == act and not sw.aux, what
+    sw, plans, act = plan(lambda g, a: (_down(g, a, "Wd0"), _down(g, a, "Wd1")))
+    assert sw.spec.endswith("q8only=1") and list(sw.aux) == [sw.args[-1]]
+    assert sum(p.args[0] == sw.args[-1] and " pro=0 " in p.spec for p in plans) == 2
 
 
 class _NoDeviceEnv:

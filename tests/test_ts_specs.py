@@ -135,3 +135,14 @@ def test_ts_constants_and_exports():
     assert runner.tensor_bytes(g.t("model.layers.3.kv_k_in")) == sizes["kv_k"]
     for expr in ("batch * 3 * QKVD * 2", "batch * D.LVH * D.LKD * D.LVD * 4", "batch * D.NKV * D.MAX_LEN * D.HD * 2"):
         assert expr in TS, expr
+
+
+def test_ts_leaves_the_swiglu_result_out_only_when_matmuls_read_all_of_it():
+    """runner._only_matmuls_read in TypeScript: no readers known, none there, or one outside of the partition means the bf16 form."""
+    body = re.search(r"^function onlyMatmulsRead\(.*?\{\n(.*?)^\}", TS, flags=re.M | re.S).group(1)
+    for term in ("readers?.get(tensor)?.consumers ?? []", "consumers.length > 0 &&", 'c.op === "gemm"', "tn(c.inputs[0]) === tensor",
+                 "planned !== undefined && planned.has(c.id)"):
+        assert term in body, term
+    guards = [l for l in TS.splitlines() if "rowsServed(N, batch)" in l and l.lstrip().startswith("if")]
+    assert len(guards) == 1 and "onlyMatmulsRead(tn(sw.outputs[0]), readers, planned)" in guards[0]
+    assert TS.count("graph.tensors, planned)") == 1

@@ -96,9 +96,16 @@ export function nodeSpec(n: GraphNode, batch = 1, deviceScalars = false, attnExa
 
 const tn = (io: NodeIO) => io.tensorName;
 
+/** Whether `tensor` has readers and every one is a matmul of the partition being compiled (node ids `planned`) that takes it as
+ * its activation.  Without that knowledge (no `readers`, no `planned`) the answer is no, and the bf16 tensor is written. */
+function onlyMatmulsRead(tensor: string, readers?: Graph["tensors"], planned?: Set<number>): boolean {
+  const consumers = readers?.get(tensor)?.consumers ?? [];
+  return consumers.length > 0 && consumers.every((c) => c.op === "gemm" && tn(c.inputs[0]) === tensor && planned !== undefined && planned.has(c.id));
+}
+
 /** Spec and slot list of a fused group (the counterpart of codegenGroup for the groups fusedPartition forms). */
 export function groupPlan(grp: GraphNode[], batch: number, deviceScalars: boolean, q8Of: Map<string, string>, attnExact = true,
-                          rawOf: Map<string, [string, string]> = new Map(), readers?: Graph["tensors"]): KernelPlan {
+                          rawOf: Map<string, [string, string]> = new Map(), readers?: Graph["tensors"], planned?: Set<number>): KernelPlan {
   const ops = grp.map((n) => n.op);
   const key = ops.join("+");
   const bpart = batch !== 1 ? fill(SPEC_SUFFIX.batch, { batch }) : "";
@@ -114,7 +121,7 @@ export function groupPlan(grp: GraphNode[], batch: number, deviceScalars: boolea
       q8Of.set(tn(sw.outputs[0]), aux);
       return plan(spec + SPEC_SUFFIX.q8out, [...args, aux], { [aux]: batch * (N / 32) * 36 });
     }
-    if (rowsServed(N, batch) && (K === 1024 || K === 2048) && (readers?.get(tn(sw.outputs[0]))?.consumers ?? []).every((c) => c.op === "gemm")) {
+    if (rowsServed(N, batch) && (K === 1024 || K === 2048) && onlyMatmulsRead(tn(sw.outputs[0]), readers, planned)) {
       // a few sequences: the activation is only ever read by the down projection, which takes it as Q8_1
       const aux = tn(sw.outputs[0]) + ".q8_1";
       q8Of.set(tn(sw.outputs[0]), aux);
@@ -187,9 +194,10 @@ export function compilePartition(graph: Graph, ordered: GraphNode[][], batch = 1
   const rawOf = new Map<string, [string, string]>();    // output of a gdn_delta_rule node in slab form -> [raw block, norm weight]
   const inConvGroup = new Set<string>();
   for (const g of ordered) if (g.length === 6) for (const n of g) if (n.op === "conv1d_decode") inConvGroup.add(tn(n.outputs[0]));
+  const planned = new Set(ordered.flat().map((n) => n.id));
   const plans: KernelPlan[] = [];
   for (const grp of ordered) {
-    if (grp.length !== 1) { plans.push(groupPlan(grp, batch, deviceScalars, q8Of, attnExact, rawOf, graph.tensors)); continue; }
+    if (grp.length !== 1) { plans.push(groupPlan(grp, batch, deviceScalars, q8Of, attnExact, rawOf, graph.tensors, planned)); continue; }
     const n = grp[0];
     const args = [...n.inputs.map(tn), ...n.outputs.map(tn)];
     const bpart = batch !== 1 ? fill(SPEC_SUFFIX.batch, { batch }) : "";
