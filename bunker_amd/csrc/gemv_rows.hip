@@ -177,14 +177,15 @@ __device__ __forceinline__ void rows_store(void* out, const uint16_t* res, int e
   else store_out<EPI_BF16_ADD>(out, res, o, v);
 }
 
-// Loads go through buffer resources: what lies past the end reads as zero (weights that are not stored anywhere), and an address
-// is a scalar offset and the lane's own, with nothing to clamp.
+// Loads go through buffer resources: what lies past the end is not fetched and reads as zero (weights that are not stored anywhere),
+// with nothing to clamp.  The range check covers the lane's offset and not the instruction's scalar offset, so the whole offset is
+// the lane's: requests past the end are common (the last workgroup of a matrix, rows shorter than KP).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00027000);
 }
 template <int AUX>
-__device__ __forceinline__ uint4 rows_load16(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off) {
-  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)lane_off, (int)off, AUX));
+__device__ __forceinline__ uint4 rows_load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, AUX));
 }
 constexpr int AUX_NT = 2;
 
@@ -197,7 +198,7 @@ template <int NP>
 __device__ __forceinline__ void rows_copy_load(RowsCopy<NP>& c, const void* xq, int pieces) {
   const __amdgpu_buffer_rsrc_t r = rows_rsrc(xq, pieces * 16);
 #pragma unroll
-  for (int i = 0; i < NP; i++) c.v[i] = rows_load16<0>(r, threadIdx.x * 16, 64 * RW * 16 * i);
+  for (int i = 0; i < NP; i++) c.v[i] = rows_load16<0>(r, threadIdx.x * 16 + 64 * RW * 16 * i);
 }
 // row_div: ceil(2^32 / pieces per row), so that the high half of p * row_div is p / (pieces per row)
 template <int NP>
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(64 * RW, TPG > 1 || KP > 2048 ? 2 : 4) void gemv_ro
     for (int i = 0; i < WLOADS; i++) {
       const int p = wave * 64 + 64 * RW * i;
       const bool up = MODE == RMODE_SWIGLU && p >= RUN;
-      wreg[i] = rows_load16<AUX_NT>(rows_rsrc((up ? A.g[1].W : M.W) + at, bytes), L.lane * 16, (up ? p - RUN : p) * 16);
+      wreg[i] = rows_load16<AUX_NT>(rows_rsrc((up ? A.g[1].W : M.W) + at, bytes), L.lane * 16 + (up ? p - RUN : p) * 16);
     }
   }
   const int tp = 16 * rp;
@@ -444,7 +445,7 @@ __global__ __launch_bounds__(64 * RW, 2) void gemv_rows_stream_kernel(RowsArgs1 
     const int n0 = chunk * SLOTS * 16;
     const __amdgpu_buffer_rsrc_t r = rows_rsrc(A.g0.W + (int64_t)n0 * (NB * 144), min(SLOTS * 16, N - n0) * (NB * 144));
 #pragma unroll
-    for (int i = 0; i < WLOADS; i++) wreg[i] = rows_load16<AUX_NT>(r, threadIdx.x * 16, 64 * RW * 16 * i);
+    for (int i = 0; i < WLOADS; i++) wreg[i] = rows_load16<AUX_NT>(r, threadIdx.x * 16 + 64 * RW * 16 * i);
   };
   int chunk = blockIdx.x;
   const int chunks = (A.tiles + SLOTS - 1) / SLOTS;

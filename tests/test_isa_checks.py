@@ -122,3 +122,16 @@ def test_argument_blocks_stay_compact_and_in_registers(tmp_path_factory, source,
         assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", meta).group(1)) == 0, m.group(3)
         assert int(re.search(r"\.vgpr_spill_count:\s+(\d+)", meta).group(1)) == 0, m.group(3)
     assert seen and seen <= kernarg_sizes and min(seen) == min(kernarg_sizes), seen
+
+
+def test_range_checked_loads_carry_their_whole_offset_in_the_lane_operand(tmp_path_factory):
+    """gemv_rows.hip lets the range check of a buffer resource answer for the pieces past the end of the weight and activation rows.
+    That check is defined over the lane's offset and the immediate one; a scalar offset operand is not part of it, so it has to be 0."""
+    asm = _compile_to_asm(tmp_path_factory, "gemv_rows.hip")
+    bodies = {k: v for k, v in _kernels(asm).items() if "gemv_rows" in k}
+    assert len(bodies) >= 13
+    for name, body in bodies.items():
+        loads = re.findall(r"^\s*buffer_load_\w+ (.*)$", body, flags=re.M)
+        assert loads, name
+        for l in loads:
+            assert re.match(r"v\[\d+:\d+\], v\d+, s\[\d+:\d+\], 0 offen\b", l), (name, l)
