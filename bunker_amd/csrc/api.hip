@@ -139,7 +139,11 @@ static int run_gemv_fused(Kernel& k, const uint64_t* s) {
   if (swiglu) out[0] = P<void>(s[si++]);
   void* q8out = swiglu && k.get("q8out", 0) ? P<void>(s[si++]) : nullptr;      // composed path only (build_gemv_fused checks)
   const bool q8only = k.get("q8only", 0) != 0;
-  if ((g_tune_rows != 0 || q8only) && gemv_rows_serves(pro, K, batch, G, swiglu)) {
+  // Row lengths without a fused form run on the plain GEMV, which also takes Q8_1 rows at four-byte alignment and epilogue 2
+  // without a residual (the bf16 result alone); gemv_rows takes neither, so such launches stay there.
+  const bool rows_ok = gemv_rows_serves(pro, K, batch, G, swiglu) &&
+                       (gemv_fused_fast_path(K, batch, swiglu) || (((uintptr_t)x & 15) == 0 && (epi[0] != 2 || res[0])));
+  if ((g_tune_rows != 0 || q8only) && rows_ok) {
     return launch_gemv_rows(pro, x, nw, K, batch, G, W, out, res, N, epi, swiglu, conv.st ? &conv : nullptr, q8only ? out[0] : nullptr);
   }
   if (gemv_fused_fast_path(K, batch, swiglu)) return launch_gemv_fused(pro, x, nw, K, batch, G, W, out, res, N, epi, swiglu, conv.st ? &conv : nullptr);

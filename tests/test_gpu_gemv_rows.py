@@ -96,3 +96,41 @@ def test_swiglu_as_bf16_and_as_q8_1(orc, dev, K, N, batch):
 def test_q8only_is_refused_where_nothing_serves_it(spec):
     with pytest.raises(rt.BunkerError, match="q8only"):
         rt.compileAndLoad(spec)
+
+
+@pytest.mark.parametrize("K,N,batch,epi", [(1536, 9000, 5, 0), (2560, 8192, 3, 1), (3072, 40, 7, 2), (4608, 100, 2, 0), (5120, 33, 4, 2), (5632, 17, 6, 1)])
+def test_q8_1_rows_at_four_byte_alignment(orc, dev, K, N, batch, epi):
+    """Row lengths that the one-row form serves from four-byte alignment on are served there for several rows too."""
+    print(f"gemv_fused pro=0 K={K} N={N} batch={batch} epi={epi}, rows at +4 bytes", flush=True)
+    g = synth.rng(2400 + K)
+    W = synth.q4k_random(g, N, K)
+    xq = np.stack([orc.pack_q8_1(f32(bf(g.standard_normal(K).astype(np.float32)))) for _ in range(batch)])
+    res = bf(g.standard_normal((batch, N)).astype(np.float32))
+    at = dev.up(np.concatenate([np.zeros(4, np.uint8), np.ascontiguousarray(xq).view(np.uint8).ravel()])) + 4
+    out = dev.empty(batch * N * (4 if epi == 0 else 2))
+    launch(f"gemv_fused K={K} pro=0 G=1 N0={N} epi0={epi} batch={batch}", [at, dev.up(W)] + ([dev.up(res)] if epi == 2 else []) + [out])
+    got = rt.from_device(out, (batch, N), np.uint32 if epi == 0 else np.uint16)
+    for b in range(batch):
+        y = orc.gemv_q4k_q8_1(W, xq[b], N, K)
+        ref = y.view(np.uint32) if epi == 0 else orc.cast_bf16(y)
+        assert np.array_equal(got[b], orc.add_bf16(ref, res[b]) if epi == 2 else ref), b
+
+
+def test_epilogue_2_without_a_residual_is_the_bf16_result(orc, dev):
+    K, N, batch = 4608, 50, 3
+    g = synth.rng(2500)
+    W = synth.q4k_random(g, N, K)
+    xq = np.stack([orc.pack_q8_1(f32(bf(g.standard_normal(K).astype(np.float32)))) for _ in range(batch)])
+    out = dev.empty(batch * N * 2)
+    launch(f"gemv_fused K={K} pro=0 G=1 N0={N} epi0=2 batch={batch}", [dev.up(xq), dev.up(W), 0, out])
+    got = rt.from_device(out, (batch, N), np.uint16)
+    for b in range(batch):
+        assert np.array_equal(got[b], orc.cast_bf16(orc.gemv_q4k_q8_1(W, xq[b], N, K))), b
+
+
+@pytest.mark.parametrize("K", [1024, 2048, 3584, 4096, 6144])
+def test_misaligned_rows_of_the_fused_lengths_stay_refused(dev, K):
+    out = dev.empty(3 * 64 * 4)
+    k = rt.compileAndLoad(f"gemv_fused K={K} pro=0 G=1 N0=64 epi0=0 batch=3")
+    x, w = dev.empty(3 * K // 32 * 36 + 16), dev.empty(64 * K // 256 * 144)
+    assert rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], [x + 4, w, out]) != 0 and "aligned" in rt.last_error()
