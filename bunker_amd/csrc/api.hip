@@ -115,8 +115,9 @@ static int run_gemm(Kernel& k, const uint64_t* s) {
 // slots:  x, [norm_w if pro=2|3], then per matrix: W, [residual if epi=2 | conv_state_in, conv_w if epi=3], out,
 //         [conv_state_new if epi=3]      (swiglu: x, [norm_w], Wg, Wu, out [, out as Q8_1 blocks when q8out=1: batch >= 8 only];
 //         q8only=1 (pro=2, K = 1024 or 2048, batch 2..7): out is the Q8_1 blocks, there is no bf16 result)
-// Two to seven rows with pro=2 and K = 1024 or 2048, or with pro=0 and one matrix, run in gemv_rows.hip.  Shapes outside the fused kernel (K other than 1024, 2048, 3584, 4096, 6144, or batch >= 8) run as rmsnorm/quantize,
-// matmuls, swiglu.
+// Two to seven rows with pro=2 and K = 1024 or 2048, or with pro=0 and one matrix, run in gemv_rows.hip where that is the
+// faster form (gemv_rows_pays).  Shapes outside the fused kernel (K other than 1024, 2048, 3584, 4096, 6144, or batch >= 8)
+// run as rmsnorm/quantize, matmuls, swiglu.
 static int run_gemv_fused(Kernel& k, const uint64_t* s) {
   const int K = (int)k.get("K", 0), pro = (int)k.get("pro", 0), G = (int)k.get("G", 1), batch = (int)k.get("batch", 1);
   const bool swiglu = k.get("swiglu", 0) != 0;
@@ -143,7 +144,9 @@ static int run_gemv_fused(Kernel& k, const uint64_t* s) {
   // without a residual (the bf16 result alone); gemv_rows takes neither, so such launches stay there.
   const bool rows_ok = gemv_rows_serves(pro, K, batch, G, swiglu) &&
                        (gemv_fused_fast_path(K, batch, swiglu) || (((uintptr_t)x & 15) == 0 && (epi[0] != 2 || res[0])));
-  if ((g_tune_rows != 0 || q8only) && rows_ok) {
+  const int64_t all_rows = (int64_t)N[0] + N[1] + N[2] + N[3];
+  const bool rows_pay = g_tune_rows == 1 ? gemv_rows_pays(pro, K, batch, all_rows, swiglu) : g_tune_rows != 0;
+  if (rows_ok && (q8only || rows_pay)) {
     return launch_gemv_rows(pro, x, nw, K, batch, G, W, out, res, N, epi, swiglu, conv.st ? &conv : nullptr, q8only ? out[0] : nullptr);
   }
   if (gemv_fused_fast_path(K, batch, swiglu)) return launch_gemv_fused(pro, x, nw, K, batch, G, W, out, res, N, epi, swiglu, conv.st ? &conv : nullptr);

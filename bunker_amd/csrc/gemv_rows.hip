@@ -491,12 +491,42 @@ __global__ __launch_bounds__(64 * RW, 2) void gemv_rows_stream_kernel(RowsArgs1 
   }
 }
 
-int g_tune_rows = 1;      // 0: these launches take the one-row forms
+int g_tune_rows = 1;      // 0: these launches take the one-row forms, 1: gemv_rows_pays decides, 2: gemv_rows wherever it serves
 
 bool gemv_rows_serves(int pro, int K, int batch, int ngroups, bool swiglu) {
   if (batch < 2 || batch > ROWS_MAX) return false;
   if (pro == RPRO_RMSNORM) return K == 1024 || K == 2048;
   return pro == RPRO_Q8 && !swiglu && ngroups == 1 && K >= 1024 && K <= 6144 && K % 512 == 0;
+}
+
+// Whether a served launch takes less time here than in the one-row forms; `rows`: weight rows of all its matrices.
+// One-row forms (gemv_fused; gemv for the lengths that it has no kernel for) cost about 3 us and then grow with rows * batch.
+// Here the batch costs little, but a launch starts later (a workgroup stages its weights, unpacks their headers and prepares
+// every activation row before the first product) and, where only one workgroup fits a CU (KP = 6144: 131 KB of LDS, K = 2048 with
+// the norm: 115), grows in whole rounds of the chip.  Measured on cold weights over 512 to 248320 rows and 2 to 7 sequences
+// (one-row form -> here, us; the lines below lie where the two meet, no measured launch is sent to a form 10 % slower):
+//   norm, K = 1024: 2048 rows x 5 5.0 -> 5.3, 5120 x 2 5.6 -> 4.6, 9216 x 7 16.9 -> 8.4; SwiGLU of 1024 x 7 6.5 -> 7.0, 3584 x 2 6.9 -> 5.8
+//   norm, K = 2048: 5120 rows x 2 5.9 -> 6.3, 9216 x 2 8.2 -> 7.7, two rounds: 18432 x 2 10.9 -> 13.9, x 4 18.1 -> 16.0;
+//                   SwiGLU of 6144 x 2 8.7 -> 9.2, x 3 12.1 -> 9.5
+//   Q8_1 rows, K = 1024: 2048 x 4 3.4 -> 3.8, x 7 4.3 -> 4.0; K = 1536: 4096 x 3 4.0 -> 4.8, x 5 5.8 -> 5.0;
+//              K = 2048: 8192 x 2 5.2 -> 5.5, 4096 x 4 4.9 -> 4.2; K = 4096: 1024 x 7 4.9 -> 5.2, 2048 x 5 6.0 -> 5.4, 12288 x 2 13.1 -> 15.1,
+//              x 3 18.1 -> 15.2; K = 6144: 2048 x 2 4.9 -> 6.2, x 4 7.8 -> 6.2; K = 3072: 49152 x 2 38.8 -> 44.9, x 3 55.8 -> 46.0
+bool gemv_rows_pays(int pro, int K, int batch, int64_t rows, bool swiglu) {
+  const int64_t work = rows * batch;
+  const auto rounds = [&](int64_t rows_per_wg) { return (rows + rows_per_wg * num_cus() - 1) / (rows_per_wg * num_cus()); };
+  if (pro == RPRO_RMSNORM) {
+    if (K == 1024) return work >= (swiglu ? 8000 + 1500 * batch : 6500 + 1000 * batch);
+    if (swiglu && batch == 2) return false;
+    const int64_t r = rounds(swiglu ? 64 : 48);
+    return work >= (r > 1 ? 34000 * r : swiglu ? 14000 + 2200 * batch : 9000 + 1800 * batch);
+  }
+  if (K <= 2048) {
+    if (batch == 2 && K > 1024) return work >= 32768;
+    return work >= (K == 1536 ? 16000 : 6500 + 1000 * batch);        // six super-blocks occupy four waves twice
+  }
+  const int64_t r = rounds(16);
+  if (gemv_fused_fast_path(K, batch, false)) return r == 1 ? work >= (K <= 4096 ? 8448 : 6656) : batch >= 3 && work >= 8192 * r;
+  return r == 1 || batch >= 3 || K >= 4608;
 }
 
 template <int PRO, int KP, int MODE, int TPG>

@@ -58,6 +58,7 @@ int launch_gemv_fused(int pro, const void* x, const void* norm_w, int K, int bat
 // gemv_rows.hip: the same for 2 to 7 activation rows (pro 0 with one matrix, pro 2); out_q8: SwiGLU as Q8_1 blocks instead of bf16
 extern int g_tune_rows;
 bool gemv_rows_serves(int pro, int K, int batch, int ngroups, bool swiglu);
+bool gemv_rows_pays(int pro, int K, int batch, int64_t rows, bool swiglu);
 int launch_gemv_rows(int pro, const void* x, const void* norm_w, int K, int batch, int ngroups, const void* const* W,
                      void* const* out, const void* const* res, const int* N, const int* epi, bool swiglu, const FusedConv* conv,
                      void* out_q8);

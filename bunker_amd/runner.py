@@ -250,6 +250,16 @@ def rows_served(K: int, batch: int) -> bool:
     return ROWS_BATCH[0] <= batch <= ROWS_BATCH[1] and 1024 <= K <= 6144 and K % 512 == 0
 
 
+def rows_swiglu_pays(K: int, N: int, batch: int) -> bool:
+    """Whether gate + up of N rows each over rows of K elements take less time in one pass over the weights (gemv_rows_pays in
+    csrc/gemv_rows.hip, where the measurements stand; 256 CUs)."""
+    work = 2 * N * batch
+    if K == 1024:
+        return work >= 8000 + 1500 * batch
+    rounds = -(-N // (32 * 256))
+    return K == 2048 and batch > 2 and work >= (34000 * rounds if rounds > 1 else 14000 + 2200 * batch)
+
+
 def _only_matmuls_read(graph: Graph, tensor: str, planned: set) -> bool:
     """Whether ``tensor`` has readers and every one is a matmul of the partition being compiled (node ids ``planned``) that takes
     it as its activation: then nothing misses the tensor when its producer leaves it as Q8_1 blocks alone."""
@@ -286,7 +296,7 @@ def _group_plan(graph: Graph, grp: list, batch: int, device_scalars: bool, q8_of
             aux = sw.outputs[0].tensorName + ".q8_1"
             q8_of[sw.outputs[0].tensorName] = aux
             return KernelPlan(spec + " q8out=1", name, args + [aux], [1, 1, 1], grp, {aux: batch * (N // 32) * 36})
-        if rows_served(N, batch) and K in (1024, 2048) and _only_matmuls_read(graph, sw.outputs[0].tensorName, planned):
+        if rows_served(N, batch) and rows_swiglu_pays(K, N, batch) and _only_matmuls_read(graph, sw.outputs[0].tensorName, planned):
             # a few sequences: the activation is only ever read by the down projection, which takes it as Q8_1
             aux = sw.outputs[0].tensorName + ".q8_1"
             q8_of[sw.outputs[0].tensorName] = aux

@@ -95,7 +95,9 @@ BK_API int bk_graph_node_count(uint64_t graph, int* count);
  * "gemv_rpi", "gemv_cap", "gemv_steps", "gemv_impl", "fused_cap" (GEMV rows per wave step, workgroups per CU up to
  * which a wave takes one step, row steps per wave, kernel variant),
  * "gemm_nw" (waves per matmul tile: 1, 2, 4, 8), "gemm_r16" (narrow matmul tiles: 1 = 16 weight rows, 2 = 8), "small_rows" (0: the two 16-row
- * matrices of a batched projection group stay in the matmul instead of the norm's launch), "gdn_cs" (column slabs of the
+ * matrices of a batched projection group stay in the matmul instead of the norm's launch), "rows" (products of 2 to 7
+ * sequences in one pass over the weights: 0 = never, 1 = where it is the faster form, the default, 2 = wherever there is a
+ * kernel for them; the bits are the same), "gdn_cs" (column slabs of the
  * GDN core op), "gdn_nt" / "attn_nt" (state / cache pages through nontemporal accesses), "attn_bal" (attention splits
  * under lengths in device memory: 0 = equal ranges of max_ctx, 2 = of each sequence's own length, 1 = the batch's
  * workgroups shared out by length, -1 = 1 for long ranges, else 2), "prefill_ksplit" (runs along K/V of the tiled prompt

@@ -1,6 +1,7 @@
 """The projections of 2 to 7 sequences that share one pass over the weights (csrc/gemv_rows.hip) against the CPU checker, to the
 bit: every batch, row counts around the 16-row tiles and 32-row SwiGLU pieces, row lengths that leave waves without a
-super-block, all epilogues, and the wave-per-tile form of a long matrix."""
+super-block, all epilogues, and the wave-per-tile form of a long matrix.  The small shapes here would run in the one-row forms,
+which are faster for them, so the tests ask for gemv_rows wherever it serves ("rows" = 2)."""
 import numpy as np
 import pytest
 
@@ -16,6 +17,13 @@ def dev():
     d = Dev()
     yield d
     d.close()
+
+
+@pytest.fixture(autouse=True)
+def rows_wherever_served():
+    rt.tune_set("rows", 2)
+    yield
+    rt.tune_set("rows", 1)
 
 
 @pytest.mark.parametrize("K,batch,N,epi", [(1024, 2, 1, 0), (1024, 7, 33, 2), (1536, 5, 100, 1), (2048, 3, 17, 0), (2048, 7, 520, 2), (2560, 6, 48, 1),
@@ -134,3 +142,34 @@ def test_misaligned_rows_of_the_fused_lengths_stay_refused(dev, K):
     k = rt.compileAndLoad(f"gemv_fused K={K} pro=0 G=1 N0=64 epi0=0 batch=3")
     x, w = dev.empty(3 * K // 32 * 36 + 16), dev.empty(64 * K // 256 * 144)
     assert rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], [x + 4, w, out]) != 0 and "aligned" in rt.last_error()
+
+
+@pytest.mark.parametrize("spec,Ks,Ns", [
+    ("pro=0 G=1 N0={0} epi0=0", 1024, (4100, 4300)), ("pro=0 G=1 N0={0} epi0=1", 2048, (16300, 16400)), ("pro=0 G=1 N0={0} epi0=0", 1536, (7900, 8100)),
+    ("pro=0 G=1 N0={0} epi0=1", 4096, (4090, 4230)), ("pro=0 G=1 N0={0} epi0=0", 2560, (4090, 4100)), ("pro=0 G=1 N0={0} epi0=0", 4608, (4090, 4100)),
+    ("pro=2 G=2 N0={0} epi0=0 N1=33 epi1=1", 1024, (4100, 4300)), ("pro=2 G=1 N0={0} epi0=1", 2048, (6200, 6400)),
+    ("pro=2 G=2 swiglu=1 N0={0} N1={0}", 1024, (2700, 2800)), ("pro=2 G=2 swiglu=1 N0={0} N1={0}", 2048, (8192, 8224))])
+@pytest.mark.parametrize("batch", [2, 3])
+def test_both_sides_of_the_rule_have_the_same_bits(dev, spec, Ks, Ns, batch):
+    """gemv_rows_pays sends the longer of the two matrices here at batch 2 or 3; never, always and by the rule agree."""
+    for N in Ns:
+        print(f"K={Ks} N={N} batch={batch} {spec}", flush=True)
+        g = synth.rng(2600 + N + Ks)
+        ns = [N, N] if "swiglu" in spec else ([N, 33] if "N1=33" in spec else [N])
+        W = [dev.up(synth.q4k_centered(g, n, Ks, 0.05)) for n in ns]
+        x, nw = dev.up(bf(g.standard_normal((batch, Ks)).astype(np.float32))), dev.up(bf((g.standard_normal(Ks) * 0.1).astype(np.float32)))
+        if "pro=0" in spec:
+            xq = dev.empty(batch * Ks // 32 * 36)
+            rt.quantize_q8_1(x, xq, Ks, batch, rt.BF16)
+            head = [xq]
+        else:
+            head = [x, nw]
+        got = []
+        for rows in (0, 1, 2):
+            rt.tune_set("rows", rows)
+            outs = [dev.empty(batch * n * 4) for n in ns]
+            args = head + W + [outs[0]] if "swiglu" in spec else head + [v for pair in zip(W, outs) for v in pair]
+            launch(f"gemv_fused K={Ks} {spec.format(N)} batch={batch}", args)
+            got.append([rt.from_device(o, (batch * n * 4,), np.uint8) for o, n in zip(outs, ns)])
+        for other in got[1:]:
+            assert all(np.array_equal(a, b) for a, b in zip(got[0], other)), N

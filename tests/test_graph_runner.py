@@ -224,6 +224,23 @@ def test_the_swiglu_result_is_left_out_only_when_matmuls_of_the_partition_read_a
     assert sum(p.args[0] == sw.args[-1] and " pro=0 " in p.spec for p in plans) == 2
 
 
+def test_the_rule_for_swiglu_as_q8_1_is_the_librarys():
+    """runner.rows_swiglu_pays and its TypeScript twin state the lines of gemv_rows_pays for gate + up (256 CUs)."""
+    import os
+    root = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..")
+    lib = open(os.path.join(root, "bunker_amd", "csrc", "gemv_rows.hip")).read()
+    lib = lib[lib.index("bool gemv_rows_pays("):][:1500]
+    assert "swiglu ? 8000 + 1500 * batch :" in lib and "swiglu && batch == 2" in lib and "rounds(swiglu ? 64 : 48)" in lib
+    assert "r > 1 ? 34000 * r : swiglu ? 14000 + 2200 * batch :" in lib
+    ts = open(os.path.join(root, "ts", "specs.ts")).read()
+    ts = ts[ts.index("function rowsSwigluPays("):][:500]
+    assert "work >= 8000 + 1500 * batch" in ts and "batch > 2 && work >= (rounds > 1 ? 34000 * rounds : 14000 + 2200 * batch)" in ts
+    pays = runner.rows_swiglu_pays
+    # the benchmark's MLP from three sequences on, the reference model's from two; a round more needs more rows
+    assert not pays(2048, 6144, 2) and pays(2048, 6144, 3) and pays(1024, 3584, 2) and not pays(1024, 1024, 7)
+    assert pays(2048, 8192, 3) and not pays(2048, 8224, 3) and not pays(3584, 8192, 5)
+
+
 class _NoDeviceEnv:
     """Stands in for a DecodeEnv in checks that must fail before anything touches the device."""
     inplace = True

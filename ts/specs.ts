@@ -78,6 +78,14 @@ function rowsServed(K: number, batch: number): boolean {
   return batch >= ROWS_BATCH[0] && batch <= ROWS_BATCH[1] && K >= 1024 && K <= 6144 && K % 512 === 0;
 }
 
+/** Whether gate + up of N rows each over rows of K elements take less time in one pass over the weights (256 CUs). */
+function rowsSwigluPays(K: number, N: number, batch: number): boolean {
+  const work = 2 * N * batch;
+  if (K === 1024) return work >= 8000 + 1500 * batch;
+  const rounds = Math.ceil(N / (32 * 256));
+  return K === 2048 && batch > 2 && work >= (rounds > 1 ? 34000 * rounds : 14000 + 2200 * batch);
+}
+
 function fill(template: string, vars: Record<string, number | string>): string {
   return template.replace(/\$\{(\w+)\}/g, (_, k) => String(vars[k]));
 }
@@ -121,7 +129,7 @@ export function groupPlan(grp: GraphNode[], batch: number, deviceScalars: boolea
       q8Of.set(tn(sw.outputs[0]), aux);
       return plan(spec + SPEC_SUFFIX.q8out, [...args, aux], { [aux]: batch * (N / 32) * 36 });
     }
-    if (rowsServed(N, batch) && (K === 1024 || K === 2048) && onlyMatmulsRead(tn(sw.outputs[0]), readers, planned)) {
+    if (rowsServed(N, batch) && rowsSwigluPays(K, N, batch) && onlyMatmulsRead(tn(sw.outputs[0]), readers, planned)) {
       // a few sequences: the activation is only ever read by the down projection, which takes it as Q8_1
       const aux = tn(sw.outputs[0]) + ".q8_1";
       q8Of.set(tn(sw.outputs[0]), aux);
