@@ -104,6 +104,8 @@ class Prefill:
             "embed": c(f"embed H={D.H} VOCAB={D.VOCAB} ids_dev=1" + bp),
             "gdn_in": c(f"gemv_fused K={D.H} pro=2 G=4 N0={D.QKVD} epi0=1 N1={D.ZD} epi1=1 N2={D.LVH} epi2=0 N3={D.LVH} epi3=0" + bp),
             "conv": c(f"conv1d_prefill QKVD={D.QKVD} T={T}"),
+            # alone=2: whether the chunk has the chip to itself is said at the launch, so both kinds of chunk share the handle's workspace
+            "gdn": c(f"gdn_prefill LVH={D.LVH} T={T}" + (" chunked=1" if self.gdn_chunked else " alone=2")),
             "gdn_out": c(f"gemv_fused K={D.ZD} pro=1 G=1 N0={D.H} epi0=2" + bp),
             "fa_in": c(f"gemv_fused K={D.H} pro=2 G=3 N0={D.QGATE} epi0=1 N1={D.KV_DIM} epi1=1 N2={D.KV_DIM} epi2=1" + bp),
             "fa": c(f"fa2_prefill HD={D.HD} NH={D.NH} NKV={D.NKV} MAX_LEN={D.MAX_LEN} ROT_HALF={D.ROT_HALF} T={T}"
@@ -117,13 +119,6 @@ class Prefill:
         k["mlp_out"] = c(f"gemv_fused K={D.INTER} pro={0 if self_q8 else 1} G=1 N0={D.H} epi0=2" + bp)
         slot.kernels[T] = k
         return k
-
-    def _gdn_kernel(self, kernels: dict, T: int, alone: bool):
-        """The recurrence of a run of T tokens, made when first asked for (each form's handle has a workspace of its own)."""
-        form = " chunked=1" if self.gdn_chunked else (" alone=1" if alone else "")
-        if "gdn" + form not in kernels:
-            kernels["gdn" + form] = rt.compileAndLoad(f"gdn_prefill LVH={self.D.LVH} T={T}" + form)
-        return kernels["gdn" + form]
 
     def _launch(self, k, args, what: str) -> None:
         rc = rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], args)
@@ -191,7 +186,7 @@ class Prefill:
         slot's own behind them."""
         D, e, B = self.D, self.env, slot.buf
         k = self._kernels(slot, T)
-        gdn = self._gdn_kernel(k, T, alone)
+        how = [] if self.gdn_chunked else [int(alone)]
         W = e.ptr
         d_ids, d_pos = self.d_ids + 4 * first_index, self.d_pos + 4 * first_index
         self._launch(k["embed"], [W["embed.weight"], d_ids, B["x"]], "embed")
@@ -208,8 +203,8 @@ class Prefill:
                 cs = self._state(f"{p}.conv_state", 3 * D.QKVD * 2, seq)
                 self._launch(k["conv"], [B["qkv"], cs, W[f"{la}.conv1d.weight"], B["conv"], cs], f"{p} conv1d")
                 ss = self._state(f"{p}.s_state", D.LVH * D.LKD * D.LVD * 4, seq)
-                self._launch(gdn, [B["conv"], B["z"], W[f"{la}.A_log"], W[f"{la}.dt_bias"], B["a"], B["b"],
-                                        W[f"{la}.norm.weight"], ss, B["mix"], ss], f"{p} gdn")
+                self._launch(k["gdn"], [B["conv"], B["z"], W[f"{la}.A_log"], W[f"{la}.dt_bias"], B["a"], B["b"],
+                                        W[f"{la}.norm.weight"], ss, B["mix"], ss] + how, f"{p} gdn")
                 slot.done[layer].record()
                 self._launch(k["gdn_out"], [B["mix"], W[f"{la}.out_proj.weight"], x, h], f"{p} out_proj")
             else:

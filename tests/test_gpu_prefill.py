@@ -79,6 +79,13 @@ def test_gdn_prefill_alone_is_T_decode_steps(orc, monkeypatch, Hg, T):
     test_gdn_prefill_is_T_decode_steps(orc, Hg, T)
 
 
+@pytest.mark.parametrize("Hg,T,alone", [(2, 80, 0), (2, 80, 1), (3, 20, 1)])
+def test_gdn_prefill_told_at_the_launch_is_T_decode_steps(orc, monkeypatch, Hg, T, alone):
+    launch = _launch
+    monkeypatch.setitem(globals(), "_launch", lambda spec, args: launch(spec + " alone=2", args + [alone]))
+    test_gdn_prefill_is_T_decode_steps(orc, Hg, T)
+
+
 @pytest.mark.parametrize("Hg,T", [(2, 1), (3, 5), (2, 64), (4, 65), (3, 200), (16, 1024)])
 def test_gdn_prefill_chunked_form_against_the_scan(Hg, T):
     """chunked=1 (chunks of 64 tokens, f32 matrix instruction) against the scan, which has the checker's bits: the

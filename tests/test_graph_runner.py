@@ -283,3 +283,30 @@ def test_dims_refuse_a_capacity_that_is_not_whole_pages():
     with pytest.raises(ValueError, match="multiple of the 16-token page"):
         model.Dims(MAX_LEN=0)
     assert model.with_context(model.TINY, 128).MAX_LEN == 128
+
+
+def test_a_prompt_chunk_keeps_one_recurrence_handle_whether_or_not_it_runs_alone(monkeypatch):
+    """The handle owns a workspace (25 MB at 1024 tokens of 16 heads): a slot that has run T tokens makes no second one for a chunk of
+    T tokens that another chunk runs beside, and says at the launch which of the two it is."""
+    from collections import defaultdict
+    from types import SimpleNamespace
+
+    from bunker_amd import prefill
+
+    made, launched = [], []
+    monkeypatch.setattr(prefill.rt, "compileAndLoad", lambda spec, *a: made.append(spec) or spec)
+    for chunked in (False, True):
+        pf = prefill.Prefill.__new__(prefill.Prefill)
+        pf.D, pf.on_attention, pf.gdn_chunked, pf.attn_exact = TINY, None, chunked, True
+        pf.d_ids = pf.d_pos = pf.d_table = 0
+        pf.env = SimpleNamespace(ptr=defaultdict(int), state_bufs=defaultdict(lambda: [0, 0]), state_cur=defaultdict(int))
+        pf._launch = lambda k, args, what: launched.append((k, args))
+        slot = SimpleNamespace(stream=None, buf=defaultdict(int), kernels={}, done=[SimpleNamespace(record=lambda: None)] * TINY.NL)
+        del made[:]
+        for alone in (True, False, True):
+            del launched[:]
+            pf._chunk(slot, None, 80, 0, 0, alone=alone)
+            scans = [(k, args) for k, args in launched if k.startswith("gdn_prefill")]
+            assert len(scans) == sum(not TINY.is_full_attention(l) for l in range(TINY.NL))
+            assert all(len(args) == (10 if chunked else 11) and (chunked or args[10] == int(alone)) for _, args in scans)
+        assert sum(s.startswith("gdn_prefill") for s in made) == 1
