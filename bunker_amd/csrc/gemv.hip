@@ -330,7 +330,7 @@ __device__ __forceinline__ float slot_dot_f32(const uint4& hdr, const uint4& q, 
 
 // Rows of up to 8 * NR super-blocks: the LDS staging of gemv_q4k_q8_1_lds_kernel (RPI contiguous rows per wave step,
 // every 128-byte line requested once, the next step's rows in flight during the arithmetic), for any nb: the lanes past
-// the row fold a clamped block against zeros.  What bounds it is latency and the reads of x: with one row per wave (the
+// the row fold a clamped block, its scales and the activations replaced by zeros.  What bounds it is latency and the reads of x: with one row per wave (the
 // form this replaces) every row pulled all of x through the L2 twice, 134 MB for a 9.4 MB matrix.  Back to back on cold
 // weights: 4096 x 4096 13.2 -> 5.5 us, 12288 x 2048 18.3 -> 6.4, 151936 x 2048 110 -> 41 (then bound by vector issue: about
 // 95 instructions per 32 weights of a lane), 50000 x 6144 208 -> 51 (3.4 TB/s).
@@ -349,8 +349,12 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
   uint4* tile = tiles[wv];
 
   XF x[NR];
+  uint32_t in_row[NR];            // all ones, or zero past the row: a lane there has d = dmin = 0 and adds nothing, whatever its block holds
 #pragma unroll
-  for (int r = 0; r < NR; r++) load_xf(x[r], xf, r * 8 + b, c, r * 8 + b < nb);
+  for (int r = 0; r < NR; r++) {
+    load_xf(x[r], xf, r * 8 + b, c, r * 8 + b < nb);
+    in_row[r] = r * 8 + b < nb ? ~0u : 0u;
+  }
 
   StageRegs<NR, RPI> g;
   auto request = [&](int r0) {
@@ -378,7 +382,9 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
 #pragma unroll
       for (int r = 0; r < NR; r++) {
         const int blk = i * row_pieces + min(r * 8 + b, nb - 1) * 9;       // piece index of the block header
-        acc[i] += slot_dot_f32(tile[blk], tile[blk + 1 + c], x[r], sel);
+        uint4 hdr = tile[blk];
+        hdr.x &= in_row[r];
+        acc[i] += slot_dot_f32(hdr, tile[blk + 1 + c], x[r], sel);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -410,7 +416,9 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_generic_kernel(
       XF x;
       load_xf(x, xf, blk, c, blk < nb);
       const int bo = (blk < nb ? blk : 0) * 144;
-      acc += slot_dot_f32(*(const uint4*)(rp + bo), *(const uint4*)(rp + bo + 16 + 16 * c), x, sel);
+      uint4 hdr = *(const uint4*)(rp + bo);
+      if (blk >= nb) hdr.x = 0;                             // past the row: d = dmin = 0
+      acc += slot_dot_f32(hdr, *(const uint4*)(rp + bo + 16 + 16 * c), x, sel);
     }
     const float tot = wave_sum(acc);
     if (lane == 0) y[row] = tot;

@@ -234,6 +234,26 @@ def test_gemv_q4k_f32_staged_rows(orc, dev, N, K):
     assert np.all(y[N:] == 7.5)
 
 
+@pytest.mark.parametrize("K,block", [(1280, 0), (1280, 4), (2304, 0), (2304, 8), (5376, 20), (6400, 0), (6400, 24)])
+def test_gemv_q4k_f32_infinite_scale(orc, dev, K, block):
+    """Lanes past the end of a row stand on a block of the row and must add nothing, also where its scale is infinite: the row's
+    result is the infinity that its own elements give (nibbles, scales and activations of that block positive, min 0)."""
+    g = synth.rng(1400 + K + block)
+    N = 5
+    W = synth.q4k_random(g, N, K)
+    blk = W.reshape(N, K // 256, 144)[2, block]
+    blk[0:4] = np.array([np.inf, 0.0], np.float16).view(np.uint8)
+    blk[4:16] = 0x11
+    blk[16:] = 0x73
+    x = np.abs(g.standard_normal(K)).astype(np.float32) + 0.1
+    dy = dev.empty(N * 4)
+    rt.gemv_q4k_f32(dev.up(W), dev.up(x), dy, N, K)
+    y, ref = rt.from_device(dy, (N,), np.float32), orc.gemv_q4k_f32(W, x, N, K, acc64=True)
+    assert ref[2] == np.inf and y[2] == np.inf, (y[2], ref[2])
+    rest = np.arange(N) != 2
+    _assert_rel(y[rest], ref[rest])
+
+
 @pytest.mark.parametrize("N,K", [(64, 2048), (50, 1024), (9, 6144)])
 def test_gemv_q4k_f32_other_shapes(orc, dev, N, K):
     g = synth.rng(13 + K)
