@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Writes node_specs.json: the op spec string of every node and every fused group of the synthetic model's decode
-graph, as the Python host layer (bunker_amd/runner.py, the code that runs against the GPU) builds them, for batch 1 and
-batch 32 with token ids and positions in device memory.  tests/test_ts_specs.py expands the literal tables of
+graph, as the Python host layer (bunker_amd/runner.py, the code that runs against the GPU) builds them, for batch 1, 4 and
+32 with token ids and positions in device memory.  tests/test_ts_specs.py expands the literal tables of
 ts/specs.ts for the same nodes and groups and must get the same strings.
 
 Needs no GPU and no built library (graph and partition code only).   Run:  python tests/golden/make_node_specs.py
@@ -44,7 +44,7 @@ def main():
     D = model.SYNTH
     doc = {"dims": {k: getattr(D, k) for k in ("H", "VOCAB", "NL", "FAI", "INTER", "NH", "NKV", "HD", "LKH", "LVH", "LKD", "LVD", "MAX_LEN", "ROT_DIM")},
            "device_scalars": True}
-    for batch in (1, 32):
+    for batch in (1, 4, 32):
         doc[f"batch{batch}"] = {"nodes": compact(plans_of(D, batch, False)), "fused": compact(plans_of(D, batch, True))}
     doc["batch1_mfma_attention"] = {"fused": compact([p for p in plans_of(D, 1, True, attn_exact=False) if "fa2_attn" in p["ops"]]),
                                     "nodes": compact([p for p in plans_of(D, 1, False, attn_exact=False) if "fa2_attn" in p["ops"]])}

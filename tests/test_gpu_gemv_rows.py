@@ -75,6 +75,61 @@ def test_norm_and_several_matrices(orc, dev, K, batch):
             assert np.array_equal(got[b], orc.add_bf16(ref, res[b]) if epis[i] == 2 else ref), (i, b)
 
 
+def _silu_conv(orc, y, st, w):
+    """Rows [B, C] (f32) through bf16 and the convolution step: outputs and new states."""
+    return [np.stack(v) for v in zip(*(orc.conv1d_decode(orc.cast_bf16(y[b]), st[b], w) for b in range(len(y))))]
+
+
+@pytest.mark.parametrize("K,batch,Ns", [(1024, 2, (50, 33, 16, 16)), (1024, 7, (6144, 2048, 32, 32)), (2048, 3, (70, 33, 16, 16)),
+                                        (2048, 2, (6144, 2048, 16, 16)), (2048, 5, (6100, 2050, 17, 33)), (2048, 7, (6144, 2048, 16, 16))])
+def test_norm_group_with_the_convolution(orc, dev, K, batch, Ns):
+    """A GDN layer's projections with the convolution behind the first: two tiles a workgroup, and three where the group has more
+    than 512 tiles (6144 + 2048 + 16 + 16 rows at K = 2048), with row counts that are and are not whole workgroups."""
+    print(f"gemv_rows conv K={K} batch={batch} N={Ns}", flush=True)
+    g = synth.rng(2700 + K + batch + Ns[0])
+    Ws = [synth.q4k_centered(g, n, K, 0.5) for n in Ns]
+    x, w = bf(g.standard_normal((batch, K)).astype(np.float32)), bf((g.standard_normal(K) * 0.1).astype(np.float32))
+    st = bf(g.standard_normal((batch, 3, Ns[0])).astype(np.float32))
+    cw = bf((g.standard_normal((Ns[0], 4)) * 0.5).astype(np.float32))
+    xq = ref_activation(orc, 2, x, w)
+    outs = [dev.empty(batch * n * s + 64) for n, s in zip(Ns, (2, 2, 4, 4))]
+    dst = dev.up(st)                                             # the new state over the old one, as the decode step has it
+    launch(f"gemv_fused K={K} pro=2 G=4 N0={Ns[0]} epi0=3 N1={Ns[1]} epi1=1 N2={Ns[2]} epi2=0 N3={Ns[3]} epi3=0 batch={batch}",
+           [dev.up(x), dev.up(w), dev.up(Ws[0]), dst, dev.up(cw), outs[0], dst, dev.up(Ws[1]), outs[1], dev.up(Ws[2]), outs[2], dev.up(Ws[3]), outs[3]])
+    ref = [np.stack([orc.gemv_q4k_q8_1(W, r, n, K) for r in xq]) for W, n in zip(Ws, Ns)]
+    ro, rs = _silu_conv(orc, ref[0], st, cw)
+    assert np.array_equal(rt.from_device(outs[0], (batch, Ns[0]), np.uint16), ro)
+    assert np.array_equal(rt.from_device(dst, st.shape, np.uint16), rs)
+    assert np.array_equal(rt.from_device(outs[1], (batch, Ns[1]), np.uint16), np.stack([orc.cast_bf16(r) for r in ref[1]]))
+    for i in (2, 3):
+        assert np.array_equal(rt.from_device(outs[i], (batch, Ns[i]), np.uint32), ref[i].view(np.uint32))
+    for o, n, s in zip(outs, Ns, (2, 2, 4, 4)):
+        assert np.all(rt.from_device(o, (batch * n * s + 64,), np.uint8)[batch * n * s:] == 0xCD)
+
+
+@pytest.mark.parametrize("batch,Ns,epis", [(2, (8192, 512, 512), (1, 1, 1)), (6, (8192, 520, 33), (1, 0, 2)), (7, (8250,), (0,))])
+def test_norm_groups_of_more_than_512_tiles(orc, dev, batch, Ns, epis):
+    """K = 2048, three tiles a workgroup without the convolution: an attention layer's q, k, v and row counts past whole workgroups."""
+    K = 2048
+    print(f"gemv_rows pro=2 K={K} batch={batch} N={Ns}", flush=True)
+    g = synth.rng(2800 + batch)
+    Ws = [synth.q4k_random(g, n, K) for n in Ns]
+    x, w = bf(g.standard_normal((batch, K)).astype(np.float32)), bf((g.standard_normal(K) * 0.1).astype(np.float32))
+    xq = ref_activation(orc, 2, x, w)
+    args, outs, ress = [dev.up(x), dev.up(w)], [], []
+    for W, n, e in zip(Ws, Ns, epis):
+        ress.append(bf(g.standard_normal((batch, n)).astype(np.float32)))
+        outs.append(dev.empty(batch * n * 4))
+        args += [dev.up(W)] + ([dev.up(ress[-1])] if e == 2 else []) + [outs[-1]]
+    launch(f"gemv_fused K={K} pro=2 G={len(Ns)} batch={batch} " + " ".join(f"N{i}={n} epi{i}={e}" for i, (n, e) in enumerate(zip(Ns, epis))), args)
+    for W, n, e, o, res in zip(Ws, Ns, epis, outs, ress):
+        got = rt.from_device(o, (batch, n), np.uint32 if e == 0 else np.uint16)
+        for b in range(batch):
+            y = orc.gemv_q4k_q8_1(W, xq[b], n, K)
+            ref = y.view(np.uint32) if e == 0 else orc.cast_bf16(y)
+            assert np.array_equal(got[b], orc.add_bf16(ref, res[b]) if e == 2 else ref), (n, b)
+
+
 @pytest.mark.parametrize("K,N,batch", [(1024, 96, 2), (1024, 3584, 5), (2048, 32, 7), (2048, 6144, 4), (1024, 100, 3), (2048, 52, 6)])
 def test_swiglu_as_bf16_and_as_q8_1(orc, dev, K, N, batch):
     print(f"gemv_rows swiglu K={K} N={N} batch={batch}", flush=True)

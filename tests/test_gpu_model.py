@@ -171,6 +171,21 @@ def test_reference_dims_decode(orc, batch):
     assert toks.shape == (3, batch)
 
 
+@pytest.mark.parametrize("dims,batch", [("REFERENCE", 2), ("REFERENCE", 5), ("SYNTH", 3), ("SYNTH", 5)])
+def test_a_few_sequences_at_full_width(orc, dims, batch):
+    """Two to seven sequences at the widths whose projections share one pass over the weights (csrc/gemv_rows.hip): one period of the
+    model's layers and a vocabulary long enough for lm_head's streaming form, step by step and free-running."""
+    from dataclasses import replace
+    D = replace(getattr(model, dims), NL=4, VOCAB=33000, MAX_LEN=64)
+    print(f"{dims} widths, batch {batch}", flush=True)
+    W = synth_model.synth_weights(D, seed=51)
+    S = synth_model.synth_state(D, batch=batch, seed=52)
+    starts = [(113 * i + 9) % D.VOCAB for i in range(batch)]
+    toks, vals = _strict_decode(D, W, S, starts, 30, 3, use_graph=True, fused=True)
+    assert toks.shape == (3, batch)
+    _free_running(D, W, S, starts, 30, 3, toks, vals)
+
+
 @pytest.mark.parametrize("seed", [100, 104, 106, 109])
 def test_free_running_decode_equals_the_checker_over_seeds(orc, seed):
     """No injection, no step-by-step resynchronisation: 4 sequences decode 23 tokens on the GPU (fused partition, replayed

@@ -241,6 +241,28 @@ def test_the_rule_for_swiglu_as_q8_1_is_the_librarys():
     assert pays(2048, 8192, 3) and not pays(2048, 8224, 3) and not pays(3584, 8192, 5)
 
 
+@pytest.mark.parametrize("D,batch,mlp", [(SYNTH, 2, ""), (SYNTH, 4, " q8only=1"), (REFERENCE, 2, " q8only=1"), (REFERENCE, 7, " q8only=1")])
+def test_plan_of_a_few_sequences(D, batch, mlp):
+    """Two to seven sequences: attention leaves its output as Q8_1 too, SwiGLU leaves it alone where gate + up share one pass over the
+    weights, and the projections behind them read that (pro=0); a GDN layer keeps its slab form."""
+    g = model.buildModelGraph(D, batch)
+    plans = runner.compilePartition(g, runner.topoOrder(g, runner.fusedPartition(g)), batch, True)
+    by_first = {p.args[0]: p for p in plans}
+    sw = [p for p in plans if "swiglu=1" in p.spec]
+    assert len(sw) == 24
+    for p in sw:
+        act = p.group[-1].outputs[0].tensorName
+        assert p.spec == f"gemv_fused K={D.H} pro=2 G=2 swiglu=1 N0={D.INTER} N1={D.INTER} batch={batch}{mlp}"
+        assert p.args[-1] == (act + ".q8_1" if mlp else act) and list(p.aux.values()) == ([batch * D.INTER // 32 * 36] if mlp else [])
+        assert by_first[p.args[-1]].spec == f"gemv_fused K={D.INTER} pro={0 if mlp else 1} G=1 N0={D.H} epi0=2 batch={batch}"
+    fa = [p for p in plans if p.spec.startswith("fa2_fused")]
+    assert len(fa) == 6
+    for p in fa:
+        assert p.spec.endswith(" pos_dev=1 q8out=1") and p.args[-2] == p.group[-1].outputs[0].tensorName and list(p.aux) == [p.args[-1]]
+        assert by_first[p.args[-1]].spec == f"gemv_fused K={D.NH * D.HD} pro=0 G=1 N0={D.H} epi0=2 batch={batch}"
+    assert sum(p.spec.startswith("gdn_slabs") for p in plans) == 18
+
+
 class _NoDeviceEnv:
     """Stands in for a DecodeEnv in checks that must fail before anything touches the device."""
     inplace = True

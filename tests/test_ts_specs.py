@@ -3,7 +3,7 @@
 The TypeScript glue a maintainer drops next to src/runner.ts builds its op spec strings from three literal tables
 (SPEC_KEYS, FUSED_SPECS, SPEC_SUFFIX).  This test reads those tables out of the file, expands them with plain ${name}
 substitution — the only thing `fill` in specs.ts does — for every node (424) and every fused group (124 plans) of the
-synthetic model at batch 1 and 32, and compares with tests/golden/node_specs.json, which tests/golden/make_node_specs.py
+synthetic model at batch 1, 4 and 32, and compares with tests/golden/node_specs.json, which tests/golden/make_node_specs.py
 writes from bunker_amd/runner.py (the code the GPU tests run).  It also checks that the fixture is what the host layer
 produces today, and the constants and exports the call sites need."""
 import json
@@ -33,6 +33,7 @@ def ts_const(name):
     return int(re.search(r"export const %s = (\d+);" % name, TS).group(1))
 
 
+ROWS_BATCH = tuple(int(v) for v in re.search(r"export const ROWS_BATCH = \[(\d+), (\d+)\];", TS).groups())
 SPEC_KEYS, FUSED, SUFFIX = ts_table("SPEC_KEYS"), ts_table("FUSED_SPECS"), ts_table("SPEC_SUFFIX")
 
 
@@ -46,6 +47,7 @@ def expand(plan, batch, attn_exact, q8_in):
     key = "+".join(ops)
     bpart = fill(SUFFIX["batch"], batch=batch) if batch != 1 else ""
     q8out = SUFFIX["q8out"] if batch >= ts_const("Q8OUT_MIN_BATCH") else ""
+    few = ROWS_BATCH[0] <= batch <= ROWS_BATCH[1]       # rowsServed; every row length of this model is among those it takes
     if len(ops) == 1:
         op, p = ops[0], P[0]
         if plan["spec"].startswith("gdn_slabs"):
@@ -66,7 +68,7 @@ def expand(plan, batch, attn_exact, q8_in):
             s += SUFFIX["exact0"]
         return s
     if key == "rmsnorm+gemm+gemm+swiglu":
-        return fill(FUSED[key], K=P[1]["K"], N=P[1]["N"]) + bpart + (q8out if P[1]["N"] % 32 == 0 else "")
+        return fill(FUSED[key], K=P[1]["K"], N=P[1]["N"]) + bpart + (SUFFIX["q8only"] if few else q8out if P[1]["N"] % 32 == 0 else "")
     if ops[0] == "rmsnorm" and "conv1d_decode" in ops:
         gem = [p for o, p in zip(ops, P) if o == "gemm"]
         mats = "".join(fill(FUSED["mat"], i=i, N=p["N"], EPI=3 if i == 0 else (1 if p.get("cast") else 0)) for i, p in enumerate(gem))
@@ -83,16 +85,16 @@ def expand(plan, batch, attn_exact, q8_in):
     if key == "qnorm+rope+knorm+ropek+fa2_attn":
         fa, rp = P[4], P[1]
         return fill(FUSED[key], HD=fa["HD"], NH=fa["NH"], NKV=fa["NKV"], MAX_LEN=fa["MAX_LEN"], ROT_HALF=rp["ROT_HALF"]) + bpart + \
-            SUFFIX["pos_dev"] + ("" if attn_exact else SUFFIX["exact0"]) + q8out
+            SUFFIX["pos_dev"] + ("" if attn_exact else SUFFIX["exact0"]) + (SUFFIX["q8out"] if few else q8out)
     raise AssertionError(key)
 
 
-@pytest.mark.parametrize("section,batch,attn_exact", [("batch1", 1, True), ("batch32", 32, True), ("batch1_mfma_attention", 1, False)])
+@pytest.mark.parametrize("section,batch,attn_exact", [("batch1", 1, True), ("batch4", 4, True), ("batch32", 32, True), ("batch1_mfma_attention", 1, False)])
 def test_ts_tables_expand_to_the_host_layers_specs(section, batch, attn_exact):
     for kind in ("nodes", "fused"):
         table = GOLD[section][kind]
         plans = [table["distinct"][i] for i in table["order"]]
-        if section in ("batch1", "batch32"):
+        if section in ("batch1", "batch4", "batch32"):
             assert len(plans) == (424 if kind == "nodes" else 124)
         for p in plans:
             # whether the activation the matmul reads already exists as Q8_1 is the partition's bookkeeping (q8Of in
@@ -104,7 +106,7 @@ def test_ts_tables_expand_to_the_host_layers_specs(section, batch, attn_exact):
 def test_fixture_is_what_the_host_layer_builds_today():
     D = model.SYNTH
     assert {k: getattr(D, k) for k in GOLD["dims"]} == GOLD["dims"]
-    for batch in (1, 32):
+    for batch in (1, 4, 32):
         g = model.buildModelGraph(D, batch)
         for kind, part in (("nodes", runner.choosePartition(g)), ("fused", runner.fusedPartition(g))):
             plans = runner.compilePartition(g, runner.topoOrder(g, part), batch, device_scalars=True)
@@ -118,12 +120,12 @@ def test_fixture_is_what_the_host_layer_builds_today():
 def test_ts_constants_and_exports():
     assert SPEC_KEYS == runner._SPEC_KEYS                      # the same 14 ops, the same constants in the same order
     assert ts_const("Q8OUT_MIN_BATCH") == runner.Q8OUT_MIN_BATCH and ts_const("LM_HEAD_ROWS") == runner.LM_HEAD_ROWS
-    assert ts_const("SLAB_MAX_BATCH") == runner.SLAB_MAX_BATCH
+    assert ts_const("SLAB_MAX_BATCH") == runner.SLAB_MAX_BATCH and ROWS_BATCH == runner.ROWS_BATCH
     assert ts_const("PAGE_TOKENS") == 16
     for fn in ("nodeSpec", "groupPlan", "compilePartition", "loadPartition", "stateBytes", "ropeTables"):
         assert re.search(r"^export function %s\(" % fn, TS, flags=re.M), fn
     # every fused group the Python partition forms has a template, and the templates name only variables groupPlan fills
-    keys = {"+".join(p["ops"]) for b in ("batch1", "batch32") for p in GOLD[b]["fused"]["distinct"] if len(p["ops"]) > 1}
+    keys = {"+".join(p["ops"]) for b in ("batch1", "batch4", "batch32") for p in GOLD[b]["fused"]["distinct"] if len(p["ops"]) > 1}
     for k in keys:
         assert k in FUSED or (k.startswith("rmsnorm+gemm") and ("rmsnorm+gemm*+conv1d_decode" if "conv1d_decode" in k else "rmsnorm+gemm*") in FUSED), k
     # state sizes of stateBytes are the graph's tensor sizes
