@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(GdnPrefillArgs A)
 // per SIMD.  The sums keep their order: even lanes run the fmaf chain over the first 8 rows of a row group, the odd lane next to
 // them goes on from there through the other 8, and the 8 group results are added in order from lanes 1, 3, .. 15 (row
 // broadcasts).  q^, k^, v, decay and beta are staged in LDS a block ahead; three buffers, one barrier per block.
-// 1024 tokens of 16 heads: 197 us against the narrow scan's 270.  Beside another chunk's matmuls it takes more from them than
+// 1024 tokens of 16 heads: 196 us against the narrow scan's 270.  Beside another chunk's matmuls it takes more from them than
 // it gains (it issues twice the instructions, on four times the SIMDs: a prompt of 2048 tokens in two overlapping chunks 30.9 ->
 // 32.1 ms), so those prompts keep the narrow scan.
 constexpr int GW_ROWS = 8;                  // rows per lane
@@ -452,7 +452,7 @@ int launch_gdn_prefill(const void* conv_out, const void* z, const float* A_log, 
   } else if (alone && Hg * GW_SLABS <= num_cus() && T >= 4 * GP_TB) {
     // With more heads the wide form's waves would share SIMDs, which takes away what it gains; the output waves' last block
     // comes behind the state waves', which a few blocks have to pay for (whole prompt, narrow -> wide, of 12 tokens 2.23 ->
-    // 2.29 ms, 70 2.80 -> 2.76, 300 7.13 -> 6.78, 1024 18.6 -> 17.4).
+    // 2.29 ms, 70 3.52 -> 3.51, 300 7.12 -> 6.80, 1024 18.6 -> 17.4).
     hipLaunchKernelGGL(gdn_prefill_wide_scan_kernel, dim3(Hg, GW_SLABS), dim3(256), 0, stream(), A);
   } else {
     hipLaunchKernelGGL(gdn_prefill_scan_kernel, dim3(Hg, GP_SLABS), dim3(256), 0, stream(), A);

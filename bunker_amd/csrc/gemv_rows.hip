@@ -4,7 +4,8 @@
 // What bounds these launches.  One workgroup per (weight rows, sequence), the form this replaces for these batches, repeats
 // the RMSNorm / Q8_1 preparation of a row in hundreds of workgroups and unpacks every weight once per sequence: vector
 // issue, growing by the whole batch-1 cost with each sequence.  Here the int32 sub-block dots come from the matrix cores
-// and the vector work left is the fold in double.
+// and the vector work left is the fold in double.  Neither is the bound now: at five rows vector issue takes 26 to 44 % of a launch, the
+// matrix pipe 2 to 11 %, and 38 to 55 % of the wave cycles wait in the chain round trip - norm - header unpack - fold - join.
 //
 // v_mfma_i32_16x16x64_i8 takes 64 elements of K: the two sub-blocks 2g and 2g+1 that share 32 bytes of a Q4_K super-block.
 // Its 16 columns are 8 activation rows twice: columns 0..7 hold the rows' sub-block 2g and zeros where the weights have the

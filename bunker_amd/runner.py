@@ -55,7 +55,7 @@ def choosePartition(graph: Graph, env=None, opts: dict | None = None) -> Partiti
 LM_HEAD_ROWS = 32768     # matmuls with more rows keep the stand-alone norm + quantizer (its cost is paid once, not per workgroup)
 
 
-ROWS_BATCH = (2, 7)      # batches whose projections share one pass over the weights (csrc/gemv_rows.hip)
+ROWS_BATCH = (2, 7)      # batches whose projections share one pass over the weights where that pays (csrc/gemv_rows.hip)
 SLAB_MAX_BATCH = 7       # up to this batch the GDN step runs in column slabs (64 workgroups for 16 heads instead of 16)
 
 
