@@ -1,0 +1,78 @@
+"""Batched Q4_K x Q8_1 matmul at the edges of its integer fold: the sums over the eight sub-blocks of a super-block are whole
+numbers of 2^-24 while every activation scale lies in [0, 4); any other scale (larger, negative, infinite, NaN) in a tile sends
+that super-block of the tile through the fold in double.  Both must return the bits of the host loop."""
+import numpy as np
+import pytest
+
+from bunker_amd import runtime as rt
+from bunker_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    rt.cu(0)
+
+
+def _same(y, ref):
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(y), nan)
+    assert np.array_equal(y[~nan].view(np.uint32), ref[~nan].view(np.uint32)), int((y[~nan] != ref[~nan]).sum())
+
+
+def _run(orc, W, xq, N, K, B):
+    dW, dxq, dy = rt.to_device(W), rt.to_device(xq), rt.cuAlloc(B * N * 4)
+    try:
+        rt.cuMemset(dy, 0xff, B * N * 4)
+        rt.gemm_q4k_q8_1(dW, dxq, dy, N, K, B)
+        y = rt.from_device(dy, (B, N), np.float32)
+    finally:
+        for p in (dW, dxq, dy):
+            rt.cuFree(p)
+    with np.errstate(all="ignore"):
+        ref = np.stack([orc.gemv_q4k_q8_1(W, xq[b], N, K) for b in range(B)])
+    _same(y, ref)
+
+
+SHAPES = [(100, 768, 32), (33, 2048, 9), (70, 1024, 33), (200, 512, 77), (130, 2304, 130), (257, 256, 260)]
+
+
+@pytest.mark.parametrize("N,K,B", SHAPES)
+@pytest.mark.parametrize("form", ["edge", "wide", "mixed", "negative", "infinite"])
+def test_scales_on_both_sides_of_the_integer_fold(orc, N, K, B, form):
+    print(f"matmul scales {form} N={N} K={K} B={B}", flush=True)
+    g = synth.rng(1200 + N + K + B + len(form))
+    W = synth.q4k_random(g, N, K)
+    xq = np.stack([orc.pack_q8_1(r) for r in g.standard_normal((B, K)).astype(np.float32)]).reshape(B, K // 32, 36)
+    scales = xq[:, :, 32:34].view(np.float16)[..., 0]
+    if form == "edge":            # the largest scale of the integer form (0x43ff), smallest normal and subnormal ones beside it
+        pick = g.integers(0, 4, scales.shape)
+        scales[pick == 0], scales[pick == 1], scales[pick == 2] = np.float16(3.998), np.float16(2.0**-14), np.float16(2.0**-24)
+        xq[:, :, :32] = g.choice(np.array([-128, 127], np.int8), xq[:, :, :32].shape).view(np.uint8)
+    elif form == "wide":          # every super-block of every row through the fold in double
+        scales[:] = np.exp2(g.integers(2, 16, scales.shape)).astype(np.float16)
+    elif form == "mixed":         # one sub-block of a few rows: only some tiles and super-blocks leave the integer form
+        for _ in range(3):
+            scales[g.integers(0, B), g.integers(0, K // 32)] = np.float16(4.0)
+    elif form == "negative":
+        scales[g.integers(0, B)] *= np.float16(-1.0)
+    else:
+        scales[g.integers(0, B), g.integers(0, K // 32)] = np.float16(np.inf)
+        scales[g.integers(0, B), g.integers(0, K // 32)] = np.float16(np.nan)
+    xq[:, :, 32:34] = scales[..., None].view(np.uint8)
+    _run(orc, W, np.ascontiguousarray(xq.reshape(B, -1)), N, K, B)
+
+
+def test_largest_sums_of_the_integer_fold(orc):
+    """Every weight 15 with scale 63 and every activation of one sign at the largest scale: the sums reach 8 * 32 * 945 * 128 * 4."""
+    N, K, B = 64, 1024, 96
+    g = synth.rng(77)
+    W = synth.q4k_random(g, N, K).reshape(-1, 144)
+    W[:, 4:16] = synth.pack_q4k_scales(np.full((W.shape[0], 8), 63), np.full((W.shape[0], 8), 63))
+    W[:, 16:] = 0xFF
+    xq = np.zeros((B, K // 32, 36), np.uint8)
+    xq[:, :, :32] = np.where(np.arange(B) % 2 == 0, 0x80, 0x7F)[:, None, None]
+    xq[:, :, 32:34] = np.float16(3.998).view(np.uint16).reshape(1).view(np.uint8)
+    xq[:, :, 34:36] = np.float16(-1.0).view(np.uint16).reshape(1).view(np.uint8)
+    _run(orc, W, xq.reshape(B, -1), N, K, B)
