@@ -384,11 +384,15 @@ static int run_fa2_prefill(Kernel& k, const uint64_t* s) {
   const int exact = (int)k.get("exact", 1);
   const size_t qn_bytes = fa2_qn_bytes(T, NH, HD), qf_bytes = exact ? attn_exact_qf_bytes(T, NKV) : 0;
   void* qn = k.scratch;
-  uint32_t* qf = exact ? (uint32_t*)((uint8_t*)k.scratch + qn_bytes) : nullptr;
+  const bool rows16 = exact && attn_prefill_exact_serves(T, NH, NKV, HD, P<uint16_t>(s[0]) + HD, P<void>(s[11]));
+  uint32_t* qf = exact && !rows16 ? (uint32_t*)((uint8_t*)k.scratch + qn_bytes) : nullptr;
   void* ws = (uint8_t*)k.scratch + qn_bytes + qf_bytes;
   int rc = launch_attn_prep(P<void>(s[0]), P<void>(s[1]), P<void>(s[2]), P<void>(s[3]), P<void>(s[4]), P<float>(s[5]), P<float>(s[6]),
                             pos, 0, half, max_len, qn, P<void>(s[9]), P<void>(s[10]), table, 0, T, NH, NKV, HD, 16, qf);
   if (rc) return rc;
+  if (rows16)
+    return launch_attn_prefill_exact(qn, P<void>(s[9]), P<void>(s[10]), table, pos, max_len, P<uint16_t>(s[0]) + HD, (int64_t)NH * 2 * HD, 2 * HD,
+                                     P<void>(s[11]), T, NH, NKV);
   if (k.get("tiled", 0))
     return launch_attn_prefill_tiled(qn, P<void>(s[9]), P<void>(s[10]), table, pos, max_len, P<uint16_t>(s[0]) + HD, (int64_t)NH * 2 * HD, 2 * HD,
                                      P<void>(s[11]), T, NH, NKV, HD, 16, ws, k.scratch_bytes - qn_bytes - qf_bytes);
@@ -572,6 +576,7 @@ int bk_tune_set(const char* key, int value) {
   else if (!strcmp(key, "attn_bal")) bk::g_tune_attn_bal = value;
   else if (!strcmp(key, "prefill_xmap")) bk::g_tune_prefill_xmap = value != 0;
   else if (!strcmp(key, "prefill_ksplit")) { BK_REQUIRE(value >= 0 && value <= 4, "bk_tune_set: prefill_ksplit=%d outside 0..4", value); bk::g_tune_prefill_ksplit = value; }
+  else if (!strcmp(key, "prefill_exact")) bk::g_tune_prefill_exact = value;
   else if (!strcmp(key, "gemm_r16")) bk::g_tune_gemm_r16 = value;
   else if (!strcmp(key, "rows")) bk::g_tune_rows = value;
   else if (!strcmp(key, "small_rows")) bk::g_tune_small_rows = value;

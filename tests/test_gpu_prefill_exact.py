@@ -1,0 +1,107 @@
+"""Causal prompt attention in double precision, 16 query rows a workgroup (fa2_prefill with enough tokens): every output must have
+the bits of the one-token-a-workgroup form and of the checker, whatever lies in the cache behind a row's context."""
+import numpy as np
+import pytest
+
+from bunker_amd import runtime as rt
+from bunker_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+bf = synth.f32_to_bf16
+f32 = synth.bf16_to_f32
+HD, HALF = 256, 32
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    rt.cu(0)
+
+
+class _Case:
+    def __init__(self, orc, seed, NH, NKV, T, pos, max_len):
+        g = synth.rng(seed)
+        self.NH, self.NKV, self.T, self.max_len, self.g = NH, NKV, T, max_len, g
+        pages = max_len // 16
+        r = lambda *s: bf(g.standard_normal(s).astype(np.float32))  # noqa: E731
+        self.cos, self.sin = orc.rope_tables(max_len, 2 * HALF, 1e7)
+        self.kc, self.vc = r(pages, NKV, 16, HD), r(pages, NKV, 16, HD)
+        self.qgate, self.k, self.v = r(T, NH, 2, HD), r(T, NKV, HD), r(T, NKV, HD)
+        self.qw, self.kw = (bf((g.standard_normal(HD) * 0.1).astype(np.float32)) for _ in range(2))
+        self.table = g.permutation(pages).astype(np.int32)
+        self.pos = np.asarray(pos, np.int32)
+
+    def run(self, form):
+        rt.tune_set("prefill_exact", form)
+        try:
+            ptrs = [rt.to_device(a) for a in (self.qgate, self.k, self.v, self.qw, self.kw, self.cos, self.sin, self.pos, self.table, self.kc,
+                                              rt.v_pages_to_device_layout(self.vc))]
+            out = rt.cuAlloc(self.T * self.NH * HD * 2)
+            rt.cuMemset(out, 0x5a, self.T * self.NH * HD * 2)
+            k = rt.compileAndLoad(f"fa2_prefill HD={HD} NH={self.NH} NKV={self.NKV} MAX_LEN={self.max_len} ROT_HALF={HALF} T={self.T}")
+            assert rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], ptrs + [out]) == 0, rt.last_error()
+            rt.cuSync()
+            y = rt.from_device(out, (self.T, self.NH, HD), np.uint16)
+            for p in ptrs + [out]:
+                rt.cuFree(p)
+            return y
+        finally:
+            rt.tune_set("prefill_exact", -1)
+
+
+def _same(a, b):
+    fa, fb = f32(a), f32(b)
+    nan = np.isnan(fa)
+    assert np.array_equal(nan, np.isnan(fb))
+    assert np.array_equal(a[~nan], b[~nan]), int((a[~nan] != b[~nan]).sum())
+
+
+@pytest.mark.parametrize("NH,NKV,T,pos0", [(16, 2, 1, 0), (16, 2, 2, 14), (16, 2, 145, 0), (16, 2, 33, 700), (8, 2, 3, 15), (8, 2, 147, 30), (4, 2, 9, 1),
+                                           (4, 2, 65, 250), (2, 2, 17, 0), (2, 2, 150, 13), (8, 1, 16, 47), (12, 2, 150, 5)])
+def test_equals_one_token_a_workgroup(orc, NH, NKV, T, pos0):
+    print(f"prefill exact NH={NH} NKV={NKV} T={T} pos0={pos0}", flush=True)
+    c = _Case(orc, 1300 + NH + T + pos0, NH, NKV, T, pos0 + np.arange(T), 1024)
+    c.vc[:] = np.where(c.g.random(c.vc.shape) < 0.01, 0x7fc0, c.vc) if pos0 == 0 else c.vc      # no cached token is a context token then
+    _same(c.run(1), c.run(0))
+
+
+def test_positions_in_any_order_and_outside_the_cache(orc):
+    g = synth.rng(5)
+    pos = g.permutation(256)[:40]
+    pos[3], pos[17] = -1, 255
+    c = _Case(orc, 1401, 16, 2, 40, pos, 256)
+    _same(c.run(1), c.run(0))
+
+
+@pytest.mark.parametrize("where", ["prompt", "cached", "key", "query"])
+def test_values_that_are_no_numbers_reach_only_the_rows_that_see_them(orc, where):
+    c = _Case(orc, 1500, 16, 2, 150, 37 + np.arange(150), 256)
+    if where == "prompt":                     # a token of the prompt whose value overflowed: the rows before it must not notice
+        c.v[9, 0, 5], c.v[64, 1, 200], c.v[65, 1, 3] = 0x7f80, 0x7fc0, 0xff80
+    elif where == "cached":
+        c.vc[c.table[1], 0, 3, 77] = 0x7f80
+    elif where == "key":
+        c.k[31, 1, 100], c.kc[c.table[0], 0, 2, 9] = 0x7fc0, 0x7f80
+    else:
+        c.qgate[12, 3, 0, 4] = 0x7fc0
+    _same(c.run(1), c.run(0))
+
+
+def test_large_scores_move_the_reference_exponent(orc):
+    c = _Case(orc, 1600, 16, 2, 150, 200 + np.arange(150), 512)
+    c.qw[:], c.kw[:] = bf(np.full(HD, 30.0, np.float32)), bf(np.full(HD, 20.0, np.float32))       # scores of several thousand
+    _same(c.run(1), c.run(0))
+
+
+def test_the_default_route_has_the_checkers_bits(orc):
+    T, NH, NKV, pos0 = 150, 16, 2, 21
+    c = _Case(orc, 1700, NH, NKV, T, pos0 + np.arange(T), 192)
+    out = c.run(-1)
+    kc, vc = c.kc.copy(), c.vc.copy()
+    for t in range(T):
+        qn = orc.rope(orc.headnorm(c.qgate[t].ravel(), c.qw, NH, HD, 2 * HD), c.cos, c.sin, c.pos[t], NH, HD, HALF).reshape(1, NH, HD)
+        kn = orc.rope(orc.headnorm(c.k[t].ravel(), c.kw, NKV, HD, HD), c.cos, c.sin, c.pos[t], NKV, HD, HALF)
+        orc.kv_append(kn.reshape(NKV, HD), c.v[t], kc, vc, c.table, c.pos[t], NKV, HD, 16)
+        ro, _ = orc.attn_decode_paged(qn, kc, vc, c.table[None], np.array([c.pos[t] + 1], np.int32), 1, NH, NKV, HD, 16,
+                                      gate=c.qgate[t].ravel()[HD:], gate_bstride=0, gate_hstride=2 * HD)
+        assert np.array_equal(f32(out[t]), ro[0].astype(np.float32) if ro.dtype != np.uint16 else f32(ro[0])), t
