@@ -76,3 +76,43 @@ def test_largest_sums_of_the_integer_fold(orc):
     xq[:, :, 32:34] = np.float16(3.998).view(np.uint16).reshape(1).view(np.uint8)
     xq[:, :, 34:36] = np.float16(-1.0).view(np.uint16).reshape(1).view(np.uint8)
     _run(orc, W, xq.reshape(B, -1), N, K, B)
+
+
+def _big(g, N, K, B):
+    W = synth.q4k_centered(g, N, K, 0.05)
+    x = g.standard_normal((B, K)).astype(np.float32)
+    dx, dxq = rt.to_device(x), rt.cuAlloc(B * (K // 32) * 36)
+    rt.quantize_q8_1(dx, dxq, K, B, rt.F32)
+    rt.cuFree(dx)
+    return W, rt.to_device(W), dxq
+
+
+@pytest.mark.parametrize("N,K,B,offset", [(32, 256, 9, 0), (96, 512, 33, 2), (160, 1024, 70, 0), (64, 2048, 31, 8)])
+def test_swiglu_blocks_of_every_split(orc, N, K, B, offset):
+    """Gate, up, SwiGLU and the Q8_1 blocks of the result with one wave a tile (a thread holds eight values of a block) and with two and
+    four (one value a lane), the bf16 result at addresses of every alignment: the host's bytes."""
+    print(f"swiglu split N={N} K={K} B={B} offset={offset}", flush=True)
+    g = synth.rng(300 + N + B)
+    Wg, dWg, dxq = _big(g, N, K, B)
+    Wu = synth.q4k_centered(g, N, K, 0.05)
+    dWu, dact, dq = rt.to_device(Wu), rt.cuAlloc(B * N * 2 + 16), rt.cuAlloc(B * (N // 32) * 36)
+    k = rt.compileAndLoad(f"gemv_fused K={K} pro=0 G=2 swiglu=1 N0={N} N1={N} batch={B} q8out=1")
+    try:
+        xq = rt.from_device(dxq, (B, K // 32 * 36), np.uint8)
+        for nw in (0, 1, 2, 4):
+            rt.tune_set("gemm_nw", nw)
+            rt.cuMemset(dact, 0, B * N * 2 + 16)
+            assert rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], [dxq, dWg, dWu, dact + offset, dq]) == 0, rt.last_error()
+            raw = rt.from_device(dact, (B * N * 2 + 16,), np.uint8)
+            act = raw[offset : offset + B * N * 2].view(np.uint16).reshape(B, N)
+            assert not raw[:offset].any() and not raw[offset + B * N * 2 :].any()
+            gq = rt.from_device(dq, (B, (N // 32) * 36), np.uint8)
+            for b in range(B):
+                ref = orc.swiglu(orc.gemv_q4k_q8_1(Wg, xq[b], N, K), orc.gemv_q4k_q8_1(Wu, xq[b], N, K))
+                assert np.array_equal(act[b], ref), (nw, b)
+                assert np.array_equal(gq[b], orc.pack_q8_1((ref.astype(np.uint32) << 16).view(np.float32))), (nw, b)
+    finally:
+        rt.tune_set("gemm_nw", 0)
+        rt.unloadKernel(k)
+        for p in (dWg, dWu, dxq, dact, dq):
+            rt.cuFree(p)
