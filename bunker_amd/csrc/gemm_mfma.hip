@@ -26,6 +26,7 @@
 // cache lines per instruction and leaves the kernel bound by the rate of the L1's address path), one super-block
 // ahead of the arithmetic, and every operand is then read from LDS.
 #include "ops.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace bk {
@@ -466,6 +467,37 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
 int g_tune_gemm_nw = 0;      // waves per tile (1, 2, 4, 8); 0 = chosen from the shape
 int g_tune_gemm_r16 = -1;    // narrow tiles (single batch tile only): 0 off, 1 = 16 weight rows, 2 = 8, -1 = from the shape
 
+// Waves that share a tile.  A CU holds eight waves of this kernel (their registers; 115 KB of LDS), so w tiles on it run in rounds of
+// 8 / nw: more waves a tile make a round shorter and leave fewer waves idle in the last one, but every wave brings a fixed part (first
+// loads, the sums through LDS), and two waves on a SIMD hide each other's waits.  Which one wins depends on how full the last round
+// is; measured in us on the sizes in brackets (tiles per CU, rounded up: nw = 1 / 2 / 4):
+//   up to one: eight (K >= 2048; 2048 x 6144 at 128 rows 40.8 / 23.6 / 15.5, eight 13.9), up to three: 42.8 / 34.4 / 22.2 (2048 x 6144 at 200),
+//   17.8 / 15.6 / 15.6 (12288 x 2048 at 64); four: 18.2 / 16.3 / 18.6 (2048 x 2048 at 512), 17.8 / 16.7 / 18.5 (8256 x 2048 at 96); five and six:
+//   25.2 / 22.5 / 21.8 (12288 x 2048 at 77), 26.1 / 28.9 / 25.5 (2048 x 2048 at 768); seven and eight: 28.0 / 29.6 / 32.2 (2048 x 2048 at 951),
+//   70.5 / 74.4 / 81.1 (2048 x 6144 at 951); nine and ten: 39.3 / 35.3 / 36.3 (12288 x 2048 at 192), 37.9 / 33.5 / 35.8 (8256 x 2048 at 256);
+//   more: 40.0 / 45.3 / 46.9 (12288 x 2048 at 256), 62.1 / 63.5 / 67.5 (at 384).
+static int waves_per_tile(int64_t tiles, int nb) {
+  const int64_t per_cu = (tiles + num_cus() - 1) / num_cus();
+  int nw;
+  if (per_cu <= 1 && nb >= 8) nw = 8;
+  else if (per_cu <= 3) nw = 4;
+  else if (per_cu == 4) nw = 2;
+  else if (per_cu <= 6) nw = 4;
+  else if (per_cu <= 8) nw = 1;
+  else if (per_cu <= 10) nw = 2;
+  else nw = 1;
+  return nb >= 4 ? nw : std::min(nw, nb >= 2 ? 2 : 1);       // no more than a row has super-blocks
+}
+
+// The SwiGLU form, by pairs of tiles per CU (a CU holds four pairs of lone waves), nw = 1 / 2 / 4 in us, gate and up of 6144 x 2048 unless said:
+// one: 18.6 / 13.7 / 11.8 (32 rows); two: 26.1 / 18.9 / 21.1 (64), 16.3 / 13.1 / 14.9 (3584 x 1024 at 128); three to five: 27.1 / 27.2 / 30.2 (96),
+// 29.5 / 33.1 / 39.8 (160), 18.2 / 22.7 / 27.7 (3584 x 1024 at 256); six: 52.6 / 47.4 / 59.7 (256); more: 54.3 / 60.9 / 77.8 (320), 85.6 / 90.0 / 118 (500).
+static int waves_per_tile_swiglu(int64_t pairs, int nb) {
+  const int64_t per_cu = (pairs + num_cus() - 1) / num_cus();
+  const int nw = per_cu <= 1 ? 4 : (per_cu == 2 || per_cu == 6 ? 2 : 1);
+  return nb >= 4 ? nw : std::min(nw, nb >= 2 ? 2 : 1);
+}
+
 template <typename ARGS>
 static void launch_mfma_plain(int tr, int nw, dim3 grid, const ARGS& A) {
   if (tr == 16) {
@@ -510,17 +542,9 @@ int launch_gemm_group_mfma(const void* xq, int K, int batch, int ngroups, const 
     for (int i = 0; i < ngroups; i++) { A.tile_first[i] = tiles; tiles += (N[i] + tr - 1) / tr; }
   }
   for (int i = ngroups; i < 5; i++) A.tile_first[i] = tiles;
-  // waves per tile (measured on the decode shapes at batch 32): long rows split eight ways, K = 2048 four ways,
-  // and not at all when the tiles alone fill the chip many times over (lm_head, prompt batches)
   const int btiles = (batch + 31) / 32;
   const int64_t wgs = (int64_t)tiles * btiles;
-  int nw = g_tune_gemm_nw;
-  if (nw <= 0) {
-    nw = A.nb >= 16 ? 8 : (A.nb >= 4 ? 4 : (A.nb >= 2 ? 2 : 1));
-    if (wgs <= num_cus() && A.nb >= 8) nw = 8;                            // at most a tile per CU: one super-block per wave
-    if (wgs > num_cus() && nw == 8) nw = 4;     // eight waves' LDS leaves room for one workgroup per CU: no second round for a few tiles
-    if (wgs >= 8 * num_cus()) nw = 1;                                     // the tiles alone fill the chip many times over
-  }
+  int nw = g_tune_gemm_nw > 0 ? g_tune_gemm_nw : waves_per_tile(wgs, A.nb);
   nw = nw >= 8 ? 8 : (nw >= 4 ? 4 : (nw >= 2 ? 2 : 1));
   A.tiles = tiles; A.btiles = btiles;
   const dim3 grid(btiles > 1 ? (unsigned)(8 * ((wgs + 7) / 8)) : (unsigned)tiles);
@@ -566,12 +590,7 @@ int launch_gemm_swiglu_mfma(const void* xq, int K, int batch, const void* Wg, co
   for (int i = 0; i < 5; i++) A.tile_first[i] = i ? tiles : 0;
   A.tiles = tiles; A.btiles = btiles;
   const int64_t wgs = (int64_t)tiles * btiles;
-  // waves per tile as in the plain form (each workgroup holds two tiles, so at most four per tile)
-  int nw = g_tune_gemm_nw;
-  if (nw <= 0) {
-    nw = A.nb >= 4 ? 4 : (A.nb >= 2 ? 2 : 1);
-    if (2 * wgs >= 8 * num_cus()) nw = 1;
-  }
+  int nw = g_tune_gemm_nw > 0 ? g_tune_gemm_nw : waves_per_tile_swiglu(wgs, A.nb);
   nw = nw >= 4 ? 4 : (nw >= 2 ? 2 : 1);
   const dim3 grid(btiles > 1 ? (unsigned)(8 * ((wgs + 7) / 8)) : (unsigned)tiles);
   const MfmaArgsSw P{A.g[0].W, A.g[1].W, act, (uint8_t*)act_q8, A.xq, N, A.nb, A.B, tiles, btiles};

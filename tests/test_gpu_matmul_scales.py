@@ -87,6 +87,32 @@ def _big(g, N, K, B):
     return W, rt.to_device(W), dxq
 
 
+@pytest.mark.parametrize("B", [33, 65, 257, 385, 449, 513, 641, 833, 1025, 1217])
+def test_every_split_of_a_tile_gives_the_same_bits(orc, B):
+    """The number of waves that share a tile follows from the tiles per CU (one to twelve over these batches); whichever it is, the
+    sums are the host loop's."""
+    N, K = 2085, 1024
+    print(f"split N={N} K={K} B={B}", flush=True)
+    W, dW, dxq = _big(synth.rng(90 + B), N, K, B)
+    dy = rt.cuAlloc(B * N * 4)
+    try:
+        outs = []
+        for nw in (0, 1, 2, 4, 8):
+            rt.tune_set("gemm_nw", nw)
+            rt.cuMemset(dy, 0xff, B * N * 4)
+            rt.gemm_q4k_q8_1(dW, dxq, dy, N, K, B)
+            outs.append(rt.from_device(dy, (B, N), np.uint32))
+        xq = rt.from_device(dxq, (B, K // 32 * 36), np.uint8)
+    finally:
+        rt.tune_set("gemm_nw", 0)
+        for p in (dW, dxq, dy):
+            rt.cuFree(p)
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0])
+    for b in (0, B // 2, B - 1):
+        assert np.array_equal(outs[0][b], orc.gemv_q4k_q8_1(W, xq[b], N, K).view(np.uint32)), b
+
+
 @pytest.mark.parametrize("N,K,B,offset", [(32, 256, 9, 0), (96, 512, 33, 2), (160, 1024, 70, 0), (64, 2048, 31, 8)])
 def test_swiglu_blocks_of_every_split(orc, N, K, B, offset):
     """Gate, up, SwiGLU and the Q8_1 blocks of the result with one wave a tile (a thread holds eight values of a block) and with two and
