@@ -37,6 +37,8 @@
 
 namespace bk {
 
+typedef f32x4_t __attribute__((aligned(4))) f32x4_a4_t;      // in a workspace, which need not be aligned to 16 bytes
+
 // PF = pages a wave requests ahead of the one it computes on (0 or 2).  Loads are issued
 // unconditionally (past its last page a wave requests a few fixed, cached lines instead), so the number of loads in
 // flight at every wait is known when the kernel is compiled and a wait covers only the page needed.
@@ -196,6 +198,40 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void attn_decode_kernel(AttnArgs A)
   }
 #pragma unroll
   for (int t = 0; t < 16; t++) { oacc[t][0] *= wscale; oacc[t][1] *= wscale; oacc[t][2] *= wscale; oacc[t][3] *= wscale; }
+  if (A.splits > 1) {
+    // Partial outputs: the four waves add up (0 + 1) + (2 + 3), each of them ending with a quarter of the dims (tiles t of 16), which it
+    // writes straight from its registers.  (All of it in wave 0, turned through LDS and written by 256 threads at a 64-byte stride of
+    // the LDS, took a third barrier: with the merge kernel's four waves 12.2 -> 11.1 us at one sequence of 4096 tokens.)
+    f32x4_t (*xch)[8][64] = (f32x4_t (*)[8][64])lds_o2;
+    const int w1 = __builtin_amdgcn_readfirstlane(wave & 1), w2 = __builtin_amdgcn_readfirstlane(wave >> 1);
+    f32x4_t k8[8], k4[4];                 // tiles 8 w1 .. +8 of this wave's pair, then 8 w1 + 4 w2 .. +4 of all
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      k8[t] = w1 ? oacc[8 + t] : oacc[t];
+      xch[wave][t][lane] = w1 ? oacc[t] : oacc[8 + t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 8; t++) k8[t] += xch[wave ^ 1][t][lane];
+    // the partner's part was read by this wave alone, so this wave can fill it again
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      k4[t] = w2 ? k8[4 + t] : k8[t];
+      xch[wave ^ 1][t][lane] = w2 ? k8[t] : k8[4 + t];
+    }
+    __syncthreads();
+    const int64_t pidx = A.slots > 0 ? (int64_t)kvh * A.slots + blockIdx.x : ((int64_t)b * A.NKV + kvh) * A.splits + split;
+    float* po = A.part_o + (pidx * 16 + n) * ATT_HD + 128 * w1 + 64 * w2 + 4 * kg;
+    if (n < A.G * ntk) {
+#pragma unroll
+      for (int t = 0; t < 4; t++) *(f32x4_a4_t*)(po + 16 * t) = k4[t] + xch[wave ^ 3][t][lane];
+      if (kg == 0 && wave == 0) {
+        A.part_ml[(pidx * 16 + n) * 2] = M;
+        A.part_ml[(pidx * 16 + n) * 2 + 1] = L;
+      }
+    }
+    return;
+  }
   auto put = [&](int buf) {
 #pragma unroll
     for (int t = 0; t < 16; t++)
@@ -225,45 +261,39 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void attn_decode_kernel(AttnArgs A)
   // ---- write: thread = dim, loop over the G heads of the group
   const int d = threadIdx.x;   // 0..255
   const int ncols = A.G * ntk;
-  if (A.splits == 1) {
-    for (int c = 0; c < ncols; c++) {
-      const int head = kvh * A.G + c % A.G;
-      const int64_t row = row0 + c / A.G;
-      // M and L live in the lanes with n == c; fetch them through LDS
-      float Mh = lds_m[0][c];
-      for (int w = 1; w < ATT_WAVES; w++) Mh = fmaxf(Mh, lds_m[w][c]);
-      float Lh = 0.0f;
-      for (int w = 0; w < ATT_WAVES; w++) {
-        const float mw = lds_m[w][c];
-        Lh += (mw == -INFINITY) ? 0.0f : lds_l[w][c] * __expf(mw - Mh);
-      }
-      // a sequence without context (length <= 0 found in device memory) has no weights: zeros and lse = -inf
-      float o = Lh > 0.0f ? lds_o[d][c] / Lh : 0.0f;
-      if (A.gate) {
-        const float gv = bf16_to_f32(A.gate[row * A.gate_bstride + (int64_t)head * A.gate_hstride + d]);
-        o = __fmul_rn(o, sigmoid_f64(gv));
-      }
-      A.out[(row * A.NH + head) * ATT_HD + d] = f32_to_bf16(o);
-      if (d == 0 && A.lse) A.lse[row * A.NH + head] = Lh > 0.0f ? Mh + logf(Lh) : -INFINITY;
+  for (int c = 0; c < ncols; c++) {
+    const int head = kvh * A.G + c % A.G;
+    const int64_t row = row0 + c / A.G;
+    // M and L live in the lanes with n == c; fetch them through LDS
+    float Mh = lds_m[0][c];
+    for (int w = 1; w < ATT_WAVES; w++) Mh = fmaxf(Mh, lds_m[w][c]);
+    float Lh = 0.0f;
+    for (int w = 0; w < ATT_WAVES; w++) {
+      const float mw = lds_m[w][c];
+      Lh += (mw == -INFINITY) ? 0.0f : lds_l[w][c] * __expf(mw - Mh);
     }
-  } else {
-    const int64_t pidx = A.slots > 0 ? (int64_t)kvh * A.slots + blockIdx.x : ((int64_t)b * A.NKV + kvh) * A.splits + split;
-    float* po = A.part_o + pidx * 16 * ATT_HD;
-    for (int c = 0; c < ncols; c++) po[c * ATT_HD + d] = lds_o[d][c];
-    if (kg == 0 && wave == 0 && n < ncols) {
-      A.part_ml[(pidx * 16 + n) * 2] = M;
-      A.part_ml[(pidx * 16 + n) * 2 + 1] = L;
+    // a sequence without context (length <= 0 found in device memory) has no weights: zeros and lse = -inf
+    float o = Lh > 0.0f ? lds_o[d][c] / Lh : 0.0f;
+    if (A.gate) {
+      const float gv = bf16_to_f32(A.gate[row * A.gate_bstride + (int64_t)head * A.gate_hstride + d]);
+      o = __fmul_rn(o, sigmoid_f64(gv));
     }
+    A.out[(row * A.NH + head) * ATT_HD + d] = f32_to_bf16(o);
+    if (d == 0 && A.lse) A.lse[row * A.NH + head] = Lh > 0.0f ? Mh + logf(Lh) : -INFINITY;
   }
 }
 
-// Merge of the split partials: one workgroup per (head, batch), thread = dim.  The weights
-// exp(m_s - M) of all splits are computed side by side first (thread = split) and kept in LDS, so the
-// loop over the partial outputs has nothing but independent loads in it.
+// Merge of the split partials: one workgroup per (head, batch).  The weights exp(m_s - M) of all splits are computed side by side
+// (thread = split) and kept in LDS.  Wave w adds up splits w, w + 4, .. in four dims per lane; the partials of its first PRE are
+// requested before the weights are worked out, all at once, so that the kernel waits for memory once.  The four sums meet in LDS as
+// (0 + 1) + (2 + 3), thread = dim.  (A thread per dim with four splits in flight at a time: 4.5 us a launch of 64 splits, now 3.6.)
+template <int PRE>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs A) {
   __shared__ float wsh[ATT_MAX_SPLITS];
   __shared__ float redm[4], redl[4];
+  __shared__ __align__(16) float osum[4][ATT_HD];
   const int head = blockIdx.x, b = blockIdx.y, d = threadIdx.x;      // b: query row
+  const int lane = d & 63, wave = __builtin_amdgcn_readfirstlane(d >> 6);
   const int kvh = head / A.G, h = (b % A.tpw) * A.G + head % A.G;     // h: the row's column in its workgroup's partials
   int64_t p0 = ((int64_t)(b / A.tpw) * A.NKV + kvh) * A.splits;
   int nsplit = A.splits;
@@ -275,33 +305,35 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs A) {
   const bool has = d < nsplit;
   const float ms = has ? A.part_ml[((p0 + d) * 16 + h) * 2] : -INFINITY;
   const float ls = has ? A.part_ml[((p0 + d) * 16 + h) * 2 + 1] : 0.0f;
+  const uint16_t gbits = A.gate ? A.gate[(int64_t)b * A.gate_bstride + (int64_t)head * A.gate_hstride + d] : (uint16_t)0;
+  const float* po = A.part_o + (p0 * 16 + h) * ATT_HD + 4 * lane;
+  f32x4_t pv[PRE];
+#pragma unroll
+  for (int i = 0; i < PRE; i++) pv[i] = *(const f32x4_a4_t*)(po + (int64_t)min(wave + 4 * i, nsplit - 1) * 16 * ATT_HD);
   float M = wave_max(ms);
-  if ((d & 63) == 0) redm[d >> 6] = M;
+  if (lane == 0) redm[wave] = M;
   __syncthreads();
   M = fmaxf(fmaxf(redm[0], redm[1]), fmaxf(redm[2], redm[3]));
   const float w = (ms == -INFINITY) ? 0.0f : __expf(ms - M);
   wsh[d] = w;
   float L = wave_sum(ls * w);
-  if ((d & 63) == 0) redl[d >> 6] = L;
+  if (lane == 0) redl[wave] = L;
   __syncthreads();
   L = (redl[0] + redl[1]) + (redl[2] + redl[3]);
-  // the output gate does not depend on the partials: requested and evaluated ahead of them
-  const float gsig = A.gate ? sigmoid_f64(bf16_to_f32(A.gate[(int64_t)b * A.gate_bstride + (int64_t)head * A.gate_hstride + d])) : 1.0f;
-  const float* po = A.part_o + (p0 * 16 + h) * ATT_HD + d;
-  float o0 = 0.0f, o1 = 0.0f, o2 = 0.0f, o3 = 0.0f;
-  int s = 0;
-  for (; s + 4 <= nsplit; s += 4) {
-    o0 = fmaf(po[(int64_t)(s + 0) * 16 * ATT_HD], wsh[s + 0], o0);
-    o1 = fmaf(po[(int64_t)(s + 1) * 16 * ATT_HD], wsh[s + 1], o1);
-    o2 = fmaf(po[(int64_t)(s + 2) * 16 * ATT_HD], wsh[s + 2], o2);
-    o3 = fmaf(po[(int64_t)(s + 3) * 16 * ATT_HD], wsh[s + 3], o3);
-  }
-  // the last one to three splits keep their own accumulators, so that splits without pages behind them change nothing
-  if (s < nsplit) o0 = fmaf(po[(int64_t)s * 16 * ATT_HD], wsh[s], o0);
-  if (s + 1 < nsplit) o1 = fmaf(po[(int64_t)(s + 1) * 16 * ATT_HD], wsh[s + 1], o1);
-  if (s + 2 < nsplit) o2 = fmaf(po[(int64_t)(s + 2) * 16 * ATT_HD], wsh[s + 2], o2);
-  float o = L > 0.0f ? ((o0 + o1) + (o2 + o3)) / L : 0.0f;      // no context at all: zeros, lse = -inf
-  if (A.gate) o = __fmul_rn(o, gsig);
+  f32x4_t o4 = (f32x4_t){0.0f, 0.0f, 0.0f, 0.0f};
+  auto take = [&](const f32x4_t v, int s) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) o4[j] = fmaf(v[j], wsh[s], o4[j]);
+  };
+#pragma unroll
+  for (int i = 0; i < PRE; i++)
+    if (wave + 4 * i < nsplit) take(pv[i], wave + 4 * i);
+#pragma unroll 4
+  for (int s = wave + 4 * PRE; s < nsplit; s += 4) take(*(const f32x4_a4_t*)(po + (int64_t)s * 16 * ATT_HD), s);
+  *(f32x4_t*)&osum[wave][4 * lane] = o4;
+  __syncthreads();
+  float o = L > 0.0f ? ((osum[0][d] + osum[1][d]) + (osum[2][d] + osum[3][d])) / L : 0.0f;      // no context at all: zeros, lse = -inf
+  if (A.gate) o = __fmul_rn(o, sigmoid_f64(bf16_to_f32(gbits)));
   const uint16_t ob = f32_to_bf16(o);
   A.out[((int64_t)b * A.NH + head) * ATT_HD + d] = ob;
   if (A.out_q8) lane32_q8_1_store(bf16_to_f32(ob), A.out_q8 + (((int64_t)b * A.NH + head) * (ATT_HD / 32) + (d >> 5)) * 36, d & 31);
@@ -410,7 +442,12 @@ int launch_attn_decode(const void* q, const void* kc, const void* vc, const int3
     if (nt) hipLaunchKernelGGL((attn_decode_kernel<0, true>), grid, block, 0, stream(), A);
     else hipLaunchKernelGGL((attn_decode_kernel<0, false>), grid, block, 0, stream(), A);
   }
-  if (splits > 1) hipLaunchKernelGGL(attn_merge_kernel, dim3(NH, batch), dim3(256), 0, stream(), A);
+  if (splits > 1) {
+    // requests in flight per wave: all of a sequence's splits up to 4, 16 and 64
+    if (splits <= 4) hipLaunchKernelGGL(attn_merge_kernel<1>, dim3(NH, batch), dim3(256), 0, stream(), A);
+    else if (splits <= 16) hipLaunchKernelGGL(attn_merge_kernel<4>, dim3(NH, batch), dim3(256), 0, stream(), A);
+    else hipLaunchKernelGGL(attn_merge_kernel<16>, dim3(NH, batch), dim3(256), 0, stream(), A);
+  }
   BK_LAUNCH_CHECK();
   // a single split writes its output from the attention kernel itself; its Q8_1 copy then takes the stand-alone quantizer
   if (splits == 1 && out_q8) return launch_quantize_q8_1(out, DT_BF16, out_q8, NH * HD, batch);

@@ -317,6 +317,23 @@ def test_attn_decode_invariants(orc, dev):
     assert np.array_equal(out_p, outs[2][0]) and np.array_equal(lse_p, outs[2][1])
 
 
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 16, 17, 63, 64, 65, 70, 128])
+def test_attn_decode_merge_at_the_edges_of_its_requests(orc, dev, splits):
+    """The merge requests the partials of up to 4, 16 or 64 splits at once and walks the rest; each of its waves takes every fourth."""
+    print(f"attn merge splits={splits}", flush=True)
+    g = synth.rng(630 + splits)
+    B, L = 2, 2100                                          # 132 pages: splits without pages among 65, 70 and 128
+    kc, vc, bt, ctx = synth.paged_kv_random(g, B, L)
+    ctx[:] = [L, 1037]
+    q = bf(g.standard_normal((B, 16, 256)).astype(np.float32))
+    out, lse, s = _run_attn(dev, q, kc, vc, bt, ctx, B, L, splits)
+    assert s == splits
+    ro, rl = orc.attn_decode_paged(q, kc, vc, bt, ctx, B, 16, 2, 256, 16)
+    # weights carry 16 significand bits and sums 24: what is left is the bf16 of the output (2^-9 of it, values below 1)
+    assert np.abs(f32(out).astype(np.float64) - f32(ro)).max() <= 4e-3
+    assert np.all(np.abs(lse - rl) <= 1e-5 * np.maximum(1, np.abs(rl)))
+
+
 def test_attn_decode_splits_follow_lengths_in_device_memory(orc, dev):
     """Lengths in device memory: relative splits (tune attn_bal = 2: every sequence cuts its own pages) and the balanced
     plan (1: the batch's workgroup slots handed out in proportion to the lengths) against the plain splits of the
