@@ -237,15 +237,23 @@ def unloadKernel(k: LoadedKernel) -> None:
     _check(cu().bk_kernel_destroy(k.fn), "bk_kernel_destroy")
 
 
+def packSlots(args: Sequence[int]):
+    """The 8-byte argument slots of a launch, for ``cuLaunchPacked``; kept, they serve any number of launches."""
+    return (u64 * len(args))(*[int(a) & 0xFFFFFFFFFFFFFFFF for a in args])
+
+
+def cuLaunchPacked(k: LoadedKernel, slots) -> int:
+    """``cuLaunch`` with the slots packed already."""
+    return cu().bk_launch(k.fn, slots, len(slots))
+
+
 def cuLaunch(k: LoadedKernel, grid: Sequence[int], block: Sequence[int], args: Sequence[int]) -> int:
     """Launch with the reference's slot packing: one 8-byte slot per argument.
 
     ``grid`` and ``block`` are accepted and ignored (each kernel owns its launch shape).
     Returns the library's return code without raising, as cuLaunch returns the driver's.
     """
-    n = len(args)
-    slots = (u64 * n)(*[int(a) & 0xFFFFFFFFFFFFFFFF for a in args])
-    return cu().bk_launch(k.fn, slots, n)
+    return cuLaunchPacked(k, packSlots(args))
 
 
 def tune_set(key: str, value: int) -> None:

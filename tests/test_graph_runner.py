@@ -332,3 +332,31 @@ def test_a_prompt_chunk_keeps_one_recurrence_handle_whether_or_not_it_runs_alone
             assert len(scans) == sum(not TINY.is_full_attention(l) for l in range(TINY.NL))
             assert all(len(args) == (10 if chunked else 11) and (chunked or args[10] == int(alone)) for _, args in scans)
         assert sum(s.startswith("gdn_prefill") for s in made) == 1
+
+
+def test_handles_of_a_step_are_shared_only_where_launches_follow_each_other(monkeypatch):
+    """compileStep(in_order=True): one handle per spec, every launch under its own label; otherwise kernels with a workspace keep a
+    handle each."""
+    made = []
+
+    def load(spec, name=None, warps=4, label=None):
+        made.append(spec)
+        return runner.rt.LoadedKernel(module=0, fn=len(made), shmem=0, label=label or spec)
+
+    monkeypatch.setattr(runner.rt, "compileAndLoad", load)
+    g = model.buildModelGraph(model.TINY, 2)
+    for part in (runner.choosePartition(g), runner.fusedPartition(g)):
+        made.clear()
+        own = runner.compileStep(g, part, 2, device_scalars=True)
+        separate = len(made)
+        made.clear()
+        shared = runner.compileStep(g, part, 2, device_scalars=True, in_order=True)
+        assert len(made) == len(set(made)) < separate
+        assert [p.spec for p, _ in shared.schedule] == [p.spec for p, _ in own.schedule]
+        assert [k.label for _, k in shared.schedule] == [p.name for p, _ in shared.schedule]
+        by_fn = {}
+        for p, k in shared.schedule:
+            assert by_fn.setdefault(k.fn, p.spec) == p.spec
+        for p, k in own.schedule:
+            if p.spec.startswith("gemv_fused") or p.group[0].op in ("gemm", "fa2_attn", "argmax"):
+                assert sum(q.fn == k.fn for _, q in own.schedule) == 1
