@@ -139,13 +139,15 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
   unsigned char* const stage = ldsW + GW_BYTES;
 
   // Copy maps.  Activations: instruction i = 2c + h covers bytes 64c.. of rows 16h + lane/4, 16 bytes per lane (the
-  // last chunk has 32 bytes per row: lanes 2, 3 of a quad repeat lane 1's piece and do not store).  Rows past B re-read
-  // row B-1 (their results are not stored).  Weights: piece p = lane + 64 i of the 288 16-byte pieces, row p / 9; rows
-  // past N re-read row N-1.
+  // last chunk has 32 bytes per row: lanes 2, 3 of a quad repeat lane 1's piece and store it where lane 1 does).  Rows past B
+  // re-read row B-1 (their results are not stored).  Weights: piece p = lane + 64 i of the 288 16-byte pieces, row p / 9
+  // (past the last piece: that piece again, to the same place); rows past N re-read row N-1.  Every lane stores in every
+  // round: a store behind a lane test costs four scalar instructions and a branch.
   const int rq = lane >> 2, k4 = lane & 3;
   const uint8_t* xsrc[2] = {xq + (int64_t)min(rq, B - 1) * xrow_bytes + 16 * k4, xq + (int64_t)min(16 + rq, B - 1) * xrow_bytes + 16 * k4};
   const int xtail = 16 * min(k4, 1) - 16 * k4;                 // moves lanes 2, 3 back onto piece 17 in the last chunk
   unsigned char* const xdst[2] = {ldsX + rq * GX_ROW + 16 * k4, ldsX + (16 + rq) * GX_ROW + 16 * k4};
+  unsigned char* const wlast = ldsW + min(lane + 64 * (TR * 9 / 64), TR * 9 - 1) * 16;      // the last, partial round of the weight pieces
   const uint8_t* const wbase = W + (int64_t)n0 * wrow_bytes;
   uint32_t woff[5];
 #pragma unroll
@@ -172,6 +174,7 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
 
   // where the lane's own weight row sits among the rows of its half: row = 8g + 4h + v  ->  [h][4g + v]
   const int wcol = col & (TR - 1);
+  const uint32_t scmask = half ? 0x0f0f0f0fu : 0x3f3f3f3fu;
   const int stage_slot = ((wcol >> 2) & 1) * 16 + 4 * (wcol >> 3) + (wcol & 3);
   const unsigned char* const myW = ldsW + wcol * GW_ROW;        // int8 operands: weight row col, batch row col,
   const unsigned char* const myX = ldsX + col * GX_ROW;         // bytes 16*half.. of every sub-block
@@ -189,20 +192,20 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
     __builtin_amdgcn_wave_barrier();     // the previous super-block has been consumed by every lane
 #pragma unroll
     for (int i = 0; i < 10; i++) {
-      uint32_t* p = (uint32_t*)(xdst[i & 1] + 64 * (i >> 1));
-      if (i < 8 || k4 < 2) { p[0] = xr[i].x; p[1] = xr[i].y; p[2] = xr[i].z; p[3] = xr[i].w; }
+      uint32_t* p = (uint32_t*)(xdst[i & 1] + 64 * (i >> 1) + (i >= 8 ? xtail : 0));
+      p[0] = xr[i].x; p[1] = xr[i].y; p[2] = xr[i].z; p[3] = xr[i].w;
     }
     *(uint4*)(ldsW + lane * 16) = wr0;
     if (TR == 8) {
-      if (lane < 8) *(uint4*)(ldsW + (lane + 64) * 16) = wr1;
+      *(uint4*)wlast = wr1;
     } else if (TR == 16) {
       *(uint4*)(ldsW + (lane + 64) * 16) = wr1;
-      if (lane < 16) *(uint4*)(ldsW + (lane + 128) * 16) = wr2;
+      *(uint4*)wlast = wr2;
     } else {
       *(uint4*)(ldsW + (lane + 64) * 16) = wr1;
       *(uint4*)(ldsW + (lane + 128) * 16) = wr2;
       *(uint4*)(ldsW + (lane + 192) * 16) = wr3;
-      if (lane < 32) *(uint4*)(ldsW + (lane + 256) * 16) = wr4;
+      *(uint4*)wlast = wr4;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -215,10 +218,12 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
     // the 6-bit scales of the lane's weight row (half 0 stages sub-blocks 0..3, half 1 sub-blocks 4..7) and its d
     {
       const uint4 hdr = *(const uint4*)myW;
-      const uint32_t scw = half ? ((hdr.w & 0x0f0f0f0fu) | (((hdr.y >> 6) & 0x03030303u) << 4)) : (hdr.y & 0x3f3f3f3fu);
+      // low bits from the word of the half's own sub-blocks, high bits (half 1) from the top of the first; the halves differ in
+      // masks, not in a branch
+      const uint32_t scw = ((half ? hdr.w : hdr.y) & scmask) | ((hdr.y >> 2) & ~scmask & 0x30303030u);
 #pragma unroll
       for (int i = 0; i < 4; i++) stage[(4 * half + i) * 32 + stage_slot] = (unsigned char)(scw >> (8 * i));
-      if (!half) ((double*)(stage + 256))[stage_slot] = (double)half_to_f32((uint16_t)(hdr.x & 0xffffu));
+      ((double*)(stage + 256))[stage_slot] = (double)half_to_f32((uint16_t)(hdr.x & 0xffffu));      // (both halves the same)
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -268,17 +273,31 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
           if (j & 1) qn = *(const uint4*)(myW + 16 + 32 * ((j + 1) >> 1) + 16 * half);
         }
         __builtin_amdgcn_sched_barrier(0);
-        const int m8 = (int)(half_to_f32((uint16_t)dsw) * 16777216.0f);
+        const int m8 = (int)fma(half_to_f32((uint16_t)dsw), 16777216.0f, 0.0f);      // (one instruction with the conversion; exact)
         const uint32_t scv[4] = {scb.x, scb.y, scb.z, scb.w};
-        // (an instruction, not a C expression: integer sums have no order of their own, and the compiler gathers all eight
-        // matrix results in front of them)
-        auto fold_row = [&](int r) {
-          const int t = __mul24(c[r], (int)((scv[r >> 2] >> (8 * (r & 3))) & 0xffu));
-          if (j == 0) asm volatile("v_mad_i64_i32 %0, vcc, %1, %2, %3" : "=v"(S[r]) : "v"(t), "v"(m8), "s"(GM_MAGIC) : "vcc");
-          else asm volatile("v_mad_i64_i32 %0, vcc, %1, %2, %0" : "+v"(S[r]) : "v"(t), "v"(m8) : "vcc");
-        };
+        // Four rows: their scales are the four bytes of one word.  (The sums are instructions, not C expressions: integer sums have
+        // no order of their own, and the compiler gathers all eight matrix results in front of them; four in a block, because
+        // it puts an idle cycle between neighbouring blocks that it cannot look into.  The products stay in C: only there does
+        // the compiler keep the distance that a matrix instruction's result needs before it is read.)
+        auto fold4 = [&](int r) {
+          int t[4];
 #pragma unroll
-        for (int r = 0; r < RF / 2; r++) fold_row(r);
+          for (int i = 0; i < 4; i++) t[i] = __mul24(c[r + i], (int)((scv[r >> 2] >> (8 * i)) & 0xffu));
+          if (j == 0)
+            asm volatile("v_mad_i64_i32 %0, vcc, %4, %8, %9\n\tv_mad_i64_i32 %1, vcc, %5, %8, %9\n\t"
+                         "v_mad_i64_i32 %2, vcc, %6, %8, %9\n\tv_mad_i64_i32 %3, vcc, %7, %8, %9"
+                         : "=&v"(S[r]), "=&v"(S[r + 1]), "=&v"(S[r + 2]), "=&v"(S[r + 3])
+                         : "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(m8), "s"(GM_MAGIC) : "vcc");
+          else
+            asm volatile("v_mad_i64_i32 %0, vcc, %4, %8, %0\n\tv_mad_i64_i32 %1, vcc, %5, %8, %1\n\t"
+                         "v_mad_i64_i32 %2, vcc, %6, %8, %2\n\tv_mad_i64_i32 %3, vcc, %7, %8, %3"
+                         : "+&v"(S[r]), "+&v"(S[r + 1]), "+&v"(S[r + 2]), "+&v"(S[r + 3])
+                         : "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(m8) : "vcc");
+        };
+        // (the first half before the matrix instruction: two blocks of the sixteen rows, one of eight, none of four)
+        constexpr int FIRST = RF / 8 * 4;
+#pragma unroll
+        for (int r = 0; r < FIRST; r += 4) fold4(r);
         __builtin_amdgcn_sched_barrier(0);
         if (j + 1 < 8) {
           if (j & 1) q = qn;
@@ -286,7 +305,7 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = RF / 2; r < RF; r++) fold_row(r);
+        for (int r = FIRST; r < RF; r += 4) fold4(r);
         __builtin_amdgcn_sched_barrier(0);
         c = cn; scb = scn; dsw = dsn;
       }
