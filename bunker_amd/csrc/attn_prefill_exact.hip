@@ -160,9 +160,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
           for (int v = 0; v < 4; v++) O[n][v] *= alpha;
       }
     }
+    // (a wave that has seen only scores of -inf has no reference yet: their weights are 0, not exp(inf - inf))
+    const double ref = mref == -INFINITY ? 0.0 : mref;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      p[v] = valid[v] ? exp(s[v] - mref) : 0.0;
+      p[v] = valid[v] ? exp(s[v] - ref) : 0.0;
       l += p[v];
     }
     // a key past every row's context has weight 0, but what its slot holds need not be a number: it enters as 0
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
 #pragma unroll
     for (int n = 0; n < 4; n++)
 #pragma unroll
-      for (int v = 0; v < 4; v++) lds[(wave * 64 + 16 * n + 4 * v + q4) * PE_PAD + l16] = mref == -INFINITY ? 0.0 : O[4 * c + n][v] * f;
+      for (int v = 0; v < 4; v++) lds[(wave * 64 + 16 * n + 4 * v + q4) * PE_PAD + l16] = O[4 * c + n][v] * f;
     __syncthreads();
     if (ot < A.T && (only < 0 || orow / G == only)) {
       uint16_t ob[4];

@@ -87,6 +87,26 @@ def test_values_that_are_no_numbers_reach_only_the_rows_that_see_them(orc, where
     _same(c.run(1), c.run(0))
 
 
+def test_a_wave_whose_pages_hold_only_scores_of_minus_infinity_adds_nothing(orc):
+    """Page 1 (all that the second of the four waves sees before page 5) has an infinite key element and every query a negative one
+    there: its 16 scores are -inf and their weights 0, and the rows are what the other pages make them."""
+    T, NH, NKV, pos0 = 150, 16, 2, 32
+    c = _Case(orc, 1650, NH, NKV, T, pos0 + np.arange(T), 256)
+    c.kc[c.table[1], :, :, 100] = 0x7f80
+    c.qgate[:, :, 0, 100] |= 0x8000
+    out = c.run(1)
+    _same(out, c.run(0))
+    kc, vc = c.kc.copy(), c.vc.copy()
+    for t in range(3):
+        kn = orc.rope(orc.headnorm(c.k[t].ravel(), c.kw, NKV, HD, HD), c.cos, c.sin, c.pos[t], NKV, HD, HALF)
+        orc.kv_append(kn.reshape(NKV, HD), c.v[t], kc, vc, c.table, c.pos[t], NKV, HD, 16)
+        qn = orc.rope(orc.headnorm(c.qgate[t].ravel(), c.qw, NH, HD, 2 * HD), c.cos, c.sin, c.pos[t], NH, HD, HALF).reshape(1, NH, HD)
+        ro, _ = orc.attn_decode_paged(qn, kc, vc, c.table[None], np.array([c.pos[t] + 1], np.int32), 1, NH, NKV, HD, 16,
+                                      gate=c.qgate[t].ravel()[HD:], gate_bstride=0, gate_hstride=2 * HD)
+        assert np.isfinite(f32(ro[0])).all() and np.abs(f32(ro[0])).max() > 0
+        assert np.array_equal(f32(out[t]), f32(ro[0])), t
+
+
 def test_large_scores_move_the_reference_exponent(orc):
     c = _Case(orc, 1600, 16, 2, 150, 200 + np.arange(150), 512)
     c.qw[:], c.kw[:] = bf(np.full(HD, 30.0, np.float32)), bf(np.full(HD, 20.0, np.float32))       # scores of several thousand
