@@ -10,6 +10,9 @@ constexpr int ATT_PAGE = 16;
 constexpr int ATT_WAVES = 4;
 constexpr int ATT_MAX_PPS = 1024;     // pages per split (the split's page table is staged in LDS)
 constexpr int ATT_MAX_SPLITS = 256;
+// Reference exponent (double) before the first score above -inf: the largest double that is -inf as a float, so that any score that
+// is finite as a float moves it and one that is -inf weighs exp(-inf) = 0 against it (against -inf it would weigh exp(inf - inf)).
+constexpr double ATT_NO_REF = -0x1.ffffffp127;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) short short4_t;

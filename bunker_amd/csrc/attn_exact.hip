@@ -229,7 +229,7 @@ __global__ __launch_bounds__(EX_THREADS) void attn_exact_kernel(AttnArgs A) {
       for (int r = 0; r < EX_TILE_PAGES; r++) kr[r] = ld16(A.kc + page_base(tile * EX_TILE_PAGES + r) + tid8 * 8);
     };
     double l_lane = 0.0;            // wave = head: this lane's share of the sum of weights
-    double mref = -INFINITY;        // wave = head: the reference exponent
+    double mref = ATT_NO_REF;       // wave = head: the reference exponent
     uint4 kpre[EX_TILE_PAGES];      // K of the next tile, requested a whole step ahead
     if (ntiles > 0) load_k(0, kpre);
     for (int tile = 0; tile <= ntiles && ntiles > 0; tile++) {      // (an empty page range: neither role enters its loop)
@@ -276,8 +276,10 @@ __global__ __launch_bounds__(EX_THREADS) void attn_exact_kernel(AttnArgs A) {
         const bool valid = tok < lim;
         const float smax = wave_max(valid ? (float)s : -INFINITY);
         double alpha = 1.0;
-        if (smax > -INFINITY && (mref == -INFINITY || (double)smax > mref + EX_REF_SLACK)) {      // wave-uniform, rare after the first tile
-          if (mref != -INFINITY) { alpha = exp(mref - (double)smax); l_lane *= alpha; }
+        if (smax > -INFINITY && (double)smax > mref + EX_REF_SLACK) {      // wave-uniform, rare after the first tile
+          int t = tile;
+          asm("" : "+s"(t));                         // (seen through, the test peels the first step off the loop)
+          if (t > 0) { alpha = exp(mref - (double)smax); l_lane *= alpha; }
           mref = (double)smax;
         }
         const double p = valid ? exp(s - mref) : 0.0;
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(EX_THREADS) void attn_exact_kernel(AttnArgs A) {
       __syncthreads();
     }
     const double lt = wave_sum_f64(l_lane);
-    if (lane == 0) { lds_l[w8] = lt; lds_m[w8] = mref; }
+    if (lane == 0) { lds_l[w8] = lt; lds_m[w8] = mref == ATT_NO_REF ? -INFINITY : mref; }
   }
 
   double acc[EX_COLS][4];

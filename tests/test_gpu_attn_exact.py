@@ -84,6 +84,25 @@ def test_exact_attention_any_split_same_bits(orc, dev):
     _same(out_n, lse_n, ro, rl, "garbage behind the context")
 
 
+@pytest.mark.parametrize("splits", [1, 2, 4, 8])
+def test_exact_attention_range_of_scores_of_minus_infinity(orc, dev, splits):
+    """Tokens 64 .. 127 have an infinite key element where every query is negative: whatever ranges the context is cut into (with four
+    and eight splits one or two hold no other token), these tokens weigh nothing and the others decide."""
+    print(f"exact attn, -inf range, splits={splits}", flush=True)
+    g = synth.rng(720)
+    B, L = 2, 256
+    kc, vc, bt, ctx = synth.paged_kv_random(g, B, L)
+    ctx[:] = [L, 200]
+    q = bf(g.standard_normal((B, 16, 256)).astype(np.float32))
+    q[:, :, 100] |= 0x8000
+    kc[bt[:, 4:8].ravel(), :, :, 100] = 0x7F80
+    out, lse, s = _run_exact(dev, q, kc, vc, bt, ctx, B, L, splits)
+    assert s == splits
+    ro, rl = orc.attn_decode_paged(q, kc, vc, bt, ctx, B, 16, 2, 256, 16)
+    assert np.isfinite(f32(ro)).all()
+    assert np.array_equal(out, ro) and np.array_equal(lse, rl)
+
+
 def test_exact_attention_other_group_sizes(orc, dev):
     """4 query heads per KV head (the reference model's 8 : 2) and one head per KV head; more than 8 is refused."""
     g = synth.rng(720)
