@@ -4,6 +4,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <sstream>
 #include <string>
@@ -390,9 +391,13 @@ static int run_fa2_prefill(Kernel& k, const uint64_t* s) {
   int rc = launch_attn_prep(P<void>(s[0]), P<void>(s[1]), P<void>(s[2]), P<void>(s[3]), P<void>(s[4]), P<float>(s[5]), P<float>(s[6]),
                             pos, 0, half, max_len, qn, P<void>(s[9]), P<void>(s[10]), table, 0, T, NH, NKV, HD, 16, qf);
   if (rc) return rc;
-  if (rows16)
+  if (rows16) {
+    // (this form cuts nothing, but a handle whose cut the decode kernel refuses is refused whatever T is)
+    const int pages = max_len / 16;
+    if ((rc = attn_check_splits(pages, std::min((int)k.get("splits", 0), pages)))) return rc;
     return launch_attn_prefill_exact(qn, P<void>(s[9]), P<void>(s[10]), table, pos, max_len, P<uint16_t>(s[0]) + HD, (int64_t)NH * 2 * HD, 2 * HD,
                                      P<void>(s[11]), T, NH, NKV);
+  }
   if (k.get("tiled", 0))
     return launch_attn_prefill_tiled(qn, P<void>(s[9]), P<void>(s[10]), table, pos, max_len, P<uint16_t>(s[0]) + HD, (int64_t)NH * 2 * HD, 2 * HD,
                                      P<void>(s[11]), T, NH, NKV, HD, 16, ws, k.scratch_bytes - qn_bytes - qf_bytes);

@@ -359,6 +359,12 @@ int attn_choose_splits(int batch, int NKV, int max_ctx) {
   return s < 1 ? 1 : (s > ATT_MAX_SPLITS ? ATT_MAX_SPLITS : s);
 }
 
+int attn_check_splits(int pages, int splits) {
+  BK_REQUIRE(splits <= ATT_MAX_SPLITS, "attn_decode: at most %d splits", ATT_MAX_SPLITS);
+  BK_REQUIRE((pages + splits - 1) / splits <= ATT_MAX_PPS, "attn_decode: %d pages in %d splits exceed %d pages per split", pages, splits, ATT_MAX_PPS);
+  return BK_OK;
+}
+
 int launch_attn_decode(const void* q, const void* kc, const void* vc, const int32_t* block_table, int bt_stride,
                        const int32_t* ctx_len, int ctx_scalar, int ctx_add, int max_ctx, const void* gate, int64_t gate_bstride,
                        int64_t gate_hstride, void* out, float* lse, void* workspace, size_t workspace_bytes, int batch,
@@ -382,8 +388,7 @@ int launch_attn_decode(const void* q, const void* kc, const void* vc, const int3
   // a context the host knows sizes the splits itself; lengths in device memory leave only their bound
   const int pages = ((ctx_len ? max_ctx : ctx_scalar + ctx_add) + ATT_PAGE - 1) / ATT_PAGE;
   if (splits > pages) splits = pages;
-  BK_REQUIRE(splits <= ATT_MAX_SPLITS, "attn_decode: at most %d splits", ATT_MAX_SPLITS);
-  BK_REQUIRE((pages + splits - 1) / splits <= ATT_MAX_PPS, "attn_decode: %d pages in %d splits exceed %d pages per split", pages, splits, ATT_MAX_PPS);
+  if (int rc = attn_check_splits(pages, splits)) return rc;
   AttnArgs A{};
   A.q = (const uint16_t*)q; A.kc = (const uint16_t*)kc; A.vc = (const uint16_t*)vc;
   A.block_table = block_table; A.ctx_len = ctx_len; A.gate = (const uint16_t*)gate;

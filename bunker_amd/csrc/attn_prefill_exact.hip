@@ -249,7 +249,7 @@ bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD, const void* gate,
 int launch_attn_prefill_exact(const void* q, const void* kc, const void* vc, const int32_t* block_table, const int32_t* pos, int max_ctx,
                               const void* gate, int64_t gate_bstride, int64_t gate_hstride, void* out, int T, int NH, int NKV) {
   BK_REQUIRE(q && kc && vc && block_table && pos && out, "fa2_prefill (exact): null pointer");
-  BK_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 7) == 0 && ((uintptr_t)out & 7) == 0 &&
+  BK_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0 && ((uintptr_t)out & 7) == 0 &&
              ((uintptr_t)gate & 7) == 0, "fa2_prefill (exact): misaligned pointer");
   BK_REQUIRE(T >= 1 && T <= 65535 && NKV >= 1 && max_ctx >= 1 && gate_bstride % 4 == 0 && gate_hstride % 4 == 0, "fa2_prefill (exact): bad shape");
   const int G = NH / NKV, TK = 16 / G;

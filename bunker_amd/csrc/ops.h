@@ -119,6 +119,7 @@ struct AttnPrepFuse {
 };
 size_t attn_workspace_bytes(int batch, int NKV, int max_splits);
 int attn_choose_splits(int batch, int NKV, int max_ctx);
+int attn_check_splits(int pages, int splits);      // the limits of a cut of `pages` pages into `splits` ranges
 int launch_attn_decode(const void* q, const void* kc, const void* vc, const int32_t* block_table, int bt_stride,
                        const int32_t* ctx_len, int ctx_scalar, int ctx_add, int max_ctx, const void* gate, int64_t gate_bstride,
                        int64_t gate_hstride, void* out, float* lse, void* workspace, size_t workspace_bytes, int batch,

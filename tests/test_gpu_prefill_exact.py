@@ -113,6 +113,27 @@ def test_large_scores_move_the_reference_exponent(orc):
     _same(c.run(1), c.run(0))
 
 
+@pytest.mark.parametrize("T", [1, 150])
+def test_a_call_is_refused_whatever_the_number_of_tokens(T):
+    """Caches that are not aligned to 16 bytes and a cut into ranges of more than 1024 pages, by the one-token form and by the
+    16-row form alike (the buffers have room for what the preparation launch in front of the refusal writes)."""
+    NH, NKV, ML = 16, 2, 16400
+    sizes = [T * NH * 2 * HD * 2, T * NKV * HD * 2, T * NKV * HD * 2, HD * 2, HD * 2, ML * HALF * 4, ML * HALF * 4, T * 4, ML // 16 * 4,
+             ML * NKV * HD * 2 + 64, ML * NKV * HD * 2 + 64, T * NH * HD * 2]
+    ptrs = [rt.cuAlloc(n) for n in sizes]
+    for p, n in zip(ptrs, sizes):
+        rt.cuMemset(p, 0, n)
+    spec = f"fa2_prefill HD={HD} NH={NH} NKV={NKV} MAX_LEN={ML} ROT_HALF={HALF} T={T}"
+    for extra, moved in ((" splits=1", None), ("", 9), ("", 10), ("", None)):
+        k = rt.compileAndLoad(spec + extra)
+        rc = rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], [p + 8 * (i == moved) for i, p in enumerate(ptrs)])
+        rt.cuSync()
+        rt.unloadKernel(k)
+        assert (rc != 0) == (bool(extra) or moved is not None), (extra, moved, rc)
+    for p in ptrs:
+        rt.cuFree(p)
+
+
 def test_the_default_route_has_the_checkers_bits(orc):
     T, NH, NKV, pos0 = 150, 16, 2, 21
     c = _Case(orc, 1700, NH, NKV, T, pos0 + np.arange(T), 192)
