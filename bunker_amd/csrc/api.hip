@@ -383,9 +383,9 @@ static int run_fa2_prefill(Kernel& k, const uint64_t* s) {
   const int32_t* table = P<int32_t>(s[8]);
   BK_REQUIRE(pos && table, "fa2_prefill: null position or block table pointer");
   const int exact = (int)k.get("exact", 1);
-  const size_t qn_bytes = fa2_qn_bytes(T, NH, HD), qf_bytes = exact ? attn_exact_qf_bytes(T, NKV) : 0;
+  const bool rows16 = k.get("rows16", 0) != 0;
+  const size_t qn_bytes = fa2_qn_bytes(T, NH, HD), qf_bytes = exact && !rows16 ? attn_exact_qf_bytes(T, NKV) : 0;
   void* qn = k.scratch;
-  const bool rows16 = exact && attn_prefill_exact_serves(T, NH, NKV, HD, P<uint16_t>(s[0]) + HD, P<void>(s[11]));
   uint32_t* qf = exact && !rows16 ? (uint32_t*)((uint8_t*)k.scratch + qn_bytes) : nullptr;
   void* ws = (uint8_t*)k.scratch + qn_bytes + qf_bytes;
   int rc = launch_attn_prep(P<void>(s[0]), P<void>(s[1]), P<void>(s[2]), P<void>(s[3]), P<void>(s[4]), P<float>(s[5]), P<float>(s[6]),
@@ -502,7 +502,10 @@ static int build_kernel(Kernel& k) {
     const int NHq = (int)k.get("NH", 0);
     const int exact = (int)k.get("exact", 1);
     BK_REQUIRE(!exact || NHq / NKV <= 8, "fa2_prefill: exact=1 serves at most 8 query heads per KV head (exact=0 takes 16)");
-    // (the double-precision kernel takes one token per workgroup)
+    // exact=1: 16 query rows a workgroup (attn_prefill_exact.hip), which needs no workspace behind the queries, or the decode kernel with a token
+    // a workgroup
+    const bool rows16 = exact && attn_prefill_exact_serves(T, NHq, NKV, (int)k.get("HD", 0));
+    k.p["rows16"] = rows16;
     // exact=0: query tiles against K/V tiles (attn_prefill.hip) where that kernel serves the shape, unless tiled=0 asks for
     // the decode kernel per token (pair) instead
     const bool tiled = !exact && k.get("tiled", 1) != 0 && attn_prefill_tiled_serves(NHq, NKV, max_len);
@@ -514,9 +517,9 @@ static int build_kernel(Kernel& k) {
     int splits = (int)k.get("splits", 0);
     if (splits <= 0) { splits = attn_choose_splits((T + tpw - 1) / tpw, NKV, max_len); k.p["splits"] = splits; }
     const size_t qbytes = fa2_qn_bytes(T, (int)k.get("NH", 0), (int)k.get("HD", 0));
-    const size_t ws_bytes = tiled ? attn_prefill_workspace_bytes(T, NHq, NKV, max_len) : fa2_ws_bytes(T, NKV, splits, exact);
+    const size_t ws_bytes = tiled ? attn_prefill_workspace_bytes(T, NHq, NKV, max_len) : rows16 ? 0 : fa2_ws_bytes(T, NKV, splits, exact);
     if ((rc = alloc_scratch(k, qbytes + ws_bytes))) return rc;
-    if (exact) BK_HIP(hipMemset(k.scratch, 0, k.scratch_bytes));
+    if (exact && !rows16) BK_HIP(hipMemset(k.scratch, 0, k.scratch_bytes));
     k.run = run_fa2_prefill; k.nslots = 12;
     return BK_OK;
   }

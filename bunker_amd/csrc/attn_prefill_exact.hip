@@ -30,6 +30,7 @@ struct PrefillExactArgs {
   uint16_t* out;
   int64_t gate_bstride, gate_hstride;
   int T, NH, NKV, max_ctx, groups;       // groups of 16 / G tokens
+  int wide;                              // gate and out at 8-byte alignment: four values at a time
   float scale;
 };
 
@@ -214,7 +215,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
     if (ot < A.T && (only < 0 || orow / G == only)) {
       uint16_t ob[4];
       uint2 gr = make_uint2(0, 0);
-      if (A.gate) gr = *(const uint2*)(A.gate + (int64_t)ot * A.gate_bstride + (int64_t)head * A.gate_hstride + 64 * c + od);
+      if (A.gate) {
+        const uint16_t* g = A.gate + (int64_t)ot * A.gate_bstride + (int64_t)head * A.gate_hstride + 64 * c + od;
+        if (A.wide) gr = *(const uint2*)g;
+        else gr = make_uint2((uint32_t)g[0] | ((uint32_t)g[1] << 16), (uint32_t)g[2] | ((uint32_t)g[3] << 16));
+      }
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const double* x = lds + (od + i) * PE_PAD + orow;
@@ -225,8 +230,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
         if (A.gate) o = __fmul_rn(o, sigmoid_f64(bf16_to_f32((uint16_t)((i < 2 ? gr.x : gr.y) >> (16 * (i & 1))))));
         ob[i] = f32_to_bf16(o);
       }
-      *(uint2*)(A.out + ((int64_t)ot * A.NH + head) * ATT_HD + 64 * c + od) =
-          make_uint2((uint32_t)ob[0] | ((uint32_t)ob[1] << 16), (uint32_t)ob[2] | ((uint32_t)ob[3] << 16));
+      uint16_t* op = A.out + ((int64_t)ot * A.NH + head) * ATT_HD + 64 * c + od;
+      if (A.wide) *(uint2*)op = make_uint2((uint32_t)ob[0] | ((uint32_t)ob[1] << 16), (uint32_t)ob[2] | ((uint32_t)ob[3] << 16));
+      else
+#pragma unroll
+        for (int i = 0; i < 4; i++) op[i] = ob[i];
     }
   }
   }
@@ -234,12 +242,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
 
 int g_tune_prefill_exact = -1;           // -1 = from the shape, 0 = one launch row per token (attn_exact.hip), 1 = always where it serves
 
-// Groups of 1, 2, 4 or 8 heads, 8-byte aligned output and gate (the other form takes any), and enough tokens: a workgroup
+// Groups of 1, 2, 4 or 8 heads (the other form takes any) and enough tokens: a workgroup
 // walks its whole context, 0.08 us per key while the launch has at most a workgroup per CU, where one workgroup per token
 // and KV head over cut ranges takes 0.28 ns per (token, KV head, key).  128 tokens behind 3000 (2 KV heads): 211 us there, 266
 // here; 300 from empty 96 and 48.
-bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD, const void* gate, const void* out) {
-  if (HD != ATT_HD || NKV < 1 || NH % NKV || (((uintptr_t)gate | (uintptr_t)out) & 7)) return false;
+bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD) {
+  if (HD != ATT_HD || NKV < 1 || NH % NKV) return false;
   const int G = NH / NKV;
   if (G != 1 && G != 2 && G != 4 && G != 8) return false;
   if (g_tune_prefill_exact >= 0) return g_tune_prefill_exact != 0;
@@ -249,12 +257,12 @@ bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD, const void* gate,
 int launch_attn_prefill_exact(const void* q, const void* kc, const void* vc, const int32_t* block_table, const int32_t* pos, int max_ctx,
                               const void* gate, int64_t gate_bstride, int64_t gate_hstride, void* out, int T, int NH, int NKV) {
   BK_REQUIRE(q && kc && vc && block_table && pos && out, "fa2_prefill (exact): null pointer");
-  BK_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0 && ((uintptr_t)out & 7) == 0 &&
-             ((uintptr_t)gate & 7) == 0, "fa2_prefill (exact): misaligned pointer");
+  BK_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0, "fa2_prefill (exact): q, K and V must be 16-byte aligned");
   BK_REQUIRE(T >= 1 && T <= 65535 && NKV >= 1 && max_ctx >= 1 && gate_bstride % 4 == 0 && gate_hstride % 4 == 0, "fa2_prefill (exact): bad shape");
   const int G = NH / NKV, TK = 16 / G;
   const PrefillExactArgs A{(const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (const uint16_t*)gate, block_table, pos,
-                           (uint16_t*)out, gate_bstride, gate_hstride, T, NH, NKV, max_ctx, (T + TK - 1) / TK, 0.0625f};
+                           (uint16_t*)out, gate_bstride, gate_hstride, T, NH, NKV, max_ctx, (T + TK - 1) / TK,
+                           (((uintptr_t)gate | (uintptr_t)out) & 7) == 0, 0.0625f};
   const dim3 grid((unsigned)(A.groups * NKV));
   if (G == 8) hipLaunchKernelGGL(attn_prefill_exact_kernel<8>, grid, dim3(256), 0, stream(), A);
   else if (G == 4) hipLaunchKernelGGL(attn_prefill_exact_kernel<4>, grid, dim3(256), 0, stream(), A);

@@ -1,5 +1,7 @@
 """Causal prompt attention in double precision, 16 query rows a workgroup (fa2_prefill with enough tokens): every output must have
 the bits of the one-token-a-workgroup form and of the checker, whatever lies in the cache behind a row's context."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -31,17 +33,22 @@ class _Case:
         self.table = g.permutation(pages).astype(np.int32)
         self.pos = np.asarray(pos, np.int32)
 
-    def run(self, form):
+    def run(self, form, shift=0):
+        """``shift``: bytes by which the query | gate and output addresses miss the allocation's alignment"""
         rt.tune_set("prefill_exact", form)
         try:
-            ptrs = [rt.to_device(a) for a in (self.qgate, self.k, self.v, self.qw, self.kw, self.cos, self.sin, self.pos, self.table, self.kc,
+            qgate = np.concatenate([np.zeros(shift, np.uint8), self.qgate.ravel().view(np.uint8)])
+            ptrs = [rt.to_device(a) for a in (qgate, self.k, self.v, self.qw, self.kw, self.cos, self.sin, self.pos, self.table, self.kc,
                                               rt.v_pages_to_device_layout(self.vc))]
-            out = rt.cuAlloc(self.T * self.NH * HD * 2)
-            rt.cuMemset(out, 0x5a, self.T * self.NH * HD * 2)
+            out = rt.cuAlloc(self.T * self.NH * HD * 2 + 16)
+            rt.cuMemset(out, 0x5a, self.T * self.NH * HD * 2 + 16)
             k = rt.compileAndLoad(f"fa2_prefill HD={HD} NH={self.NH} NKV={self.NKV} MAX_LEN={self.max_len} ROT_HALF={HALF} T={self.T}")
-            assert rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], ptrs + [out]) == 0, rt.last_error()
+            assert rt.cuLaunch(k, [1, 1, 1], [128, 1, 1], [ptrs[0] + shift, *ptrs[1:], out + shift]) == 0, rt.last_error()
             rt.cuSync()
-            y = rt.from_device(out, (self.T, self.NH, HD), np.uint16)
+            raw = rt.from_device(out, (self.T * self.NH * HD * 2 + 16,), np.uint8)
+            assert (raw[:shift] == 0x5a).all() and (raw[raw.size - 16 + shift:] == 0x5a).all()
+            y = raw[shift:raw.size - 16 + shift].view(np.uint16).reshape(self.T, self.NH, HD)
+            rt.unloadKernel(k)
             for p in ptrs + [out]:
                 rt.cuFree(p)
             return y
@@ -63,6 +70,36 @@ def test_equals_one_token_a_workgroup(orc, NH, NKV, T, pos0):
     c = _Case(orc, 1300 + NH + T + pos0, NH, NKV, T, pos0 + np.arange(T), 1024)
     c.vc[:] = np.where(c.g.random(c.vc.shape) < 0.01, 0x7fc0, c.vc) if pos0 == 0 else c.vc      # no cached token is a context token then
     _same(c.run(1), c.run(0))
+
+
+@pytest.mark.parametrize("shift", [2, 4, 8])
+def test_gate_and_output_at_any_address(orc, shift):
+    c = _Case(orc, 1350, 16, 2, 37, 5 + np.arange(37), 64)
+    want = c.run(0)
+    _same(c.run(1), want)
+    _same(c.run(1, shift), want)
+    _same(c.run(0, shift), want)
+
+
+@pytest.mark.parametrize("T,NKV,max_len,rows16", [(4096, 2, 4352, True), (2048, 8, 16384, True), (143, 2, 4352, False)])
+def test_a_handle_keeps_no_workspace_that_its_form_does_not_read(T, NKV, max_len, rows16):
+    """The 16-row form needs the normalised queries (bf16) alone; a token a workgroup also their copy in double (4 bytes a value, eight
+    columns a KV head) and the partial results of its cut."""
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert rt.cu().hipMemGetInfo(C.byref(free), C.byref(total)) == 0      # (of the runtime that the library is linked against)
+        return free.value
+
+    NH = 16
+    spec = f"fa2_prefill HD={HD} NH={NH} NKV={NKV} MAX_LEN={max_len} ROT_HALF={HALF} T={T}"
+    rt.unloadKernel(rt.compileAndLoad(spec))
+    rt.cuSync()
+    free = free_bytes()
+    k = rt.compileAndLoad(spec)
+    used = free - free_bytes()
+    rt.unloadKernel(k)
+    queries, copy = T * NH * HD * 2, T * NKV * HD * 8 * 4
+    assert used <= queries + (4 << 20) if rows16 else used >= queries + copy, (used, queries, copy)
 
 
 def test_positions_in_any_order_and_outside_the_cache(orc):
