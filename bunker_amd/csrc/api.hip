@@ -502,10 +502,6 @@ static int build_kernel(Kernel& k) {
     const int NHq = (int)k.get("NH", 0);
     const int exact = (int)k.get("exact", 1);
     BK_REQUIRE(!exact || NHq / NKV <= 8, "fa2_prefill: exact=1 serves at most 8 query heads per KV head (exact=0 takes 16)");
-    // exact=1: 16 query rows a workgroup (attn_prefill_exact.hip), which needs no workspace behind the queries, or the decode kernel with a token
-    // a workgroup
-    const bool rows16 = exact && attn_prefill_exact_serves(T, NHq, NKV, (int)k.get("HD", 0));
-    k.p["rows16"] = rows16;
     // exact=0: query tiles against K/V tiles (attn_prefill.hip) where that kernel serves the shape, unless tiled=0 asks for
     // the decode kernel per token (pair) instead
     const bool tiled = !exact && k.get("tiled", 1) != 0 && attn_prefill_tiled_serves(NHq, NKV, max_len);
@@ -516,6 +512,10 @@ static int build_kernel(Kernel& k) {
     k.p["pair"] = tpw == 2;
     int splits = (int)k.get("splits", 0);
     if (splits <= 0) { splits = attn_choose_splits((T + tpw - 1) / tpw, NKV, max_len); k.p["splits"] = splits; }
+    // exact=1: 16 query rows a workgroup (attn_prefill_exact.hip), which needs no workspace behind the queries, or the decode kernel with a token
+    // a workgroup
+    const bool rows16 = exact && attn_prefill_exact_serves(T, NHq, NKV, (int)k.get("HD", 0), splits);
+    k.p["rows16"] = rows16;
     const size_t qbytes = fa2_qn_bytes(T, (int)k.get("NH", 0), (int)k.get("HD", 0));
     const size_t ws_bytes = tiled ? attn_prefill_workspace_bytes(T, NHq, NKV, max_len) : rows16 ? 0 : fa2_ws_bytes(T, NKV, splits, exact);
     if ((rc = alloc_scratch(k, qbytes + ws_bytes))) return rc;

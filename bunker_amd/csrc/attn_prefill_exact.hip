@@ -242,16 +242,25 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
 
 int g_tune_prefill_exact = -1;           // -1 = from the shape, 0 = one launch row per token (attn_exact.hip), 1 = always where it serves
 
-// Groups of 1, 2, 4 or 8 heads (the other form takes any) and enough tokens: a workgroup
-// walks its whole context, 0.08 us per key while the launch has at most a workgroup per CU, where one workgroup per token
-// and KV head over cut ranges takes 0.28 ns per (token, KV head, key).  128 tokens behind 3000 (2 KV heads): 211 us there, 266
-// here; 300 from empty 96 and 48.
-bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD) {
+// Groups of 1, 2, 4 or 8 heads (the other form takes any) and enough tokens, against one workgroup per (token, KV head) and range
+// of the context, of which a CU holds one (0.054 us a key).
+// One range a token (contexts of up to 16384 tokens): from 288 pairs of token and KV head there are two rounds of those workgroups, where
+// this kernel takes 0.083 us a key while it has at most a workgroup per CU and 0.075 per workgroup on a CU beyond that.  us, there and
+// here, 8 heads a KV head: 288 pairs from empty 48 / 34, behind 16000 tokens 1739 / 1343; 516 pairs behind 15000 2479 / 2226;
+// 256 pairs, one round there, behind 1000 90 / 111; groups of 4, 2 and 1 alike (one head: 288 pairs from empty 24.5 / 20.4).
+// Several ranges a token: the last round no longer has to be full to be short, and only the work counts, 0.054 us per 256 pairs and key
+// there.  384 pairs behind 64000 tokens 5175 / 5257, 448 6030 / 5269; at two workgroups a CU here 704 pairs 9501 / 9628, 768 10374 / 9576;
+// three, 1030 pairs 14688 / 14368.  (Below that line prompts that fill little of a long cache would be faster here, 265 / 196
+// at 288 pairs behind 2000: how much of it they fill is known on the device alone.)
+bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD, int splits) {
   if (HD != ATT_HD || NKV < 1 || NH % NKV) return false;
   const int G = NH / NKV;
   if (G != 1 && G != 2 && G != 4 && G != 8) return false;
   if (g_tune_prefill_exact >= 0) return g_tune_prefill_exact != 0;
-  return (int64_t)T * NKV >= 288;
+  const int64_t pairs = (int64_t)T * NKV;
+  if (splits <= 1) return pairs >= 288;
+  const int64_t per_cu = ((T + 16 / G - 1) / (16 / G) * (int64_t)NKV + num_cus() - 1) / num_cus();
+  return 100 * pairs >= num_cus() * (per_cu == 1 ? 156 : 141 * per_cu);
 }
 
 int launch_attn_prefill_exact(const void* q, const void* kc, const void* vc, const int32_t* block_table, const int32_t* pos, int max_ctx,

@@ -134,7 +134,7 @@ int launch_attn_prefill_tiled(const void* q, const void* kc, const void* vc, con
                               int page_size, void* workspace = nullptr, size_t workspace_bytes = 0);
 // attn_prefill_exact.hip: causal attention of T prompt tokens on the double-precision matrix instruction, the bits of T decode launches
 extern int g_tune_prefill_exact;
-bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD);
+bool attn_prefill_exact_serves(int T, int NH, int NKV, int HD, int splits);      // splits: ranges that the other form would cut a context into
 int launch_attn_prefill_exact(const void* q, const void* kc, const void* vc, const int32_t* block_table, const int32_t* pos, int max_ctx,
                               const void* gate, int64_t gate_bstride, int64_t gate_hstride, void* out, int T, int NH, int NKV);
 // attn_exact.hip: the double-precision form (workspace: f64 partials, plan, f64 copy of q)

@@ -81,9 +81,13 @@ def test_gate_and_output_at_any_address(orc, shift):
     _same(c.run(0, shift), want)
 
 
-@pytest.mark.parametrize("T,NKV,max_len,rows16", [(4096, 2, 4352, True), (2048, 8, 16384, True), (143, 2, 4352, False)])
+@pytest.mark.parametrize("T,NKV,max_len,rows16", [
+    (4096, 2, 4352, True), (2048, 8, 16384, True), (143, 2, 4352, False), (144, 2, 16384, True),
+    # longer caches, cut into ranges: the one-token form keeps the launches of few tokens and those just past a workgroup per CU (512 pairs)
+    (144, 2, 16400, False), (199, 2, 65536, False), (200, 2, 65536, True), (256, 2, 65536, True), (258, 2, 65536, False), (360, 2, 32768, False),
+    (361, 2, 32768, True), (515, 2, 65536, False), (1024, 2, 65536, True)])
 def test_a_handle_keeps_no_workspace_that_its_form_does_not_read(T, NKV, max_len, rows16):
-    """The 16-row form needs the normalised queries (bf16) alone; a token a workgroup also their copy in double (4 bytes a value, eight
+    """The form follows from the shape, as the lines of the table say, and the memory from the form: the 16-row form needs the normalised queries (bf16) alone; a token a workgroup also their copy in double (4 bytes a value, eight
     columns a KV head) and the partial results of its cut."""
     def free_bytes():
         free, total = C.c_size_t(), C.c_size_t()
