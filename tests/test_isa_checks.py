@@ -17,15 +17,32 @@ CSRC = os.path.join(ROOT, "bunker_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 
+def _makefile_flags(source):
+    """The flags that the Makefile compiles ``source`` with: HIPFLAGS and, where its object has them, EXTRA."""
+    mk = open(os.path.join(CSRC, "Makefile")).read()
+    flags = re.search(r"^HIPFLAGS \?= (.*?)(?<!\\)$", mk, flags=re.M | re.S).group(1).replace("\\\n", " ").replace("$(ARCH)", "gfx950").split()
+    for targets, extra in re.findall(r"^(build/[^:=%$]*): EXTRA := (.*)$", mk, flags=re.M):
+        if "build/" + source.replace(".hip", ".o") in targets.split():
+            flags += extra.split()
+    return flags
+
+
 def _compile_to_asm(tmp_path_factory, source):
     if not (os.path.exists(HIPCC) or shutil.which(HIPCC)):
         pytest.skip("hipcc not found")
     out = str(tmp_path_factory.mktemp("isa") / (source + ".s"))
-    flags = re.search(r"^HIPFLAGS \?= (.*?)(?<!\\)$", open(os.path.join(CSRC, "Makefile")).read(), flags=re.M | re.S).group(1)
-    flags = flags.replace("\\\n", " ").replace("$(ARCH)", "gfx950").split()
-    subprocess.check_call([HIPCC, *flags, "-S", "--cuda-device-only", "-o", out, os.path.join(CSRC, source)],
+    subprocess.check_call([HIPCC, *_makefile_flags(source), "-S", "--cuda-device-only", "-o", out, os.path.join(CSRC, source)],
                           stderr=subprocess.DEVNULL)
     return open(out).read()
+
+
+def test_the_checks_compile_what_the_makefile_compiles():
+    """Every source with the command line that make would run for it (a source checked without its own flags is other code)."""
+    out = subprocess.run(["make", "-C", CSRC, "-n", "-B"], check=True, capture_output=True, text=True).stdout
+    lines = {m.group(2): m.group(1).split() for m in re.finditer(r"hipcc (.*) -c (\S+\.hip) -o", out.replace("\\\n", " "))}
+    assert len(lines) >= 16 and any("-mllvm" in f for f in lines.values())
+    for source, flags in lines.items():
+        assert _makefile_flags(source) == flags, source
 
 
 @pytest.fixture(scope="module")
