@@ -18,6 +18,9 @@
 // exponentials bring a page to 5 us (the vector unit stands still while that instruction runs).  1024 tokens x 16 heads from
 // empty 430 -> 196 us, behind 1024 cached 874 -> 482; 8 heads (four tokens a workgroup) 348 -> 134 and 784 -> 284.  Eight waves a
 // workgroup instead of two workgroups of four: 228 and 526.
+// Registers: 256, two workgroups a CU.  What the loop over the one-token passes would carry across the pages (addresses of the tail
+// and of the query copy) is worked out where it is used, behind an index that the compiler cannot see through: with 30 registers
+// in scratch the whole op took 213 us from empty and 493 behind 1024, now 201 and 478.
 #include "attn_args.h"
 
 namespace bk {
@@ -85,7 +88,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
 
   // Q^T to LDS: thread (row, 16 dims)
   {
-    const int row = tid & 15, part = tid >> 4, t = min(t0 + row / G, A.T - 1);
+    int tq = tid;
+    asm volatile("" : "+v"(tq));           // (worked out in every pass, as below the pages)
+    const int row = tq & 15, part = tq >> 4, t = min(t0 + row / G, A.T - 1);
     const uint4* p = (const uint4*)(A.q + ((int64_t)t * A.NH + kvh * G + row % G) * ATT_HD + 16 * part);
     const uint4 a = p[0], b = p[1];
     const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -109,7 +114,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
   d64x4_t O[16];
 #pragma unroll
   for (int n = 0; n < 16; n++) O[n] = (d64x4_t){0.0, 0.0, 0.0, 0.0};
-  double mref = -INFINITY, l = 0.0;
+  double mref = ATT_NO_REF, l = 0.0;
 
   int64_t base = 0;
   if (wave < npages) { base = page_at(wave); load_k(base); }
@@ -152,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
       smax = fmaxf(smax, __shfl_xor(smax, 16));
       smax = fmaxf(smax, __shfl_xor(smax, 32));
       if (smax > -INFINITY && (double)smax > mref + PE_REF_SLACK) {      // the same in the four lanes of a row
-        const double alpha = mref == -INFINITY ? 0.0 : exp(mref - (double)smax);
+        const double alpha = exp(mref - (double)smax);                  // (0 the first time: only zeros have been added)
         mref = (double)smax;
         l *= alpha;
 #pragma unroll
@@ -161,11 +166,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
           for (int v = 0; v < 4; v++) O[n][v] *= alpha;
       }
     }
-    // (a wave that has seen only scores of -inf has no reference yet: their weights are 0, not exp(inf - inf))
-    const double ref = mref == -INFINITY ? 0.0 : mref;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      p[v] = valid[v] ? exp(s[v] - ref) : 0.0;
+      p[v] = valid[v] ? exp(s[v] - mref) : 0.0;
       l += p[v];
     }
     // a key past every row's context has weight 0, but what its slot holds need not be a number: it enters as 0
@@ -187,15 +190,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
   }
 
   // ---- the waves' partial results: weights exp(ref_w - M) per row, then 64 dims at a time through LDS
+  int tl = tid;
+  asm volatile("" : "+v"(tl));             // (the rest works out its addresses here: carried across the pages they would have no registers)
+  const int c16 = tl & 15, r4 = (tl >> 4) & 3, w4 = tl >> 6;
   l += __shfl_xor(l, 16);
   l += __shfl_xor(l, 32);
-  if (q4 == 0) { lds_m[wave][l16] = mref; lds_l[wave][l16] = l; }
+  if (r4 == 0) { lds_m[w4][c16] = mref == ATT_NO_REF ? -INFINITY : mref; lds_l[w4][c16] = l; }
   __syncthreads();                         // (and every wave is done with Q)
-  double M = lds_m[0][l16];
+  double M = lds_m[0][c16];
 #pragma unroll
-  for (int w = 1; w < NW; w++) M = fmax(M, lds_m[w][l16]);
-  const double f = mref == -INFINITY ? 0.0 : exp(mref - M);
-  const int orow = tid >> 4, od = 4 * (tid & 15), ot = t0 + orow / G, head = kvh * G + orow % G;
+  for (int w = 1; w < NW; w++) M = fmax(M, lds_m[w][c16]);
+  const double f = mref == ATT_NO_REF ? 0.0 : exp(mref - M);
+  const int orow = tl >> 4, od = 4 * (tl & 15), ot = t0 + orow / G, head = kvh * G + orow % G;
   double L = 0.0;
   {
     double Mo = lds_m[0][orow];
@@ -210,7 +216,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
 #pragma unroll
     for (int n = 0; n < 4; n++)
 #pragma unroll
-      for (int v = 0; v < 4; v++) lds[(wave * 64 + 16 * n + 4 * v + q4) * PE_PAD + l16] = O[4 * c + n][v] * f;
+      for (int v = 0; v < 4; v++) lds[(w4 * 64 + 16 * n + 4 * v + r4) * PE_PAD + c16] = O[4 * c + n][v] * f;
     __syncthreads();
     if (ot < A.T && (only < 0 || orow / G == only)) {
       uint16_t ob[4];

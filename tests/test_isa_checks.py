@@ -152,3 +152,18 @@ def test_range_checked_loads_carry_their_whole_offset_in_the_lane_operand(tmp_pa
         assert loads, name
         for l in loads:
             assert re.match(r"v\[\d+:\d+\], v\d+, s\[\d+:\d+\], 0 offen\b", l), (name, l)
+
+
+def test_prompt_attention_in_double_precision_walks_its_pages_without_scratch(tmp_path_factory):
+    """attn_prefill_exact.hip is sized for 256 registers and two workgroups a CU.  The forms of 2, 4 and 8 heads use no scratch; that of one
+    head parks a single constant, outside the page loop (the blocks with matrix instructions, and what lies between them)."""
+    asm = _compile_to_asm(tmp_path_factory, "attn_prefill_exact.hip")
+    bodies = {k: v for k, v in _kernels(asm).items() if "attn_prefill_exact_kernel" in k}
+    assert len(bodies) == 4
+    for name, body in bodies.items():
+        meta = re.search(r"\.name:\s+%s\n(.*?)\.wavefront_size" % re.escape(name), asm, flags=re.S).group(1)
+        spills = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", meta).group(1))
+        assert spills <= (2 if "ILi1E" in name else 0), (name, spills)
+        assert int(re.search(r"\.sgpr_spill_count:\s+(\d+)", meta).group(1)) == 0, name
+        first, last = body.index("v_mfma_f64_16x16x4"), body.rindex("v_mfma_f64_16x16x4")
+        assert "scratch_" not in body[first:last], name
