@@ -306,6 +306,10 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = FIRST; r < RF; r += 4) fold4(r);
+        // A narrow tile ignores half of the matrix instruction's results or more.  Their registers stay taken until these blocks are done: a
+        // sum placed in one of them would be overwritten when the instruction ends (the compiler keeps its own instructions at
+        // a distance, but does not see what the blocks write).
+        if (RF < 16) asm volatile("" :: "v"(cn));
         __builtin_amdgcn_sched_barrier(0);
         c = cn; scb = scn; dsw = dsn;
       }

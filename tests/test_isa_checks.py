@@ -167,3 +167,38 @@ def test_prompt_attention_in_double_precision_walks_its_pages_without_scratch(tm
         assert int(re.search(r"\.sgpr_spill_count:\s+(\d+)", meta).group(1)) == 0, name
         first, last = body.index("v_mfma_f64_16x16x4"), body.rindex("v_mfma_f64_16x16x4")
         assert "scratch_" not in body[first:last], name
+
+
+def _registers(operand):
+    m = re.match(r"v\[(\d+):(\d+)\]$|v(\d+)$", operand)
+    return set() if not m else set(range(int(m.group(1)), int(m.group(2)) + 1)) if m.group(1) else {int(m.group(3))}
+
+
+def test_nothing_is_placed_in_the_results_of_a_matrix_instruction_in_flight(tmp_path_factory):
+    """gemm_mfma.hip adds up in asm blocks between a matrix instruction and the first read of its results.  The compiler keeps the distance
+    that the matrix unit needs before a register of its results may be written again, but not from what it cannot look into:
+    up to the last of these blocks no instruction may write any of the sixteen registers (also those that a narrow tile ignores)."""
+    asm = _compile_to_asm(tmp_path_factory, "gemm_mfma.hip")
+    bodies = {k: v for k, v in _kernels(asm).items() if "gemm_q4k_q8_1_mfma_kernel" in k}
+    assert len(bodies) >= 15
+    for name, body in bodies.items():
+        ins = [l.strip().replace(",", "").split() for l in body.split("\n") if re.match(r"\s+[a-z]\w+(\s|$)", l)]
+        checked = 0
+        for i, first in enumerate(ins):
+            if not first[0].startswith("v_mfma_i32_32x32x32_i8"):
+                continue
+            results, written = _registers(first[1]), None
+            assert len(results) == 16
+            for x in ins[i + 1:]:
+                if x[0].startswith(("s_cbranch", "s_branch", "s_endpgm")):
+                    break
+                writes = len(x) > 1 and not x[0].startswith(("ds_write", "global_store", "s_"))
+                if any(_registers(r) & results for r in x[2 if writes else 1:]):
+                    break
+                if writes and _registers(x[1]) & results:
+                    written = written or x
+                    results = results - _registers(x[1])
+                if x[0] == "v_mad_i64_i32":
+                    assert not written, (name, first, written)
+                    checked += 1
+        assert checked >= 7 * 4, (name, checked)
