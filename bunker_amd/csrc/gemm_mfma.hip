@@ -87,13 +87,14 @@ __device__ __forceinline__ MfmaArgs mfma_args_full(const MfmaArgsSw& P) {
 
 enum : int { GX_ROW = 292, GW_ROW = 144, GX_BYTES = 32 * GX_ROW, GW_BYTES = 32 * GW_ROW, G_WAVE_LDS = GX_BYTES + GW_BYTES + 512 };
 
+// Two waves a SIMD, 256 registers; a lone wave gets there by itself, and told so it is scheduled 1 % slower.
 // SWIGLU: the workgroup holds 2 NW waves; waves 0..NW-1 form the tile of 32 gate rows, waves NW..2NW-1 the tile of the
 // same 32 up rows, and the last step writes act = bf16(silu(g) * u) and its Q8_1 block instead of g and u.
 // TR: weight rows of the tile.  16 or 8 (the other rows of the matrix instruction repeat them and are ignored) for launches
 // with so few tiles that the time is the length of one wave's instruction stream: a half or a quarter of the fold per
 // super-block, two or four times the tiles.
 template <int NW, bool SWIGLU, int TR = 32, typename ARGS = MfmaArgs>
-__global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma_kernel(ARGS A_in) {
+__global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void gemm_q4k_q8_1_mfma_kernel(ARGS A_in) {
   const auto& A = mfma_args_full(A_in);
   static_assert(TR == 32 || TR == 16 || TR == 8, "tiles of 32, 16 or 8 weight rows");
   static_assert(!(SWIGLU && TR != 32), "the SwiGLU form quantizes 32 outputs at a time");
@@ -235,8 +236,8 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
                                 (int)((q.w >> 4) & 0x0f0f0f0fu)};
       return (i32x4_t){(int)(q.x & 0x0f0f0f0fu), (int)(q.y & 0x0f0f0f0fu), (int)(q.z & 0x0f0f0f0fu), (int)(q.w & 0x0f0f0f0fu)};
     };
-    auto load_x = [&](int j) {
-      const uint32_t* xp = (const uint32_t*)(myX + j * 36 + 16 * half);
+    auto load_x = [&](const unsigned char* mX, int j) {
+      const uint32_t* xp = (const uint32_t*)(mX + j * 36 + 16 * half);
       return (i32x4_t){(int)xp[0], (int)xp[1], (int)xp[2], (int)xp[3]};
     };
     auto mfma = [](i32x4_t wb, i32x4_t xa) {
@@ -249,31 +250,36 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
     // is a whole number below 2^26 (fp16 has nothing finer than 2^-24), so one 64-bit multiply-add per dot holds the sum exactly
     // where the double form takes a conversion and an FMA.  It starts from the bit pattern of 1.5 * 2^28, whose last bit
     // is worth 2^-24: |sum| < 8 * 2^21.9 * 2^26 < 2^51, so the bits are the double 1.5 * 2^28 + sum * 2^-24 and one
-    // subtraction, exact, gives the double.  Units with a larger, negative or non-finite d8 in any row of the tile fold in double.
-    uint32_t dmax = 0;
-#pragma unroll
-    for (int j = 0; j < 8; j++) dmax = max(dmax, (uint32_t)*(const uint16_t*)(myX + j * 36 + 32));
+    // subtraction, exact, gives the double.  Units with a larger d8 in any row of the tile run the same fold from 0 and convert its
+    // sum in two halves (rounded once): below 128 (values below 16256) d8_j * 2^24 still fits 31 bits, above that the fold
+    // takes d8_j * 2^(24 - s) as long as these are whole numbers, which scales of 2^(s - 14) and more are.  What is left (non-finite
+    // scales, and one of 2^(7 + s) beside one below 2^(s - 14)) is folded in double, one sub-block after the other.  us for
+    // 77 rows x 12288 x 2048 and for gate + up of 1024 x 6144 x 2048, every unit of a kind: scales below 4 24.0 and 171, up to 128 24.9
+    // and 172, above 26.1 and 179, non-finite 30.4 and 221; everything in double, pipelined over the sub-blocks: 25.3 and 184.  (That
+    // form beside this one takes more than the 256 registers of two waves a SIMD.)
     double S1[RF];
-    if (__builtin_expect(__ballot(dmax >= 0x4400u) == 0, 1)) {
+    auto fold = [&](auto small_scales, const unsigned char* mW, const unsigned char* mX, const unsigned char* mS, int s) __attribute__((always_inline)) {
+      constexpr bool SMALL = decltype(small_scales)::value;
+      const float to_whole = SMALL ? 16777216.0f : __builtin_bit_cast(float, (151 - s) << 23);      // 2^(24 - s): d8_j times this is the whole number
       // The fold runs as a pipeline over the sub-blocks: the operands and scale bytes of sub-block j+1 are requested from
       // LDS before sub-block j is folded and its matrix instruction is issued halfway through that fold, when they have
       // arrived; the second half of the fold covers the matrix instruction's latency.
       int64_t S[RF];
-      uint4 q = *(const uint4*)(myW + 16 + 16 * half), qn = q;
-      uint4 scb = *(const uint4*)(stage + 16 * half), scn = scb;
-      uint32_t dsw = *(const uint16_t*)(myX + 32), dsn = dsw;
-      i32x4_t xn = load_x(0);
+      uint4 q = *(const uint4*)(mW + 16), qn = q;
+      uint4 scb = *(const uint4*)mS, scn = scb;
+      uint32_t dsw = *(const uint16_t*)(mX + 32), dsn = dsw;
+      i32x4_t xn = load_x(mX, 0);
       i32x16_t c = mfma(unpack(q, 0), xn), cn = c;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         if (j + 1 < 8) {
-          scn = *(const uint4*)(stage + (j + 1) * 32 + 16 * half);
-          dsn = *(const uint16_t*)(myX + (j + 1) * 36 + 32);
-          xn = load_x(j + 1);
-          if (j & 1) qn = *(const uint4*)(myW + 16 + 32 * ((j + 1) >> 1) + 16 * half);
+          scn = *(const uint4*)(mS + (j + 1) * 32);
+          dsn = *(const uint16_t*)(mX + (j + 1) * 36 + 32);
+          xn = load_x(mX, j + 1);
+          if (j & 1) qn = *(const uint4*)(mW + 16 + 32 * ((j + 1) >> 1));
         }
         __builtin_amdgcn_sched_barrier(0);
-        const int m8 = (int)fma(half_to_f32((uint16_t)dsw), 16777216.0f, 0.0f);      // (one instruction with the conversion; exact)
+        const int m8 = (int)fma(half_to_f32((uint16_t)dsw), to_whole, 0.0f);      // (one instruction with the conversion; exact)
         const uint32_t scv[4] = {scb.x, scb.y, scb.z, scb.w};
         // Four rows: their scales are the four bytes of one word.  (The sums are instructions, not C expressions: integer sums have
         // no order of their own, and the compiler gathers all eight matrix results in front of them; four in a block, because
@@ -287,7 +293,7 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
             asm volatile("v_mad_i64_i32 %0, vcc, %4, %8, %9\n\tv_mad_i64_i32 %1, vcc, %5, %8, %9\n\t"
                          "v_mad_i64_i32 %2, vcc, %6, %8, %9\n\tv_mad_i64_i32 %3, vcc, %7, %8, %9"
                          : "=&v"(S[r]), "=&v"(S[r + 1]), "=&v"(S[r + 2]), "=&v"(S[r + 3])
-                         : "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(m8), "s"(GM_MAGIC) : "vcc");
+                         : "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(m8), "s"(SMALL ? GM_MAGIC : (int64_t)0) : "vcc");
           else
             asm volatile("v_mad_i64_i32 %0, vcc, %4, %8, %0\n\tv_mad_i64_i32 %1, vcc, %5, %8, %1\n\t"
                          "v_mad_i64_i32 %2, vcc, %6, %8, %2\n\tv_mad_i64_i32 %3, vcc, %7, %8, %3"
@@ -314,18 +320,48 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1)) void gemm_q4k_q8_1_mfma
         c = cn; scb = scn; dsw = dsn;
       }
 #pragma unroll
-      for (int r = 0; r < RF; r++) S1[r] = __builtin_bit_cast(double, S[r]) - 0x1.8p28;
+      for (int r = 0; r < RF; r++)
+        S1[r] = SMALL ? __builtin_bit_cast(double, S[r]) - 0x1.8p28
+                      : ldexp(fma((double)(int)(S[r] >> 32), 4294967296.0, (double)(uint32_t)S[r]), s - 24);
+    };
+    uint32_t dmax = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) dmax = max(dmax, (uint32_t)*(const uint16_t*)(myX + j * 36 + 32));
+    if (__builtin_expect(__ballot(dmax >= 0x4400u) == 0, 1)) {
+      fold(std::true_type{}, myW + 16 * half, myX, stage + 16 * half, 0);
     } else {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));         // (addresses worked out here, not kept in registers around the loop over K)
+      const int hf = ln >> 5;
+      const unsigned char *const mW = ldsW + (ln & (TR - 1)) * GW_ROW + 16 * hf, *const mX = ldsX + (ln & 31) * GX_ROW, *const mS = stage + 16 * hf;
+      int s = 0;
+      bool in_double = false;
+      if (__ballot(dmax >= 0x5800u) != 0) {
+        uint32_t top = 0, low = 0xffffu;   // the largest scale and the smallest that is not zero, less one
 #pragma unroll
-      for (int r = 0; r < RF; r++) S1[r] = 0.0;
+        for (int j = 0; j < 8; j++) {
+          const uint32_t d = *(const uint16_t*)(mX + j * 36 + 32) & 0x7fffu;
+          top = max(top, d);
+          low = min(low, d - 1u);
+        }
+        const int wtop = __builtin_amdgcn_readfirstlane((int)wave_max((float)top)), wlow = 1 - __builtin_amdgcn_readfirstlane((int)wave_max(-(float)low));
+        s = max((wtop >> 10) - 21, 0);
+        in_double = wtop >= 0x7c00 || (s > 0 && wlow < ((s + 1) << 10));
+      }
+      if (!in_double) {
+        fold(std::false_type{}, myW + 16 * half, myX, stage + 16 * half, s);
+      } else {
+#pragma unroll
+        for (int r = 0; r < RF; r++) S1[r] = 0.0;
 #pragma unroll 1
-      for (int j = 0; j < 8; j++) {
-        const i32x16_t c = mfma(unpack(*(const uint4*)(myW + 16 + 32 * (j >> 1) + 16 * half), j & 1), load_x(j));
-        const double d8 = (double)half_to_f32(*(const uint16_t*)(myX + j * 36 + 32));
-        const uint4 scb = *(const uint4*)(stage + j * 32 + 16 * half);
-        const uint32_t scv[4] = {scb.x, scb.y, scb.z, scb.w};
+        for (int j = 0; j < 8; j++) {
+          const i32x16_t c = mfma(unpack(*(const uint4*)(mW + 16 + 32 * (j >> 1)), j & 1), load_x(mX, j));
+          const double d8 = (double)half_to_f32(*(const uint16_t*)(mX + j * 36 + 32));
+          const uint4 scb = *(const uint4*)(mS + j * 32);
+          const uint32_t scv[4] = {scb.x, scb.y, scb.z, scb.w};
 #pragma unroll
-        for (int r = 0; r < RF; r++) S1[r] = fma(d8, (double)__mul24(c[r], (int)((scv[r >> 2] >> (8 * (r & 3))) & 0xffu)), S1[r]);
+          for (int r = 0; r < RF; r++) S1[r] = fma(d8, (double)__mul24(c[r], (int)((scv[r >> 2] >> (8 * (r & 3))) & 0xffu)), S1[r]);
+        }
       }
     }
     {

@@ -1,6 +1,7 @@
-"""Batched Q4_K x Q8_1 matmul at the edges of its integer fold: the sums over the eight sub-blocks of a super-block are whole
-numbers of 2^-24 while every activation scale lies in [0, 4); any other scale (larger, negative, infinite, NaN) in a tile sends
-that super-block of the tile through the fold in double.  Both must return the bits of the host loop."""
+"""Batched Q4_K x Q8_1 matmul at the edges of its integer fold.  The sums over the eight sub-blocks of a super-block are whole numbers of
+2^-24 that start from a double's bit pattern while every activation scale of the tile lies in [0, 4); of 2^-24, or of 2^(s - 24) where one
+reaches 2^(7 + s), converted at the end, for larger and negative ones; in double for non-finite scales, and where one reaches 2^(7 + s)
+and another is below 2^(s - 14).  All must return the bits of the host loop."""
 import numpy as np
 import pytest
 
@@ -39,18 +40,23 @@ SHAPES = [(100, 768, 32), (33, 2048, 9), (70, 1024, 33), (200, 512, 77), (130, 2
 
 
 @pytest.mark.parametrize("N,K,B", SHAPES)
-@pytest.mark.parametrize("form", ["edge", "wide", "mixed", "negative", "infinite"])
+@pytest.mark.parametrize("form", ["edge", "edge128", "shifted", "gap", "wide", "mixed", "negative", "infinite"])
 def test_scales_on_both_sides_of_the_integer_fold(orc, N, K, B, form):
     print(f"matmul scales {form} N={N} K={K} B={B}", flush=True)
     g = synth.rng(1200 + N + K + B + len(form))
     W = synth.q4k_random(g, N, K)
     xq = np.stack([orc.pack_q8_1(r) for r in g.standard_normal((B, K)).astype(np.float32)]).reshape(B, K // 32, 36)
     scales = xq[:, :, 32:34].view(np.float16)[..., 0]
-    if form == "edge":            # the largest scale of the integer form (0x43ff), smallest normal and subnormal ones beside it
+    tops = {"edge": 3.998, "edge128": 127.9, "shifted": 255.8, "gap": 255.8}
+    if form in tops:              # the largest scale of a form (0x43ff; 0x57ff: 31 bits; s = 1) with the smallest ones that it takes, or (gap) just below
+        low = {"shifted": 2.0**-13, "gap": 2.0**-13 - 2.0**-24}.get(form, 2.0**-24)
         pick = g.integers(0, 4, scales.shape)
-        scales[pick == 0], scales[pick == 1], scales[pick == 2] = np.float16(3.998), np.float16(2.0**-14), np.float16(2.0**-24)
+        scales[pick == 0], scales[pick == 1], scales[pick == 2] = np.float16(tops[form]), np.float16(2.0**-13), np.float16(low)
+        scales[(pick == 3) & (g.random(scales.shape) < 0.2)] = 0
+        if form == "shifted":
+            scales[(scales > 0) & (scales < np.float16(2.0**-13))] = 0
         xq[:, :, :32] = g.choice(np.array([-128, 127], np.int8), xq[:, :, :32].shape).view(np.uint8)
-    elif form == "wide":          # every super-block of every row through the fold in double
+    elif form == "wide":          # scales of 4 to 32768 in every super-block
         scales[:] = np.exp2(g.integers(2, 16, scales.shape)).astype(np.float16)
     elif form == "mixed":         # one sub-block of a few rows: only some tiles and super-blocks leave the integer form
         for _ in range(3):
@@ -64,8 +70,9 @@ def test_scales_on_both_sides_of_the_integer_fold(orc, N, K, B, form):
     _run(orc, W, np.ascontiguousarray(xq.reshape(B, -1)), N, K, B)
 
 
-def test_largest_sums_of_the_integer_fold(orc):
-    """Every weight 15 with scale 63 and every activation of one sign at the largest scale: the sums reach 8 * 32 * 945 * 128 * 4."""
+@pytest.mark.parametrize("top", [3.998, 127.9, 65504.0, -65504.0])
+def test_largest_sums_of_the_integer_fold(orc, top):
+    """Every weight 15 with scale 63 and every activation of one sign at the largest scale: the sums reach 8 * 32 * 945 * 128 * 4, * 128 and * 65504."""
     N, K, B = 64, 1024, 96
     g = synth.rng(77)
     W = synth.q4k_random(g, N, K).reshape(-1, 144)
@@ -73,7 +80,7 @@ def test_largest_sums_of_the_integer_fold(orc):
     W[:, 16:] = 0xFF
     xq = np.zeros((B, K // 32, 36), np.uint8)
     xq[:, :, :32] = np.where(np.arange(B) % 2 == 0, 0x80, 0x7F)[:, None, None]
-    xq[:, :, 32:34] = np.float16(3.998).view(np.uint16).reshape(1).view(np.uint8)
+    xq[:, :, 32:34] = np.float16(top).view(np.uint16).reshape(1).view(np.uint8)
     xq[:, :, 34:36] = np.float16(-1.0).view(np.uint16).reshape(1).view(np.uint8)
     _run(orc, W, xq.reshape(B, -1), N, K, B)
 
