@@ -529,12 +529,17 @@ int g_tune_gemm_r16 = -1;    // narrow tiles (single batch tile only): 0 off, 1 
 // Waves that share a tile.  A CU holds eight waves of this kernel (their registers; 115 KB of LDS), so w tiles on it run in rounds of
 // 8 / nw: more waves a tile make a round shorter and leave fewer waves idle in the last one, but every wave brings a fixed part (first
 // loads, the sums through LDS), and two waves on a SIMD hide each other's waits.  Which one wins depends on how full the last round
-// is; measured in us on the sizes in brackets (tiles per CU, rounded up: nw = 1 / 2 / 4):
-//   up to one: eight (K >= 2048; 2048 x 6144 at 128 rows 40.8 / 23.6 / 15.5, eight 13.9), up to three: 42.8 / 34.4 / 22.2 (2048 x 6144 at 200),
-//   17.8 / 15.6 / 15.6 (12288 x 2048 at 64); four: 18.2 / 16.3 / 18.6 (2048 x 2048 at 512), 17.8 / 16.7 / 18.5 (8256 x 2048 at 96); five and six:
-//   25.2 / 22.5 / 21.8 (12288 x 2048 at 77), 26.1 / 28.9 / 25.5 (2048 x 2048 at 768); seven and eight: 28.0 / 29.6 / 32.2 (2048 x 2048 at 951),
-//   70.5 / 74.4 / 81.1 (2048 x 6144 at 951); nine and ten: 39.3 / 35.3 / 36.3 (12288 x 2048 at 192), 37.9 / 33.5 / 35.8 (8256 x 2048 at 256);
-//   more: 40.0 / 45.3 / 46.9 (12288 x 2048 at 256), 62.1 / 63.5 / 67.5 (at 384).
+// is, and where two are close on the length of a row, whose stream outweighs the fixed part; us on the sizes in brackets, by tiles per CU,
+// rounded up, nw = 1 / 2 / 4, each at K = 1024, 2048 and 6144:
+//   up to one: eight (K >= 2048; 2048 x 6144 at 128 rows 40.8 / 23.6 / 15.5, eight 13.9);
+//   two (N = 1024 at 512 rows): 10.9 / 9.8 / 8.0, 17.2 / 14.9 / 11.5, 42.5 / 35.6 / 23.8; three (1536): 11.3 / 10.4 / 10.6, 18.1 / 16.0 / 15.6, 44.3 / 37.9 / 33.1;
+//   four (2048): 11.5 / 11.2 / 12.8, 18.8 / 17.5 / 19.2, 45.4 / 39.7 / 41.0; five (2560): 15.7 / 15.3 / 15.4, 26.5 / 23.5 / 22.4, 66.8 / 55.9 / 49.9;
+//   six (3072): 16.3 / 19.0 / 17.9, 27.1 / 29.9 / 25.8, 68.2 / 72.3 / 59.2;
+//   seven (3584): 17.1 / 19.7 / 20.3, 28.4 / 30.9 / 29.3, 70.9 / 73.0 / 67.3 (13312 x 3584 at 128 rows 45.9 / 46.9 / 45.6, x 4096 51.7 / 52.9 / 49.1, 3584 x 4096 at 512 53.0 / - / 53.3);
+//   eight (4096): 17.9 / 21.5 / 22.8, 28.8 / 33.0 / 32.8, 72.3 / 81.8 / 75.7; nine (4608): 24.3 / 23.3 / 25.4, 40.4 / 36.0 / 36.2, 103.3 / 88.6 / 84.7;
+//   ten (5120): 24.7 / 25.8 / 27.8, 40.6 / 40.4 / 40.0 (4900 rows 39.7 / 39.1 / -), 104.1 / 100.1 / 92.9; eleven (5376): 25.0 / 26.9 / 30.3, 40.6 / 42.2 / 43.1, 104.5 / 106.0 / 101.2;
+//   twelve (6144): 25.3 / 28.8 / 32.8, 41.6 / 45.6 / 46.6, 109.7 / 116.0 / 111.0.
+// (Left to two and one although four is 3 to 7 % faster: nine to eleven at K = 6144.  Six at K = 1024 would be 9 % faster with one.)
 static int waves_per_tile(int64_t tiles, int nb) {
   const int64_t per_cu = (tiles + num_cus() - 1) / num_cus();
   int nw;
@@ -542,18 +547,23 @@ static int waves_per_tile(int64_t tiles, int nb) {
   else if (per_cu <= 3) nw = 4;
   else if (per_cu == 4) nw = 2;
   else if (per_cu <= 6) nw = 4;
-  else if (per_cu <= 8) nw = 1;
-  else if (per_cu <= 10) nw = 2;
+  else if (per_cu == 7) nw = nb >= 20 ? 4 : 1;
+  else if (per_cu == 8) nw = 1;
+  else if (per_cu == 9 || (per_cu == 10 && nb >= 8)) nw = 2;
   else nw = 1;
   return nb >= 4 ? nw : std::min(nw, nb >= 2 ? 2 : 1);       // no more than a row has super-blocks
 }
 
-// The SwiGLU form, by pairs of tiles per CU (a CU holds four pairs of lone waves), nw = 1 / 2 / 4 in us, gate and up of 6144 x 2048 unless said:
-// one: 18.6 / 13.7 / 11.8 (32 rows); two: 26.1 / 18.9 / 21.1 (64), 16.3 / 13.1 / 14.9 (3584 x 1024 at 128); three to five: 27.1 / 27.2 / 30.2 (96),
-// 29.5 / 33.1 / 39.8 (160), 18.2 / 22.7 / 27.7 (3584 x 1024 at 256); six: 52.6 / 47.4 / 59.7 (256); more: 54.3 / 60.9 / 77.8 (320), 85.6 / 90.0 / 118 (500).
+// The SwiGLU form, by pairs of tiles per CU (a CU holds four pairs of lone waves), nw = 1 / 2 / 4 in us at K = 1024, 2048 and 6144 (N of gate and up in
+// brackets, at 512 rows):
+// one (512): 12.4 / 10.8 / 9.5, 18.8 / 14.4 / 12.7, 43.9 / 28.1 / 24.7; two (1024): 18.1 / 14.8 / 16.7, 26.9 / 20.1 / 22.4, 65.3 / 42.4 / 44.3;
+// three (1536): 18.4 / 19.7 / 22.3, 28.7 / 28.2 / 32.0, 69.7 / 60.8 / 65.0 (5120 x 3584 at 128 rows 44.9 / 40.8 / 48.1, x 4096 50.1 / 45.0 / 49.3);
+// four (2048): 19.6 / 23.7 / 28.9, 31.1 / 35.1 / 41.7, 77.5 / 76.5 / 85.9; five (2560): 26.8 / 28.7 / 35.4, 42.8 / 41.7 / 51.6, 105.8 / 95.4 / 106.3;
+// six (3072): 34.5 / 33.8 / 42.5, 55.3 / 49.0 / 61.3, 136.9 / 112.2 / 127.7; seven (3328): 34.9 / 38.2 / 48.6, 56.0 / 55.3 / 70.7, 139.3 / 127.2 / 148.4;
+// eight (4096): 37.9 / 42.4 / 55.4, 62.2 / 62.8 / 80.8, 153.6 / 145.2 / 169.3.  (Left to one although two is 6 to 10 % faster: five, seven and eight at 6144.)
 static int waves_per_tile_swiglu(int64_t pairs, int nb) {
   const int64_t per_cu = (pairs + num_cus() - 1) / num_cus();
-  const int nw = per_cu <= 1 ? 4 : (per_cu == 2 || per_cu == 6 ? 2 : 1);
+  const int nw = per_cu <= 1 ? 4 : (per_cu == 2 || per_cu == 6 || (per_cu == 3 && nb >= 12) ? 2 : 1);
   return nb >= 4 ? nw : std::min(nw, nb >= 2 ? 2 : 1);
 }
 

@@ -94,11 +94,14 @@ def _big(g, N, K, B):
     return W, rt.to_device(W), dxq
 
 
-@pytest.mark.parametrize("B", [33, 65, 257, 385, 449, 513, 641, 833, 1025, 1217])
-def test_every_split_of_a_tile_gives_the_same_bits(orc, B):
-    """The number of waves that share a tile follows from the tiles per CU (one to twelve over these batches); whichever it is, the
-    sums are the host loop's."""
-    N, K = 2085, 1024
+@pytest.mark.parametrize("K,B", [(1024, B) for B in (33, 65, 129, 257, 385, 449, 513, 641, 833, 961, 1025, 1153, 1217, 1345)]
+                         + [(2048, 33), (2048, 1153), (5120, 833)])
+def test_every_split_of_a_tile_gives_the_same_bits(orc, K, B):
+    """The number of waves that share a tile follows from the tiles per CU (one to twelve over these batches: 66 tiles of rows, 256 CUs) and,
+    where two choices are close, from the length of a row; eight share one from K = 2048.  Whichever it is, the sums are the host
+    loop's."""
+    N = 2085
+    assert {-(-66 * -(-b // 32) // 256) for b in (33, 65, 129, 257, 385, 449, 513, 641, 833, 961, 1025, 1153, 1217, 1345)} == set(range(1, 13))
     print(f"split N={N} K={K} B={B}", flush=True)
     W, dW, dxq = _big(synth.rng(90 + B), N, K, B)
     dy = rt.cuAlloc(B * N * 4)
