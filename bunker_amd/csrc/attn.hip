@@ -44,7 +44,7 @@ typedef f32x4_t __attribute__((aligned(4))) f32x4_a4_t;      // in a workspace, 
 // flight at every wait is known when the kernel is compiled and a wait covers only the page needed.
 template <int PF, bool NT>
 __global__ __launch_bounds__(ATT_WAVES * 64) void attn_decode_kernel(AttnArgs A) {
-  __shared__ float lds_o2[2][ATT_HD][16];       // exchange buffers for the merge of the four waves, 2 x 16 KiB
+  __shared__ __align__(16) float lds_o2[2][ATT_HD][16];       // exchange buffers for the merge of the four waves, 2 x 16 KiB
   __shared__ float lds_m[ATT_WAVES][16], lds_l[ATT_WAVES][16];
   __shared__ int lds_bt[ATT_MAX_PPS];           // physical page of every page of this split
 
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void attn_decode_kernel(AttnArgs A)
 
 // Merge of the split partials: one workgroup per (head, batch).  The weights exp(m_s - M) of all splits are computed side by side
 // (thread = split) and kept in LDS.  Wave w adds up splits w, w + 4, .. in four dims per lane; the partials of its first PRE are
-// requested before the weights are worked out, all at once, so that the kernel waits for memory once.  The four sums meet in LDS as
+// requested before the weights are worked out, all at once, so that the kernel waits for memory once where they are all.  The four sums meet in LDS as
 // (0 + 1) + (2 + 3), thread = dim.  (A thread per dim with four splits in flight at a time: 4.5 us a launch of 64 splits, now 3.6.)
 template <int PRE>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs A) {
@@ -448,7 +448,9 @@ int launch_attn_decode(const void* q, const void* kc, const void* vc, const int3
     else hipLaunchKernelGGL((attn_decode_kernel<0, false>), grid, block, 0, stream(), A);
   }
   if (splits > 1) {
-    // requests in flight per wave: all of a sequence's splits up to 4, 16 and 64
+    // requests in flight per wave: all of a sequence's splits up to 4, 16 and 64.  Under the balanced plan a long sequence among short
+    // ones owns more than `splits` and its waves walk the rest, four in flight (one of 32768 tokens among 31 of 100, splits 4: 29.0 us with a
+    // thread per dim, now 27.4)
     if (splits <= 4) hipLaunchKernelGGL(attn_merge_kernel<1>, dim3(NH, batch), dim3(256), 0, stream(), A);
     else if (splits <= 16) hipLaunchKernelGGL(attn_merge_kernel<4>, dim3(NH, batch), dim3(256), 0, stream(), A);
     else hipLaunchKernelGGL(attn_merge_kernel<16>, dim3(NH, batch), dim3(256), 0, stream(), A);
