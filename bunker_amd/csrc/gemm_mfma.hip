@@ -87,14 +87,14 @@ __device__ __forceinline__ MfmaArgs mfma_args_full(const MfmaArgsSw& P) {
 
 enum : int { GX_ROW = 292, GW_ROW = 144, GX_BYTES = 32 * GX_ROW, GW_BYTES = 32 * GW_ROW, G_WAVE_LDS = GX_BYTES + GW_BYTES + 512 };
 
-// Two waves a SIMD, 256 registers; a lone wave gets there by itself, and told so it is scheduled 1 % slower.
+// Two waves a SIMD, 256 registers; lone waves and narrow tiles get there by themselves, and told so are scheduled 1 to 3 % slower.
 // SWIGLU: the workgroup holds 2 NW waves; waves 0..NW-1 form the tile of 32 gate rows, waves NW..2NW-1 the tile of the
 // same 32 up rows, and the last step writes act = bf16(silu(g) * u) and its Q8_1 block instead of g and u.
 // TR: weight rows of the tile.  16 or 8 (the other rows of the matrix instruction repeat them and are ignored) for launches
 // with so few tiles that the time is the length of one wave's instruction stream: a half or a quarter of the fold per
 // super-block, two or four times the tiles.
 template <int NW, bool SWIGLU, int TR = 32, typename ARGS = MfmaArgs>
-__global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void gemm_q4k_q8_1_mfma_kernel(ARGS A_in) {
+__global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 || TR < 32 ? 1 : 2) void gemm_q4k_q8_1_mfma_kernel(ARGS A_in) {
   const auto& A = mfma_args_full(A_in);
   static_assert(TR == 32 || TR == 16 || TR == 8, "tiles of 32, 16 or 8 weight rows");
   static_assert(!(SWIGLU && TR != 32), "the SwiGLU form quantizes 32 outputs at a time");
@@ -179,6 +179,11 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void g
   const int stage_slot = ((wcol >> 2) & 1) * 16 + 4 * (wcol >> 3) + (wcol & 3);
   const unsigned char* const myW = ldsW + wcol * GW_ROW;        // int8 operands: weight row col, batch row col,
   const unsigned char* const myX = ldsX + col * GX_ROW;         // bytes 16*half.. of every sub-block
+  // The fold's operands; opaque, so that the two forms of the fold share the addresses instead of each working them out in every super-block
+  // (1 % on launches of 4 to 10 us; the gate/up form is 0.5 % faster without).
+  int off_w = (int)(myW - lds_raw) + 16 * half, off_x = (int)(myX - lds_raw), off_s = (int)(stage - lds_raw) + 16 * half;
+  if (!SWIGLU) asm volatile("" : "+v"(off_w), "+v"(off_x), "+v"(off_s));
+  const unsigned char *const foldW = lds_raw + off_w, *const foldX = lds_raw + off_x, *const foldS = lds_raw + off_s;
 
   double acc[RF];
 #pragma unroll
@@ -266,21 +271,24 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void g
       // arrived; the second half of the fold covers the matrix instruction's latency.
       int64_t S[RF];
       uint4 q = *(const uint4*)(mW + 16), qn = q;
-      uint4 scb = *(const uint4*)mS, scn = scb;
+      // a narrow tile reads the scales of its own rows alone (of a wider read it would wait for the part that it has no use for)
+      using scales_t = std::conditional_t<RF == 16, uint4, std::conditional_t<RF == 8, uint2, uint32_t>>;
+      scales_t scb = *(const scales_t*)mS, scn = scb;
       uint32_t dsw = *(const uint16_t*)(mX + 32), dsn = dsw;
       i32x4_t xn = load_x(mX, 0);
       i32x16_t c = mfma(unpack(q, 0), xn), cn = c;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         if (j + 1 < 8) {
-          scn = *(const uint4*)(mS + (j + 1) * 32);
+          scn = *(const scales_t*)(mS + (j + 1) * 32);
           dsn = *(const uint16_t*)(mX + (j + 1) * 36 + 32);
           xn = load_x(mX, j + 1);
           if (j & 1) qn = *(const uint4*)(mW + 16 + 32 * ((j + 1) >> 1));
         }
         __builtin_amdgcn_sched_barrier(0);
         const int m8 = (int)fma(half_to_f32((uint16_t)dsw), to_whole, 0.0f);      // (one instruction with the conversion; exact)
-        const uint32_t scv[4] = {scb.x, scb.y, scb.z, scb.w};
+        uint32_t scv[RF / 4];
+        __builtin_memcpy(scv, &scb, sizeof scv);
         // Four rows: their scales are the four bytes of one word.  (The sums are instructions, not C expressions: integer sums have
         // no order of their own, and the compiler gathers all eight matrix results in front of them; four in a block, because
         // it puts an idle cycle between neighbouring blocks that it cannot look into.  The products stay in C: only there does
@@ -289,6 +297,10 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void g
           int t[4];
 #pragma unroll
           for (int i = 0; i < 4; i++) t[i] = __mul24(c[r + i], (int)((scv[r >> 2] >> (8 * i)) & 0xffu));
+          // A narrow tile ignores half of the matrix instruction's results or more.  All their registers stay taken up to the first use
+          // of the results: a sum of the sub-block before, placed in one of them, would be overwritten when the instruction ends
+          // (the compiler keeps its own instructions at a distance, but does not see what the blocks write).
+          if (RF < 16 && r == 0) asm volatile("" :: "v"(c));
           if (j == 0)
             asm volatile("v_mad_i64_i32 %0, vcc, %4, %8, %9\n\tv_mad_i64_i32 %1, vcc, %5, %8, %9\n\t"
                          "v_mad_i64_i32 %2, vcc, %6, %8, %9\n\tv_mad_i64_i32 %3, vcc, %7, %8, %9"
@@ -312,10 +324,6 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void g
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = FIRST; r < RF; r += 4) fold4(r);
-        // A narrow tile ignores half of the matrix instruction's results or more.  Their registers stay taken until these blocks are done: a
-        // sum placed in one of them would be overwritten when the instruction ends (the compiler keeps its own instructions at
-        // a distance, but does not see what the blocks write).
-        if (RF < 16) asm volatile("" :: "v"(cn));
         __builtin_amdgcn_sched_barrier(0);
         c = cn; scb = scn; dsw = dsn;
       }
@@ -328,7 +336,7 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void g
 #pragma unroll
     for (int j = 0; j < 8; j++) dmax = max(dmax, (uint32_t)*(const uint16_t*)(myX + j * 36 + 32));
     if (__builtin_expect(__ballot(dmax >= 0x4400u) == 0, 1)) {
-      fold(std::true_type{}, myW + 16 * half, myX, stage + 16 * half, 0);
+      fold(std::true_type{}, foldW, foldX, foldS, 0);
     } else {
       int ln = lane;
       asm volatile("" : "+v"(ln));         // (addresses worked out here, not kept in registers around the loop over K)
@@ -349,7 +357,7 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 ? 1 : 2) void g
         in_double = wtop >= 0x7c00 || (s > 0 && wlow < ((s + 1) << 10));
       }
       if (!in_double) {
-        fold(std::false_type{}, myW + 16 * half, myX, stage + 16 * half, s);
+        fold(std::false_type{}, foldW, foldX, foldS, s);
       } else {
 #pragma unroll
         for (int r = 0; r < RF; r++) S1[r] = 0.0;
