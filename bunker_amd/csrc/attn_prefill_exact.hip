@@ -15,12 +15,12 @@
 // partial results meet through LDS at the end.
 //
 // Bound: the double-precision unit, 128 matrix instructions of 27 ns per page and 16 rows (3.4 us of a SIMD); conversions and
-// exponentials bring a page to 5 us (the vector unit stands still while that instruction runs).  1024 tokens x 16 heads from
-// empty 430 -> 196 us, behind 1024 cached 874 -> 482; 8 heads (four tokens a workgroup) 348 -> 134 and 784 -> 284.  Eight waves a
-// workgroup instead of two workgroups of four: 228 and 526.
+// exponentials bring a page to 5 us (the vector unit stands still while that instruction runs).  The whole op for 1024 tokens x 16
+// heads, a token a workgroup and here: from empty 413 / 197 us, behind 1024 cached 840 / 474, behind 15360 6873 / 4485; 8 heads (four
+// tokens a workgroup) 348 / 134 and 778 / 280.  Eight waves a workgroup instead of two workgroups of four: 16 % and 9 % slower.
 // Registers: 256, two workgroups a CU.  What the loop over the one-token passes would carry across the pages (addresses of the tail
 // and of the query copy) is worked out where it is used, behind an index that the compiler cannot see through: with 30 registers
-// in scratch the whole op took 213 us from empty and 493 behind 1024, now 201 and 478.
+// in scratch the whole op took 213 us from empty and 493 behind 1024, now 201 and 478 (same box).
 #include "attn_args.h"
 
 namespace bk {

@@ -52,7 +52,7 @@ class Prefill:
         False = 1: everything on the library's first stream).  ``gdn_chunked``: the Gated-DeltaNet recurrence in chunks of
         64 tokens on the f32 matrix instruction (the form of the reference's prefill prototypes) instead of the scan;
         state and outputs then agree with T decode steps to ~1e-6 relative, not to the bit.  ``attn_exact=False``: the
-        causal attention of a chunk on the bf16 matrix cores (within 2e-2) instead of the double-precision decode kernel."""
+        causal attention of a chunk on the bf16 matrix cores (within 2e-2) instead of in double precision."""
         if chunk < 1 or chunk > 4096:
             raise ValueError("Prefill: chunk must be 1..4096 tokens")
         self.D, self.env, self.chunk, self.on_attention = D, env, int(chunk), on_attention
