@@ -589,6 +589,7 @@ int bk_tune_set(const char* key, int value) {
   else if (!strcmp(key, "rows")) bk::g_tune_rows = value;
   else if (!strcmp(key, "small_rows")) bk::g_tune_small_rows = value;
   else if (!strcmp(key, "gdn_nt")) bk::g_tune_gdn_nt = value;
+  else if (!strcmp(key, "gemm_tiles")) bk::g_tune_gemm_tiles = value;
   else if (!strcmp(key, "gemm_nw")) bk::g_tune_gemm_nw = value;
   else if (!strcmp(key, "memread_unroll")) bk::g_tune_mr_unroll = value;
   else if (!strcmp(key, "memread_cap")) bk::g_tune_mr_cap = value;

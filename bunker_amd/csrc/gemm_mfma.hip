@@ -35,8 +35,6 @@ typedef __attribute__((ext_vector_type(4))) int i32x4_t;
 typedef __attribute__((ext_vector_type(16))) int i32x16_t;
 typedef __attribute__((ext_vector_type(4))) double f64x4_t;
 
-enum : int { GEPI_F32 = 0, GEPI_BF16 = 1, GEPI_BF16_ADD = 2 };
-
 constexpr int64_t GM_MAGIC = 0x41B8000000000000;      // the bits of 1.5 * 2^28
 
 // rows of the 32x32 accumulator held by a lane: r = 0..15 -> 8*(r/4) + 4*(lane/32) + r%4
@@ -606,6 +604,7 @@ int launch_gemm_group_mfma(const void* xq, int K, int batch, int ngroups, const 
     A.tile_first[i] = tiles;
     tiles += (N[i] + 31) / 32;
   }
+  if (g_tune_gemm_nw == 0 && gemm_tiles_pay(tiles, batch, A.nb, false)) return launch_gemm_tiles(xq, A.nb, batch, ngroups, W, out, res, N, epi);
   // One batch tile and so few weight tiles that CUs would stay empty: tiles of 16 weight rows (twice as many
   // workgroups, half the fold per wave) when that still leaves half of them empty... of 8 when a quarter.  Measured on the
   // 64-tile shapes at batch 32.
@@ -663,6 +662,7 @@ int launch_gemm_swiglu_mfma(const void* xq, int K, int batch, const void* Wg, co
   A.g[0].W = (const uint8_t*)Wg; A.g[0].out = act; A.g[0].N = N;
   A.g[1].W = (const uint8_t*)Wu; A.g[1].N = N;
   A.out_q8 = (uint8_t*)act_q8;
+  if (g_tune_gemm_nw == 0 && gemm_tiles_pay(N / 32, batch, A.nb, true)) return launch_gemm_swiglu_tiles(xq, A.nb, batch, Wg, Wu, N, act, act_q8);
   const int tiles = N / 32, btiles = (batch + 31) / 32;
   for (int i = 0; i < 5; i++) A.tile_first[i] = i ? tiles : 0;
   A.tiles = tiles; A.btiles = btiles;

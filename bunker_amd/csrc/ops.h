@@ -64,6 +64,7 @@ int launch_gemv_rows(int pro, const void* x, const void* norm_w, int K, int batc
                      void* out_q8);
 
 // gemm_mfma.hip
+enum : int { GEPI_F32 = 0, GEPI_BF16 = 1, GEPI_BF16_ADD = 2 };      // what a matmul writes
 extern int g_tune_small_rows;
 extern int g_tune_gemm_nw, g_tune_gemm_r16, g_tune_gdn_nt, g_tune_attn_nt, g_tune_attn_bal;
 int launch_gemm_group_mfma(const void* xq, int K, int batch, int ngroups, const void* const* W, void* const* out,
@@ -71,6 +72,12 @@ int launch_gemm_group_mfma(const void* xq, int K, int batch, int ngroups, const 
 int launch_gemm_swiglu_mfma(const void* xq, int K, int batch, const void* Wg, const void* Wu, int N, void* act, void* act_q8);
 int launch_gemm_q4k_q8_1_mfma(const void* W, const void* xq, void* y, int N, int K, int batch, int out_dtype,
                               const void* residual);
+
+// gemm_tiles.hip: the same products in tiles of 64 x 64 (nb = K / 256)
+extern int g_tune_gemm_tiles;
+bool gemm_tiles_pay(int tiles, int batch, int nb, bool swiglu);
+int launch_gemm_tiles(const void* xq, int nb, int batch, int n, const void* const* W, void* const* out, const void* const* res, const int* N, const int* epi);
+int launch_gemm_swiglu_tiles(const void* xq, int nb, int batch, const void* Wg, const void* Wu, int N, void* act, void* act_q8);
 
 // glue.hip
 enum : int { EW_CAST_OP = 0, EW_ADD_OP = 1, EW_SWIGLU_OP = 2 };

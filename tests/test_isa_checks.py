@@ -202,3 +202,38 @@ def test_nothing_is_placed_in_the_results_of_a_matrix_instruction_in_flight(tmp_
                     assert not written, (name, first, written)
                     checked += 1
         assert checked >= 7 * 4, (name, checked)
+
+
+def test_results_of_the_tiles_matmul_are_first_read_where_the_compiler_sees_it(tmp_path_factory):
+    """gemm_tiles.hip multiplies and adds in asm blocks.  The compiler keeps the distance that the results of a matrix instruction need
+    before they are read or written, but does not look into the blocks: of every int8 product some result must be read by
+    an instruction outside them first, and none may be written before that.  Three waves share a SIMD: 168 registers, no scratch."""
+    asm = _compile_to_asm(tmp_path_factory, "gemm_tiles.hip")
+    bodies = {k: v for k, v in _kernels(asm).items() if "gemm_q4k_q8_1_tiles_kernel" in k}
+    assert len(bodies) == 2
+    for name, body in bodies.items():
+        meta = re.search(r"\.name:\s+%s\n(.*?)\.wavefront_size" % re.escape(name), asm, flags=re.S).group(1)
+        assert int(re.search(r"\.vgpr_count:\s+(\d+)", meta).group(1)) <= 168, name
+        assert int(re.search(r"\.vgpr_spill_count:\s+(\d+)", meta).group(1)) == 0, name
+        assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", meta).group(1)) == 0, name
+        ins, inside = [], False
+        for l in body.split("\n"):
+            inside = True if "#ASMSTART" in l else False if "#ASMEND" in l else inside
+            if re.match(r"\s+[a-z]\w+(\s|$)", l):
+                ins.append((inside, l.strip().replace(",", "").split()))
+        checked = 0
+        for i, (_, first) in enumerate(ins):
+            if not first[0].startswith("v_mfma_i32_16x16x32_i8"):
+                continue
+            results = _registers(first[1])
+            assert len(results) == 4
+            for in_block, x in ins[i + 1:]:
+                if x[0].startswith(("s_cbranch", "s_branch", "s_endpgm")):
+                    break
+                writes = len(x) > 1 and not x[0].startswith(("ds_write", "global_store", "s_"))
+                if any(_registers(r) & results for r in x[2 if writes else 1:]):
+                    assert not in_block, (name, first, x)
+                    checked += 1
+                    break
+                assert not (writes and _registers(x[1]) & results), (name, first, x)
+        assert checked >= 2 * 32, (name, checked)
