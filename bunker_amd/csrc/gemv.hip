@@ -276,22 +276,28 @@ struct XF {
   float sum_c;   // sum of the 32 activations of sub-block c (for the lane's share of the mins)
 };
 
-__device__ __forceinline__ float nibdot4(uint32_t n4, const float* x, float acc) {
-  acc = fmaf((float)(n4 & 0xffu), x[0], acc);
-  acc = fmaf((float)((n4 >> 8) & 0xffu), x[1], acc);
-  acc = fmaf((float)((n4 >> 16) & 0xffu), x[2], acc);
-  acc = fmaf((float)(n4 >> 24), x[3], acc);
+// Four bytes' low nibbles (SHIFT 0) or high ones (SHIFT 4) against four activations, times 2^-24: a nibble alone in 16 bits is a subnormal half, and the
+// mixed FMA reads it as it is, in either half of a register.
+typedef __attribute__((ext_vector_type(2))) _Float16 half2_t;
+template <int SHIFT>
+__device__ __forceinline__ float nibdot4(uint32_t q, const float* x, float acc) {
+  const half2_t n02 = __builtin_bit_cast(half2_t, (q >> SHIFT) & 0x000f000fu), n13 = __builtin_bit_cast(half2_t, (q >> (SHIFT + 8)) & 0x000f000fu);
+  acc = fmaf((float)n02[0], x[0], acc);
+  acc = fmaf((float)n13[0], x[1], acc);
+  acc = fmaf((float)n02[1], x[2], acc);
+  acc = fmaf((float)n13[1], x[3], acc);
   return acc;
 }
 
-// The lane's 32 activations of super-block blk.  Lanes c and c ^ 1 hold the two halves of sub-blocks 2g and 2g+1, so the
-// sum of sub-block c is the lane's own half plus its neighbour's.  Every lane of the wave takes part in the exchange.
-__device__ __forceinline__ void load_xf(XF& x, const float* __restrict__ xf, int blk, int c, bool active) {
+// The lane's 32 activations of super-block blk (taken from at(i), float4 i of the row).  Lanes c and c ^ 1 hold the two halves of sub-blocks 2g and
+// 2g+1, so the sum of sub-block c is the lane's own half plus its neighbour's.  Every lane of the wave takes part in the exchange.
+template <typename AT>
+__device__ __forceinline__ void load_xf(XF& x, AT at, int blk, int c, bool active) {
   const int g = c >> 1, half = c & 1;
-  const float4* p0 = (const float4*)(xf + (active ? blk : 0) * 256 + 64 * g + 16 * half);
+  const int p0 = (active ? blk : 0) * 64 + 16 * g + 4 * half;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const float4 a = p0[i], b = p0[8 + i];
+    const float4 a = at(p0 + i), b = at(p0 + 8 + i);
     x.lo[4 * i] = a.x; x.lo[4 * i + 1] = a.y; x.lo[4 * i + 2] = a.z; x.lo[4 * i + 3] = a.w;
     x.hi[4 * i] = b.x; x.hi[4 * i + 1] = b.y; x.hi[4 * i + 2] = b.z; x.hi[4 * i + 3] = b.w;
   }
@@ -307,22 +313,47 @@ __device__ __forceinline__ void load_xf(XF& x, const float* __restrict__ xf, int
   x.sum_c = half ? s1 : s0;
 }
 
+// The dots are formed 2^-24 smaller than they are (nibdot4).  Activations that are all below 2^-63 (no exponent has one of its two top bits) are taken times
+// 2^64, so that nothing is lost below the normal range; what has to be done to the result is returned.
+constexpr uint32_t XF_NOT_TINY = 0x60000000u;
+template <int NR>
+__device__ __forceinline__ float lift_tiny(XF (&x)[NR], bool tiny) {
+  if (__builtin_expect(!tiny, 1)) return 1.0f;
+#pragma unroll
+  for (int r = 0; r < NR; r++) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) { x[r].lo[i] *= 0x1p64f; x[r].hi[i] *= 0x1p64f; }
+    x[r].sum_c *= 0x1p64f;
+  }
+  return 0x1p-64f;
+}
+// the same for the activations that the lanes of a wave hold between them
+template <int NR>
+__device__ __forceinline__ float lift_tiny(XF (&x)[NR]) {
+  uint32_t bits = 0;
+#pragma unroll
+  for (int r = 0; r < NR; r++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) bits |= __float_as_uint(x[r].lo[i]) | __float_as_uint(x[r].hi[i]);
+  return lift_tiny(x, __ballot(bits & XF_NOT_TINY) == 0);
+}
+
 __device__ __forceinline__ float slot_dot_f32(const uint4& hdr, const uint4& q, const XF& x, const ScaleSel& sel) {
   const float d = half_to_f32((uint16_t)(hdr.x & 0xffffu));
   const float dmin = half_to_f32((uint16_t)(hdr.x >> 16));
   uint32_t sc, m;
   lane_scale_min(sel, hdr.y, hdr.z, hdr.w, sc, m);
-  const float fsc = d * (float)sc;
+  const float fsc = (d * (float)sc) * 16777216.0f;
   const float fm = (dmin * (float)m) * x.sum_c;
   float a = 0.0f, b = 0.0f;
-  a = nibdot4(q.x & 0x0f0f0f0fu, &x.lo[0], a);
-  b = nibdot4((q.x >> 4) & 0x0f0f0f0fu, &x.hi[0], b);
-  a = nibdot4(q.y & 0x0f0f0f0fu, &x.lo[4], a);
-  b = nibdot4((q.y >> 4) & 0x0f0f0f0fu, &x.hi[4], b);
-  a = nibdot4(q.z & 0x0f0f0f0fu, &x.lo[8], a);
-  b = nibdot4((q.z >> 4) & 0x0f0f0f0fu, &x.hi[8], b);
-  a = nibdot4(q.w & 0x0f0f0f0fu, &x.lo[12], a);
-  b = nibdot4((q.w >> 4) & 0x0f0f0f0fu, &x.hi[12], b);
+  a = nibdot4<0>(q.x, &x.lo[0], a);
+  b = nibdot4<4>(q.x, &x.hi[0], b);
+  a = nibdot4<0>(q.y, &x.lo[4], a);
+  b = nibdot4<4>(q.y, &x.hi[4], b);
+  a = nibdot4<0>(q.z, &x.lo[8], a);
+  b = nibdot4<4>(q.z, &x.hi[8], b);
+  a = nibdot4<0>(q.w, &x.lo[12], a);
+  b = nibdot4<4>(q.w, &x.hi[12], b);
   const float f0 = dpp_f32<DPP_PAIR_EVEN>(fsc);
   const float f1 = dpp_f32<DPP_PAIR_ODD>(fsc);
   return (f0 * a + f1 * b) - fm;
@@ -330,15 +361,19 @@ __device__ __forceinline__ float slot_dot_f32(const uint4& hdr, const uint4& q, 
 
 // Rows of up to 8 * NR super-blocks: the LDS staging of gemv_q4k_q8_1_lds_kernel (RPI contiguous rows per wave step,
 // every 128-byte line requested once, the next step's rows in flight during the arithmetic), for any nb: the lanes past
-// the row fold a clamped block, its scales and the activations replaced by zeros.  What bounds it is latency and the reads of x: with one row per wave (the
-// form this replaces) every row pulled all of x through the L2 twice, 134 MB for a 9.4 MB matrix.  Back to back on cold
-// weights: 4096 x 4096 13.2 -> 5.5 us, 12288 x 2048 18.3 -> 6.4, 151936 x 2048 110 -> 41 (then bound by vector issue: about
-// 95 instructions per 32 weights of a lane), 50000 x 6144 208 -> 51 (3.4 TB/s).
+// the row fold a clamped block, its scales and the activations replaced by zeros.  What bounds it is latency (launch, one memory round trip, x to the
+// lanes, fold) up to a few thousand rows, then vector issue.  The workgroup reads x once and hands it to its four waves through LDS: read by every
+// wave in 16-byte pieces 64 bytes apart, x was 33 MB through the caches for a 9.4 MB matrix, and the weights were only asked for behind it.  With that and
+// the mixed FMAs (fifteen instructions for eight weights where conversions made it nineteen), us back to back on cold weights: 1024 x 1024 2.75 -> 2.6,
+// 4096 x 4096 6.1 -> 5.15 (5.46 -> 4.35 on weights in the memory-side cache), 2048 x 6144 5.85 -> 4.6, 12288 x 2048 6.85 -> 5.7, 40000 x 1024 13.4 -> 10.6,
+// 151936 x 2048 43.3 -> 38-41, 50000 x 6144 51.7 -> 42 (4.1 TB/s).
 template <int NR, int RPI>
 __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
     const uint8_t* __restrict__ W, const float* __restrict__ xf, float* __restrict__ y, int N, int nb, int nwg) {
-  constexpr int LOADS = StageRegs<NR, RPI>::LOADS;
-  __shared__ uint4 tiles[GEMV_WAVES][StageRegs<NR, RPI>::PIECES];
+  constexpr int LOADS = StageRegs<NR, RPI>::LOADS, TILE = StageRegs<NR, RPI>::PIECES, XLOADS = NR * 8 * 64 / (GEMV_WAVES * 64);
+  __shared__ uint4 lds[GEMV_WAVES * TILE + NR * 8 * 64];
+  __shared__ int4 not_tiny;
+  uint4* const xlds = lds + GEMV_WAVES * TILE;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int c = lane & 7, b = lane >> 3;
   const ScaleSel sel = make_scale_sel(c);
@@ -346,16 +381,16 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
   const int64_t last_piece = (int64_t)N * row_pieces - 1;
   const int step = nwg * GEMV_WAVES * RPI;
   int row0 = (blockIdx.x * GEMV_WAVES + wv) * RPI;
-  uint4* tile = tiles[wv];
+  uint4* tile = lds + wv * TILE;
 
   XF x[NR];
   uint32_t in_row[NR];            // all ones, or zero past the row: a lane there has d = dmin = 0 and adds nothing, whatever its block holds
 #pragma unroll
-  for (int r = 0; r < NR; r++) {
-    load_xf(x[r], xf, r * 8 + b, c, r * 8 + b < nb);
-    in_row[r] = r * 8 + b < nb ? ~0u : 0u;
-  }
-
+  for (int r = 0; r < NR; r++) in_row[r] = r * 8 + b < nb ? ~0u : 0u;
+  // x first (all workgroups but the first ones find it in a cache), the first rows right behind it: one memory round trip for both
+  uint4 xp[XLOADS];
+#pragma unroll
+  for (int u = 0; u < XLOADS; u++) xp[u] = ((const uint4*)xf)[min((int)threadIdx.x + GEMV_WAVES * 64 * u, nb * 64 - 1)];
   StageRegs<NR, RPI> g;
   auto request = [&](int r0) {
     const int64_t base = (int64_t)r0 * row_pieces;
@@ -367,6 +402,21 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
     }
   };
   request(min(row0, N - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  // piece p lies at p ^ ((p >> 4) & 3): the eight lanes of a super-block read from eight different banks
+  auto at_piece = [](int p) { return p ^ ((p >> 4) & 3); };
+  uint32_t bits = 0;
+#pragma unroll
+  for (int u = 0; u < XLOADS; u++) {
+    xlds[at_piece(threadIdx.x + GEMV_WAVES * 64 * u)] = xp[u];
+    bits |= xp[u].x | xp[u].y | xp[u].z | xp[u].w;
+  }
+  ((int*)&not_tiny)[wv] = __ballot(bits & XF_NOT_TINY) != 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < NR; r++) load_xf(x[r], [&](int i) { return __builtin_bit_cast(float4, xlds[at_piece(i)]); }, r * 8 + b, c, r * 8 + b < nb);
+  const int4 f = not_tiny;
+  const float unlift = lift_tiny(x, __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w) == 0);
   while (row0 < N) {
 #pragma unroll
     for (int u = 0; u < LOADS; u++)
@@ -392,7 +442,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
 #pragma unroll
     for (int i = 0; i < RPI; i++) {
       const float tot = wave_sum(acc[i]);
-      if (lane == 0 && row0 + i < N) y[row0 + i] = tot;
+      if (lane == 0 && row0 + i < N) y[row0 + i] = tot * unlift;
     }
     row0 += step;
   }
@@ -413,12 +463,13 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_generic_kernel(
     float acc = 0.0f;
     for (int r = 0; r < rounds; r++) {
       const int blk = r * 8 + (lane >> 3);
-      XF x;
-      load_xf(x, xf, blk, c, blk < nb);
+      XF x[1];
+      load_xf(x[0], [&](int i) { return ((const float4*)xf)[i]; }, blk, c, blk < nb);
+      const float unlift = lift_tiny(x);
       const int bo = (blk < nb ? blk : 0) * 144;
       uint4 hdr = *(const uint4*)(rp + bo);
       if (blk >= nb) hdr.x = 0;                             // past the row: d = dmin = 0
-      acc += slot_dot_f32(hdr, *(const uint4*)(rp + bo + 16 + 16 * c), x, sel);
+      acc += slot_dot_f32(hdr, *(const uint4*)(rp + bo + 16 + 16 * c), x[0], sel) * unlift;
     }
     const float tot = wave_sum(acc);
     if (lane == 0) y[row] = tot;
@@ -437,8 +488,8 @@ int launch_gemv_q4k_f32(const void* W, const float* x, float* y, int N, int K) {
   BK_REQUIRE(((uintptr_t)W & 15) == 0 && ((uintptr_t)x & 15) == 0, "gemv_q4k_f32: W and x must be 16-byte aligned");
   const int nb = K / 256, rounds = (nb + 7) / 8;
   const uint8_t* w = (const uint8_t*)W;
-  // Two rows per wave step.  One where two would leave CUs without a workgroup and the rows are short (1024 x 1024: 3.6 us
-  // against 4.0; rows of 6144 lose with one, 2048 of them 5.8 us against 5.3).  Four do not help a long matrix
+  // Two rows per wave step.  One where two would leave CUs without a workgroup and the rows are short (1024 x 1024 2.55 us
+  // against 3.13; rows of 6144 lost with one, 2048 of them 5.8 us against 5.3).  Four did not help a long matrix
   // (151936 x 2048: 41.1 us with two, 41.2 with four).
   switch (rounds) {
     case 1: if (N <= GEMV_WAVES * 2 * num_cus()) launch_f32_lds<1, 1>(w, x, y, N, nb); else launch_f32_lds<1, 2>(w, x, y, N, nb); break;

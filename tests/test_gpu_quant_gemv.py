@@ -352,3 +352,26 @@ def test_gemm_mfma_every_split_of_k_returns_the_same_bits(orc, dev, N, K, B):
     finally:
         rt.tune_set("gemm_nw", 0)
         rt.tune_set("gemm_r16", -1)
+
+
+@pytest.mark.parametrize("exponent", [-139, -126, -100, -64, -62, 0, 60, 100])
+@pytest.mark.parametrize("N,K", [(5, 256), (300, 1024), (1030, 2304), (2100, 2048), (9, 6144), (7, 6400)])
+def test_gemv_q4k_f32_activations_of_any_magnitude(orc, dev, N, K, exponent):
+    """The dots run on nibbles as subnormal halves, 2^-24 below their value; activations down to the smallest must keep their bits, in every form of the
+    kernel (x shared by the workgroup or not, one to three rounds, rows of any length).  The same activations times a power of two give the
+    same result times that power, unless it leaves the normal range: there half a unit of its last place (rows of more than 6144: of every lane's
+    share of every round of 2048, which leave that range before they are added)."""
+    print(f"gemv f32 magnitude N={N} K={K} 2^{exponent}", flush=True)
+    g = synth.rng(9 + N + K)
+    W = synth.q4k_random(g, N, K)
+    x = (1 + g.random(K)).astype(np.float32) * g.choice(np.array([-1, 1], np.float32), K)
+    if exponent < -126:      # subnormal activations: few significant bits, so that the scaling is exact
+        x = np.round(x * 1024) / np.float32(1024)
+    ys = []
+    for e in (0, exponent):
+        dy = dev.empty(N * 4)
+        rt.gemv_q4k_f32(dev.up(W), dev.up((x.astype(np.float64) * 2.0**e).astype(np.float32)), dy, N, K)
+        ys.append(rt.from_device(dy, (N,), np.float32))
+    want = ys[0].astype(np.float64) * 2.0**exponent
+    assert np.isfinite(ys[1]).all() and (np.abs(ys[1].astype(np.float64) - want) <= 2.0**-150 * (1 if K <= 6144 else 64 * -(-K // 2048))).all()
+    _assert_rel(ys[0], orc.gemv_q4k_f32(W, x, N, K, acc64=True))
