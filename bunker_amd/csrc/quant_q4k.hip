@@ -9,10 +9,11 @@
 // One lane per sub-block: the fit is a chain of f32 sums in ascending element order, so a lane runs it exactly
 // as the host loop does (one IEEE operation per written operation) and the bytes equal the host's.  The eight
 // lanes of a super-block meet only for the two maxima (order-free), the 12 scale bytes (an OR) and the nibble
-// pairing of sub-blocks 2g and 2g+1.  The work is ALU-bound, not memory-bound: about 610 vector instructions per candidate
+// pairing of sub-blocks 2g and 2g+1.  The work is ALU-bound, not memory-bound: about 580 vector instructions per candidate
 // grid and wave, 21 grids, at 1.2-1.3 ns each on a SIMD, the rate of two-operand f32 operations.  What the search does not
 // need (packed copies of the levels, integer conversions, the wrap-around of nearest_int for quotients that large do not
-// occur) is kept out of it: 6144 x 2048 from bf16 128.5 -> 111 us, 32768 x 6144 1918 -> 1625.  Four waves per SIMD instead
+// occur) is kept out of it: 6144 x 2048 from bf16 128.5 -> 111 us, 32768 x 6144 1918 -> 1625; with levels in three or four
+// instructions instead of five where a wave's values allow it (grid_level_unit) 110.4 -> 105.6 us.  Four waves per SIMD instead
 // of three (128 registers) spill 21 and take 129 us.
 #include <type_traits>
 
@@ -35,6 +36,14 @@ __device__ __forceinline__ float grid_level(float iscale, float x, float mn) {
   if (!WIDE) return __builtin_amdgcn_fmed3f(__fsub_rn(t, 12582912.f), 0.f, 15.f);
   const float m = __uint_as_float((__float_as_uint(t) & 0x007fffffu) | 0x4b000000u);
   return __fsub_rn(__builtin_amdgcn_fmed3f(m, 12582912.f, 12582927.f), 12582912.f);
+}
+// The same where every |iscale * (x - mn)| is small enough for nearest_int, 0 < mx - mn < 1 (then iscale > 0 and x - mn < 1) and
+// iscale * (x - mn) rounds to 15 at most (TOP: where that is not known): v_rndne rounds to nearest even as the pair of additions does,
+// and the subtraction's own clamp to [0, 1] is the clamp to 0.  (With a maximum in its place 107.4 us, with the pair of additions 3 us more.)
+template <bool TOP>
+__device__ __forceinline__ float grid_level_unit(float iscale, float x, float mn) {
+  const float l = __builtin_rintf(__fmul_rn(iscale, __builtin_amdgcn_fmed3f(__fsub_rn(x, mn), 0.f, 1.f)));
+  return TOP ? fminf(l, 15.f) : l;
 }
 __device__ __forceinline__ uint16_t f32_to_half_rne(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
 
@@ -122,10 +131,12 @@ __global__ __launch_bounds__(256) void quantize_q4k_kernel(const void* __restric
     for (int is = 0; is <= NSTEP; is++) {
       iscale = __fdiv_rn(__fadd_rn(__fadd_rn(-1.f, __fmul_rn(0.1f, (float)is)), (float)NMAX), __fsub_rn(mx, mn));
       float sum_l = 0.f, sum_l2 = 0.f, sum_xl = 0.f;
-      auto levels_and_sums = [&](auto wide) {
+      auto levels_and_sums = [&](auto kind) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 32; i++) {
-          lf[i] = grid_level<decltype(wide)::value>(iscale, x[i], mn);
+          constexpr int KIND = decltype(kind)::value;
+          if constexpr (KIND >= 2) lf[i] = grid_level_unit<KIND == 3>(iscale, x[i], mn);
+          else lf[i] = grid_level<KIND == 1>(iscale, x[i], mn);
           const float wl = __fmul_rn(w[i], lf[i]);
           sum_l = __fadd_rn(sum_l, wl);
           sum_l2 = __fadd_rn(sum_l2, __fmul_rn(wl, lf[i]));
@@ -135,8 +146,10 @@ __global__ __launch_bounds__(256) void quantize_q4k_kernel(const void* __restric
       // every |iscale * (x - mn)| is at most the one of the two ends; a fitted min that met the maximum (sub-blocks whose
       // values differ by a few ulps) makes it infinite or NaN
       const float reach = fabsf(iscale) * fmaxf(fabsf(mx - mn), fabsf(lowest - mn));
-      if (__any(!(reach <= 1048576.f))) levels_and_sums(std::true_type{});
-      else levels_and_sums(std::false_type{});
+      if (__any(!(reach <= 1048576.f))) levels_and_sums(std::integral_constant<int, 1>{});
+      else if (__any(!(mx - mn > 0.f && mx - mn < 1.f))) levels_and_sums(std::integral_constant<int, 0>{});
+      else if (is <= 14) levels_and_sums(std::integral_constant<int, 2>{});      // 15.4 at the maximum, a few roundings aside
+      else levels_and_sums(std::integral_constant<int, 3>{});
       const float D = __fsub_rn(__fmul_rn(sum_w, sum_l2), __fmul_rn(sum_l, sum_l));
       if (D > 0.f) {
         float this_scale = __fdiv_rn(__fsub_rn(__fmul_rn(sum_w, sum_xl), __fmul_rn(sum_x, sum_l)), D);

@@ -72,6 +72,23 @@ def test_quantize_q4k_sub_blocks_a_few_ulps_wide(orc, base):
     assert np.array_equal(got, ref), f"{np.count_nonzero(got != ref)} bytes differ"
 
 
+@pytest.mark.parametrize("top", [0.5, 1.0, 1.001, 60.0])
+def test_quantize_q4k_ranges_around_one(orc, top):
+    """The search has a shorter form for waves whose sub-blocks all span less than 1, with levels cut at 15 only where the grid can pass it: spans just below,
+    at and above 1, mins fitted above the lowest value (outliers below a narrow bulk), sub-blocks of one sign; the bytes stay the checker's."""
+    g = synth.rng(4300)
+    w = g.uniform(0, 1, (96, 32, 32)).astype(np.float32)
+    w[:, :, 0], w[:, :, 1] = 0, 1
+    w[::4] -= 0.5
+    w[1::4] = -w[1::4]
+    w[2::4, :, 2:] = 0.9 + 0.1 * w[2::4, :, 2:]
+    w[3::4] = w[3::4] * -0.01 - 0.99
+    w[3::4, :, 0] = -1.9
+    w = np.ascontiguousarray((w * np.float32(top)).reshape(96, 1024))
+    got, ref = _quantize_dev(w, rt.F32), orc.quantize_q4k(w)
+    assert np.array_equal(got, ref), f"{np.count_nonzero(got != ref)} bytes differ"
+
+
 def test_quantize_q4k_rejects_bad_shapes():
     d = rt.to_device(np.zeros(512, np.float32))
     with pytest.raises(rt.BunkerError):
