@@ -121,6 +121,95 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_q8_1_lds_kernel(
   }
 }
 
+// Rows that do not fill whole rounds (K is no multiple of 2048).  The super-blocks of a step's RPI rows are numbered through, slot group
+// b of round r takes number 8 r + b, whichever row that is in: S rounds for all of them, S = ceil(RPI nb / 8), where rounds row by row
+// would leave up to half of the lanes without work.  A lane's activation slices still depend on the lane alone.  nb lies between NB0
+// and NB1 = 8 S / RPI, so that most rounds are known to lie in one row; in the others a lane adds its term to the row it is in.
+// Bound by the instructions of a round (about 70 for 64 slots) and the waves that the registers allow, no longer by idle lanes: 1.5 to 2 times the
+// rounds made K = 4608 with 67527 rows 43.9 us (4.0 TB/s), here 31.4 (5.6); K = 2560, 100000 rows 34.0 -> 26.1 (5.5 TB/s).  Without the activation row
+// through LDS, with a grid of two steps a wave and all of a step's operands in registers at once (a wave a SIMD less): 38.8 and 30.2.
+// Waves a SIMD that the registers allow (what a lane keeps for the slots is ten registers a round).
+constexpr int flat_waves(int S, int RPI) { return S <= 1 ? 8 : S == 2 ? 6 : S == 3 ? 5 : S <= 5 || RPI == 2 ? 4 : 3; }
+template <int S, int RPI, int EPI>
+__global__ __launch_bounds__(GEMV_WAVES * 64, flat_waves(S, RPI)) void gemv_q4k_q8_1_flat_kernel(
+    const uint8_t* __restrict__ W, const uint8_t* __restrict__ xq_all, void* __restrict__ y,
+    const uint16_t* __restrict__ res, int N, int nb) {
+  constexpr int NB1 = 8 * S / RPI, NB0 = 8 * (S - 1) / RPI + 1;
+  static_assert(RPI == 2 || RPI == 4, "the sums of two or four rows share their steps");
+  __shared__ uint4 tiles[GEMV_WAVES][S * 72];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int wave = blockIdx.x * GEMV_WAVES + wv;
+  const int bidx = blockIdx.y;
+  const uint8_t* xq = xq_all + (int64_t)bidx * nb * 8 * 36;
+  const int c = lane & 7, b = lane >> 3;
+  const ScaleSel sel = make_scale_sel(c);
+  const int64_t row_bytes = (int64_t)nb * 144, last_piece_off = (int64_t)N * row_bytes - 16, ybase = (int64_t)bidx * N;
+  const bool odd = c & 1;
+  const int step = gridDim.x * GEMV_WAVES * RPI, pieces = RPI * nb * 9;
+  int row0 = wave * RPI;
+  uint4* tile = tiles[wv];
+
+  constexpr int LOADS = (S * 72 + 63) / 64;
+  uint4 g[LOADS];
+  auto load = [&](int row) __attribute__((always_inline)) {
+    const uint8_t* rp = W + (int64_t)row * row_bytes;
+    const int last = (int)min((int64_t)(pieces - 1), (last_piece_off - (int64_t)row * row_bytes) >> 4);      // past the step or the matrix: its last piece again
+#pragma unroll
+    for (int u = 0; u < LOADS; u++) g[u] = load_w16(rp + min(lane + 64 * u, last) * 16);
+  };
+  // the activation row goes through LDS once per workgroup, its loads ahead of those of the weights (loads return in issue order); a row is
+  // at most 18 NB1 pieces of 16 bytes, 4-byte aligned
+  __shared__ __align__(16) uint32_t xl[NB1 * 72];
+  constexpr int XLOADS = (NB1 * 72 + 255) / 256;
+  uint32_t xr[XLOADS];
+#pragma unroll
+  for (int u = 0; u < XLOADS; u++) xr[u] = ((const uint32_t*)xq)[min((int)threadIdx.x + 256 * u, nb * 72 - 1)];
+  load(min(row0, N - 1));
+#pragma unroll
+  for (int u = 0; u < XLOADS; u++)
+    if ((int)threadIdx.x + 256 * u < NB1 * 72) xl[threadIdx.x + 256 * u] = xr[u];
+  __syncthreads();
+  XQ x[S];
+  int in_row[S];                 // the row of the step; past the last one: RPI
+#pragma unroll
+  for (int r = 0; r < S; r++) {
+    const int f = 8 * r + b;
+    in_row[r] = f / nb;
+    load_xq(x[r], (const uint8_t*)xl, f - in_row[r] * nb, c, in_row[r] < RPI);
+  }
+
+  while (row0 < N) {
+#pragma unroll
+    for (int u = 0; u < LOADS; u++)
+      if (64 * u + 63 < S * 72 || lane + 64 * u < S * 72) tile[lane + 64 * u] = g[u];
+    if (row0 + step < N) load(row0 + step);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double acc[RPI];
+#pragma unroll
+    for (int i = 0; i < RPI; i++) acc[i] = 0.0;
+#pragma unroll
+    for (int r = 0; r < S; r++) {
+      int I0, I1;
+      const uint4 hdr = tile[(8 * r + b) * 9], q = tile[(8 * r + b) * 9 + 1 + c];
+      const double t = slot_dot(hdr, q, x[r], sel, I0, I1, odd);
+      const int first = 8 * r / NB1, last = min((8 * r + 7) / NB0, RPI);      // rows that the round can lie in
+#pragma unroll
+      for (int i = 0; i < RPI; i++)
+        if (i >= first && i <= last) acc[i] += first == last || in_row[r] == i ? t : 0.0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();                     // every lane has read its pieces before the tile is overwritten
+    double tot;
+    if constexpr (RPI == 4) tot = wave_sum4_f64(acc[0], acc[1], acc[2], acc[3], lane);
+    else tot = wave_sum2_f64(acc[0], acc[1], lane);
+    const int row = row0 + (RPI == 4 ? 2 * (lane & 1) + ((lane >> 1) & 1) : (lane & 1));
+    if (lane < RPI && row < N) store_out<EPI>(y, res, ybase + row, (float)tot);
+    row0 += step;
+  }
+}
+
 // Any K that is a multiple of 256: rounds are a run-time loop and the activation
 // slice is re-read (from L2) in every round.
 template <int EPI>
@@ -185,8 +274,8 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q4k_q8_1_subdots_kernel(
   }
 }
 
-int g_tune_gemv_impl = 2;               // 2: rows staged through LDS when K is a multiple of 2048 (else as 0),
-                                        // 0: direct loads in the (block, chunk) mapping
+int g_tune_gemv_impl = 2;               // 2: rows staged through LDS when K is a multiple of 2048, else the rule of gemv_flat_rounds;
+                                        // 3: the flat form wherever it exists; 0: direct loads in the (block, chunk) mapping
 int g_tune_rpi = 0, g_tune_cap = 16;     // tuning hooks (bk_tune_set): rows per wave step (0: from the shape), workgroups per CU
 int g_tune_steps = 0;                    // > 0: the grid that gives every wave this many row steps (the last one may be short)
 
@@ -222,18 +311,58 @@ static void launch_q8_1_lds(dim3 block, const uint8_t* w, const uint8_t* x, void
   else hipLaunchKernelGGL((gemv_q4k_q8_1_lds_kernel<NR, EPI, 2>), grid, block, 0, stream(), w, x, y, r, N);
 }
 
+// As many workgroups as the chip holds at once, with the steps dealt out evenly.
+template <int S, int RPI, int EPI>
+static void launch_q8_1_flat(const uint8_t* w, const uint8_t* x, void* y, const uint16_t* r, int N, int nb, int batch) {
+  const int64_t wgs = ((int64_t)N + GEMV_WAVES * RPI - 1) / (GEMV_WAVES * RPI), room = num_cus() * flat_waves(S, RPI);
+  const int64_t steps = g_tune_steps > 0 ? g_tune_steps : (wgs * batch + room - 1) / room;
+  hipLaunchKernelGGL((gemv_q4k_q8_1_flat_kernel<S, RPI, EPI>), dim3((unsigned)((wgs + steps - 1) / steps), batch), dim3(GEMV_WAVES * 64), 0, stream(), w, x, y, r, N, nb);
+}
+
+// Rounds a step, 10 S + RPI, of the flat form where it is the faster one, 0 where direct loads are: these start sooner (no pass through LDS), so launches of
+// about one step a wave stay with them, the more rounds the flat form saves the fewer.  us by rows, direct -> flat (1024 SIMDs):
+//   K =  512: 13000 5.3 -> 5.6, 26000 6.05 -> 5.3, 54000  9.8 ->  6.6, 100000 15.8 ->  9.9;  1024: 17000 5.7 -> 5.7, 26000 6.7 -> 6.45, 54000 10.4 -> 9.1, 100000 16.3 -> 12.6;
+//   K = 1536: 33000 8.7 -> 8.9, 54000 11.5 -> 11.3, 100000 18.6 -> 16.9 (1792 saves no round and stays);  2304: 8000 6.5 -> 6.5, 13000 8.5 -> 7.9, 33000 14.6 -> 11.4, 100000 32.7 -> 25.1;
+//   K = 3072: 8000 6.9 -> 6.9, 10000 7.7 -> 7.9, 13000 9.1 -> 8.4, 54000 22.3 -> 18.7;  3584: 8000 7.3 -> 7.4, 10000 8.0 -> 8.7, 13000 9.8 -> 9.2, 86820 38.1 -> 31.4;
+//   K = 3840: 17000 11.7 -> 12.6, 26000 15.2 -> 16.2, 33000 17.9 -> 16.7, 81032 36.6 -> 31.3;  4608: 4000 7.3 -> 6.1, 8000 8.7 -> 8.7, 13000 12.1 -> 10.9, 67527 43.9 -> 31.4;
+//   K = 5120: 13000 12.6 -> 11.1, 60774 40.2 -> 30.3;  5888: 4000 8.1 -> 7.05, 8000 9.0 -> 9.85, 13000 13.5 -> 12.6, 54000 40.3 -> 31.2.
+static int gemv_flat_rounds(int nb, int N, int batch) {
+  if (nb % 8 == 0 || nb == 7 || nb > 23) return 0;
+  const int rpi = nb < 16 ? 4 : 2, S = (rpi * nb + 7) / 8;
+  const int64_t wgs = ((int64_t)N + GEMV_WAVES * rpi - 1) / (GEMV_WAVES * rpi) * batch, cus = num_cus();
+  bool pays = true;
+  if (S == 1) pays = wgs > 5 * cus;
+  else if (S == 2) pays = wgs > 6 * cus;
+  else if (S == 3) pays = wgs > 15 * cus;
+  else if (S == 6) pays = wgs <= 2 * cus || wgs > flat_waves(S, rpi) * cus;
+  else if (S == 7) pays = wgs > 3 * cus;
+  else if (S == 8) pays = wgs > 7 * cus;
+  return pays || g_tune_gemv_impl == 3 ? 10 * S + rpi : 0;
+}
+
 template <int EPI>
 static void launch_q8_1_variant(const void* W, const void* xq, void* y, const void* res, int N, int nb, int batch) {
   const int rounds = (nb + 7) / 8;
   dim3 block(GEMV_WAVES * 64);
   dim3 grid(1, batch);
   const uint8_t* w = (const uint8_t*)W; const uint8_t* x = (const uint8_t*)xq; const uint16_t* r = (const uint16_t*)res;
+  switch (g_tune_gemv_impl == 0 ? 0 : gemv_flat_rounds(nb, N, batch)) {
+    case 14: return launch_q8_1_flat<1, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 24: return launch_q8_1_flat<2, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 34: return launch_q8_1_flat<3, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 54: return launch_q8_1_flat<5, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 64: return launch_q8_1_flat<6, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 74: return launch_q8_1_flat<7, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 84: return launch_q8_1_flat<8, 4, EPI>(w, x, y, r, N, nb, batch);
+    case 52: return launch_q8_1_flat<5, 2, EPI>(w, x, y, r, N, nb, batch);
+    case 62: return launch_q8_1_flat<6, 2, EPI>(w, x, y, r, N, nb, batch);
+  }
   switch (rounds) {
-    case 1: if (g_tune_gemv_impl == 2 && nb == 8) launch_q8_1_lds<1, EPI>(block, w, x, y, r, N, batch); else launch_q8_1_rpi<1, EPI>(block, w, x, y, r, N, nb, batch);
+    case 1: if (g_tune_gemv_impl != 0 && nb == 8) launch_q8_1_lds<1, EPI>(block, w, x, y, r, N, batch); else launch_q8_1_rpi<1, EPI>(block, w, x, y, r, N, nb, batch);
       break;
-    case 2: if (g_tune_gemv_impl == 2 && nb == 16) launch_q8_1_lds<2, EPI>(block, w, x, y, r, N, batch); else launch_q8_1_rpi<2, EPI>(block, w, x, y, r, N, nb, batch);
+    case 2: if (g_tune_gemv_impl != 0 && nb == 16) launch_q8_1_lds<2, EPI>(block, w, x, y, r, N, batch); else launch_q8_1_rpi<2, EPI>(block, w, x, y, r, N, nb, batch);
       break;
-    case 3: if (g_tune_gemv_impl == 2 && nb == 24) launch_q8_1_lds<3, EPI>(block, w, x, y, r, N, batch); else launch_q8_1_rpi<3, EPI>(block, w, x, y, r, N, nb, batch);
+    case 3: if (g_tune_gemv_impl != 0 && nb == 24) launch_q8_1_lds<3, EPI>(block, w, x, y, r, N, batch); else launch_q8_1_rpi<3, EPI>(block, w, x, y, r, N, nb, batch);
       break;
     default:
       grid.x = gemv_grid(N, GEMV_WAVES);

@@ -93,7 +93,8 @@ BK_API int bk_graph_node_count(uint64_t graph, int* count);
 
 /* Launch-shape knobs for experiments and tests; the defaults (0, or -1 = chosen from the shape) are the tuned values:
  * "gemv_rpi", "gemv_cap", "gemv_steps", "gemv_impl", "fused_cap" (GEMV rows per wave step, workgroups per CU up to
- * which a wave takes one step, row steps per wave, kernel variant),
+ * which a wave takes one step, row steps per wave, kernel variant: 0 = direct loads, 2 = from the shape, 3 = several rows'
+ * super-blocks numbered through wherever K is no multiple of 2048),
  * "gemm_tiles" (workgroups of 64 x 64 outputs: 1 = always, 0 = never, -1 = from the shape; "gemm_nw" comes first), "gemm_nw" (waves per matmul tile: 1, 2, 4, 8), "gemm_r16" (narrow matmul tiles: 1 = 16 weight rows, 2 = 8), "small_rows" (0: the two 16-row
  * matrices of a batched projection group stay in the matmul instead of the norm's launch), "rows" (products of 2 to 7
  * sequences in one pass over the weights: 0 = never, 1 = where it is the faster form, the default, 2 = wherever there is a

@@ -185,6 +185,47 @@ def test_gemv_q4k_q8_1_ragged_shapes(orc, dev, N, K):
     assert np.array_equal(rt.from_device(dI, (N, K // 32), np.int32), orc.q4k_q8_1_subdots(W, xq, N, K))
 
 
+@pytest.mark.parametrize("nb", [1, 2, 3, 4, 5, 6, 9, 10, 11, 12, 13, 14, 15, 17, 18, 20, 21, 23])
+def test_gemv_q4k_q8_1_rows_numbered_through(orc, dev, nb):
+    """Rows that do not fill whole rounds of 64 slots, in the form that numbers the super-blocks of several rows through: every class of row length at both
+    ends, fewer rows than a step has, one and several steps a wave, each epilogue, two batch rows, and a row with an infinite scale,
+    which its neighbours in the same rounds do not see.  One unit of an output's last place: its sum is formed in double in another order."""
+    K = 256 * nb
+    g = synth.rng(60 + nb)
+    try:
+        rt.tune_set("gemv_impl", 3)
+        for N, steps in ((1, 0), (3, 0), (50, 0), (301, 3), (170, 8)):
+            print(f"gemv flat nb={nb} N={N} steps={steps}", flush=True)
+            rt.tune_set("gemv_steps", steps)
+            W = synth.q4k_random(g, N, K)
+            bad = N // 2
+            if N > 1:
+                W.reshape(N, nb, 144)[bad, (nb - 1) // 2, 0:2] = np.array([0x7C00], np.uint16).view(np.uint8)
+            xq = np.stack([orc.pack_q8_1(g.standard_normal(K).astype(np.float32)) for _ in range(2)])
+            res = synth.f32_to_bf16(g.standard_normal((2, N)).astype(np.float32))
+            keep = np.arange(N) != bad if N > 1 else np.ones(N, bool)
+            ref = np.stack([orc.gemv_q4k_q8_1(W, xq[i], N, K) for i in range(2)])[:, keep]
+            dW, dx, dr = dev.up(W), dev.up(xq), dev.up(res)
+            dy = dev.empty(2 * N * 4 + 64)
+            rt.cuMemset(dy, 0xCD, 2 * N * 4 + 64)
+            rt.gemv_q4k_q8_1(dW, dx, dy, N, K, batch=2)
+            raw = rt.from_device(dy, (2 * N + 16,), np.float32)
+            got = raw[:2 * N].reshape(2, N)
+            assert (raw[2 * N:].view(np.uint32) == 0xCDCDCDCD).all()
+            assert np.isfinite(got[:, keep]).all() and (N == 1 or not np.isfinite(got[:, bad]).any())
+            assert (np.abs(got[:, keep].astype(np.float64) - ref) <= np.spacing(np.abs(ref))).all()
+            for r in (0, dr):
+                db = dev.empty(2 * N * 2)
+                rt.gemv_q4k_q8_1(dW, dx, db, N, K, batch=2, out_dtype=rt.BF16, residual=r)
+                want = synth.f32_to_bf16(got)
+                if r:
+                    want = synth.f32_to_bf16(synth.bf16_to_f32(want) + synth.bf16_to_f32(res))
+                assert np.array_equal(rt.from_device(db, (2, N), np.uint16)[:, keep], want[:, keep])
+    finally:
+        rt.tune_set("gemv_impl", 2)
+        rt.tune_set("gemv_steps", 0)
+
+
 def test_gemv_q4k_q8_1_epilogues_and_batch(orc, dev):
     g = synth.rng(11)
     N, K, B = 2048, 2048, 3
