@@ -182,6 +182,10 @@ __device__ __forceinline__ void fold_rows(const RowTile<NR, RPI>& t, const XQ (&
     const double tot = wave_sum4_f64(acc[0], acc[1], acc[2], acc[3], lane);
     const int row = row0 + 2 * (lane & 1) + ((lane >> 1) & 1);
     if (lane < 4 && row < N) store_out<EPI>(y, res, ybase + row, (float)tot);
+  } else if (RPI == 2) {
+    const double tot = wave_sum2_f64(acc[0], acc[RPI - 1], lane);
+    const int row = row0 + (lane & 1);
+    if (lane < 2 && row < N) store_out<EPI>(y, res, ybase + row, (float)tot);
   } else {
 #pragma unroll
     for (int i = 0; i < RPI; i++) {
