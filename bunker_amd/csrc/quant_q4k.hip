@@ -13,7 +13,8 @@
 // grid and wave, 21 grids, at 1.2-1.3 ns each on a SIMD, the rate of two-operand f32 operations.  What the search does not
 // need (packed copies of the levels, integer conversions, the wrap-around of nearest_int for quotients that large do not
 // occur) is kept out of it: 6144 x 2048 from bf16 128.5 -> 111 us, 32768 x 6144 1918 -> 1625; with levels in three or four
-// instructions instead of five where a wave's values allow it (grid_level_unit) 110.4 -> 105.6 us.  Four waves per SIMD instead
+// instructions instead of five where a wave's values allow it (grid_level_unit) 110.4 -> 105.6 us, with the
+// stored levels from a reciprocal 104.7 (the first grid's levels in the short form too: 108.5, the compiler schedules the search worse).  Four waves per SIMD instead
 // of three (128 registers) spill 21 and take 129 us.
 #include <type_traits>
 
@@ -197,10 +198,27 @@ __global__ __launch_bounds__(256) void quantize_q4k_kernel(const void* __restric
   const float d = __fmul_rn(half_to_f32(hd), (float)ls);
   if (d != 0.f) {
     const float dm = __fmul_rn(half_to_f32(hm), (float)lm);
+    // The quotients by a reciprocal first (three roundings: off by less than 2^-21 of themselves): where none of a wave's lies within 2^-15 of the
+    // middle between two levels, nor is so large that nearest_int wraps, these are the levels of the rounded quotients.
+    const float inv = __builtin_amdgcn_rcpf(d);
+    float off = 0.f;
+    bool large = false;
 #pragma unroll
     for (int i = 0; i < 32; i++) {
-      const int l = clamp_i(nearest_int(__fdiv_rn(__fadd_rn(x[i], dm), d)), 0, 15);
+      const float t = __fmul_rn(__fadd_rn(x[i], dm), inv), r = __builtin_rintf(t);
+      const float l = __builtin_amdgcn_fmed3f(r, 0.f, 15.f);
+      // (below 0 and above 15 no middle matters: the distance is taken from the level itself, cut at the ends)
+      off = fmaxf(off, fabsf(__fsub_rn(__builtin_amdgcn_fmed3f(t, 0.f, 15.f), l)));
+      large |= !(fabsf(t) < 1048576.f);      // (or not a number)
       Lp[i >> 3] |= (uint32_t)l << (4 * (i & 7));
+    }
+    if (__any(large || off >= 0.5f - 0x1p-15f)) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        Lp[g] = 0u;
+#pragma unroll
+        for (int i = 8 * g; i < 8 * g + 8; i++) Lp[g] |= (uint32_t)clamp_i(nearest_int(__fdiv_rn(__fadd_rn(x[i], dm), d)), 0, 15) << (4 * (i & 7));
+      }
     }
   } else if (win_iscale != 0.f) {               // the stored scale is zero: the winning grid's own levels stay
 #pragma unroll

@@ -89,6 +89,28 @@ def test_quantize_q4k_ranges_around_one(orc, top):
     assert np.array_equal(got, ref), f"{np.count_nonzero(got != ref)} bytes differ"
 
 
+@pytest.mark.parametrize("kind", ["halves", "ulps", "huge", "random"])
+def test_quantize_q4k_levels_at_the_middle(orc, kind):
+    """The stored levels come from a reciprocal unless a quotient lies next to the middle between two levels: values on and an ulp or so beside the
+    middles of the grid that the super-block stores, quotients past 2^22, and many random values; the bytes stay the checker's."""
+    g = synth.rng(4400)
+    w = (g.standard_normal((256, 1024)) * 0.02).astype(np.float32)
+    if kind in ("halves", "ulps"):      # a grid of scale and min 63 steps of a half-precision number, with values on its half steps
+        k = g.integers(0, 31, (256, 32, 32))
+        k[:, :, 0], k[:, :, 1] = 0, 30
+        w = (k * (63 * 2.0**-12 / 2) - 63 * 2.0**-10).astype(np.float32)
+        if kind == "ulps":
+            w = (w.view(np.int32) + g.integers(-2, 3, w.shape, dtype=np.int32)).view(np.float32)
+        w = w.reshape(256, 1024)
+    elif kind == "huge":                # a sub-block of large offset beside narrow ones: min and scale of very different size
+        w = w.reshape(256, 32, 32)
+        w[:, ::8] = (-1000 - 1e-4 * g.random((256, 4, 32))).astype(np.float32)
+        w[::2, 1::8] = 3e4
+        w = np.ascontiguousarray(w.reshape(256, 1024))
+    got, ref = _quantize_dev(np.ascontiguousarray(w), rt.F32), orc.quantize_q4k(w)
+    assert np.array_equal(got, ref), f"{np.count_nonzero(got != ref)} bytes differ"
+
+
 def test_quantize_q4k_rejects_bad_shapes():
     d = rt.to_device(np.zeros(512, np.float32))
     with pytest.raises(rt.BunkerError):
