@@ -14,7 +14,7 @@
 // need (packed copies of the levels, integer conversions, the wrap-around of nearest_int for quotients that large do not
 // occur) is kept out of it: 6144 x 2048 from bf16 128.5 -> 111 us, 32768 x 6144 1918 -> 1625; with levels in three or four
 // instructions instead of five where a wave's values allow it (grid_level_unit) 110.4 -> 105.6 us, with the
-// stored levels from a reciprocal 104.7 (the first grid's levels in the short form too: 108.5, the compiler schedules the search worse).  Four waves per SIMD instead
+// stored levels from a reciprocal 104.7, with one test in front of the short forms 99.0 (the compiler's schedule of the search depends on it).  Four waves per SIMD instead
 // of three (128 registers) spill 21 and take 129 us.
 #include <type_traits>
 
@@ -147,10 +147,15 @@ __global__ __launch_bounds__(256) void quantize_q4k_kernel(const void* __restric
       // every |iscale * (x - mn)| is at most the one of the two ends; a fitted min that met the maximum (sub-blocks whose
       // values differ by a few ulps) makes it infinite or NaN
       const float reach = fabsf(iscale) * fmaxf(fabsf(mx - mn), fabsf(lowest - mn));
-      if (__any(!(reach <= 1048576.f))) levels_and_sums(std::integral_constant<int, 1>{});
-      else if (__any(!(mx - mn > 0.f && mx - mn < 1.f))) levels_and_sums(std::integral_constant<int, 0>{});
-      else if (is <= 14) levels_and_sums(std::integral_constant<int, 2>{});      // 15.4 at the maximum, a few roundings aside
-      else levels_and_sums(std::integral_constant<int, 3>{});
+      const float span = mx - mn;
+      if (!__any(!(reach <= 1048576.f && span > 0.f && span < 1.f))) {
+        if (is <= 14) levels_and_sums(std::integral_constant<int, 2>{});      // 15.4 at the maximum, a few roundings aside
+        else levels_and_sums(std::integral_constant<int, 3>{});
+      } else if (__any(!(reach <= 1048576.f))) {
+        levels_and_sums(std::integral_constant<int, 1>{});
+      } else {
+        levels_and_sums(std::integral_constant<int, 0>{});
+      }
       const float D = __fsub_rn(__fmul_rn(sum_w, sum_l2), __fmul_rn(sum_l, sum_l));
       if (D > 0.f) {
         float this_scale = __fdiv_rn(__fsub_rn(__fmul_rn(sum_w, sum_xl), __fmul_rn(sum_x, sum_l)), D);
