@@ -123,7 +123,8 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void attn_decode_kernel(AttnArgs A)
       sc[r] = (tok0 + r < len) ? s4[r] * A.scale : -INFINITY;
       tmax = fmaxf(tmax, sc[r]);
     }
-    tmax = row_pair_max<32>(row_pair_max<16>(tmax));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
     const float m_new = fmaxf(m_run, tmax);
     // a column whose own length ends before this page (the shorter of two rows) has seen nothing yet: keep exp() off inf - inf
     const float m_ref = (m_new == -INFINITY) ? 0.0f : m_new;
@@ -181,7 +182,8 @@ __global__ __launch_bounds__(ATT_WAVES * 64) void attn_decode_kernel(AttnArgs A)
   }
 
   // ---- merge the four waves as (0 + 1) + (2 + 3): two exchange rounds through LDS, a third for the transposed write
-  const float l_tot = row_pair_sum<32>(row_pair_sum<16>(l_run));
+  float l_tot = l_run + __shfl_xor(l_run, 16);
+  l_tot += __shfl_xor(l_tot, 32);
   if (kg == 0) { lds_m[wave][n] = m_run; lds_l[wave][n] = l_tot; }
   __syncthreads();
   float M = lds_m[0][n];

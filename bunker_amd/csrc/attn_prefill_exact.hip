@@ -154,7 +154,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
       smax = fmaxf(smax, valid[v] ? (float)s[v] : -INFINITY);
     }
     if (__ballot(smax > -INFINITY && (double)smax > mref + PE_REF_SLACK) != 0) {     // the first page with a key of a row, rarely again
-      smax = row_pair_max<32>(row_pair_max<16>(smax));
+      smax = fmaxf(smax, __shfl_xor(smax, 16));
+      smax = fmaxf(smax, __shfl_xor(smax, 32));
       if (smax > -INFINITY && (double)smax > mref + PE_REF_SLACK) {      // the same in the four lanes of a row
         const double alpha = exp(mref - (double)smax);                  // (0 the first time: only zeros have been added)
         mref = (double)smax;
@@ -192,7 +193,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_exact_kernel(PrefillExact
   int tl = tid;
   asm volatile("" : "+v"(tl));             // (the rest works out its addresses here: carried across the pages they would have no registers)
   const int c16 = tl & 15, r4 = (tl >> 4) & 3, w4 = tl >> 6;
-  l = row_pair_sum<32>(row_pair_sum<16>(l));
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
   if (r4 == 0) { lds_m[w4][c16] = mref == ATT_NO_REF ? -INFINITY : mref; lds_l[w4][c16] = l; }
   __syncthreads();                         // (and every wave is done with Q)
   double M = lds_m[0][c16];

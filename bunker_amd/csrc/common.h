@@ -141,27 +141,6 @@ __device__ __forceinline__ double div127_f64(double a) {
   return fma(fma(-127.0, q1, a), c, q1);
 }
 
-// A value across the wave's rows of 16: v of this lane and of lane ^ 16 (lane ^ 32), the lower row's first in both.  The swap instructions exchange rows of
-// two registers on the vector unit; __shfl_xor of these distances goes through the LDS crossbar, two round trips for a double.
-template <int DIST, typename T>
-__device__ __forceinline__ void row_pair(T v, T& a, T& b) {
-  static_assert(DIST == 16 || DIST == 32, "lanes 16 or 32 apart");
-  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two registers");
-  uint32_t w[sizeof(T) / 4], l[sizeof(T) / 4], h[sizeof(T) / 4];
-  __builtin_memcpy(w, &v, sizeof(T));
-#pragma unroll
-  for (unsigned i = 0; i < sizeof(T) / 4; i++) {
-    const auto p = DIST == 16 ? __builtin_amdgcn_permlane16_swap(w[i], w[i], false, false) : __builtin_amdgcn_permlane32_swap(w[i], w[i], false, false);
-    l[i] = p[0]; h[i] = p[1];
-  }
-  __builtin_memcpy(&a, l, sizeof(T));
-  __builtin_memcpy(&b, h, sizeof(T));
-}
-template <int DIST, typename T>
-__device__ __forceinline__ T row_pair_sum(T v) { T a, b; row_pair<DIST>(v, a, b); return a + b; }
-template <int DIST>
-__device__ __forceinline__ float row_pair_max(float v) { float a, b; row_pair<DIST>(v, a, b); return fmaxf(a, b); }
-
 __device__ __forceinline__ double readlane_f64(double v, int lane) {
   const long long b = __builtin_bit_cast(long long, v);
   const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
@@ -248,11 +227,11 @@ __device__ __forceinline__ uint32_t quad_q8_1(const float (&f)[8], uint32_t (&pk
 // `blk` points at the 36-byte block, l = lane % 32.
 __device__ __forceinline__ void lane32_q8_1_store(float v, uint8_t* __restrict__ blk, int l, bool store = true) {
   float amax = row16_max(fabsf(v));
-  amax = row_pair_max<16>(amax);
+  amax = fmaxf(amax, __shfl_xor(amax, 16));
   const double d = div127_f64((double)amax);
   int q = q8_1_round(v, q8_1_inv(amax), d != 0.0 ? d : 1.0);
   int sum = row16_sum_i32(q);
-  sum = row_pair_sum<16>(sum);
+  sum += __shfl_xor(sum, 16);
   q = q < -128 ? -128 : (q > 127 ? 127 : q);
   if (!store) return;                      // the group took part in the exchanges above; nothing of it is kept
   blk[l] = (uint8_t)(int8_t)q;

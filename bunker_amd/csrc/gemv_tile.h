@@ -109,7 +109,9 @@ __device__ __forceinline__ double wave_sum4_f64(double a0, double a1, double a2,
   double v = k + dpp_f64<DPP_QUAD_XOR2>(g);
   v += dpp_f64<0x124>(v);      // row_ror:4  (lane i gets lane (i+4) mod 16 of its row of 16)
   v += dpp_f64<0x128>(v);      // row_ror:8
-  return row_pair_sum<32>(row_pair_sum<16>(v));
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  return v;
 }
 
 // Two rows: one exchange-and-halve step, then lane parity is kept; lane L ends with row L & 1.
@@ -120,7 +122,9 @@ __device__ __forceinline__ double wave_sum2_f64(double a0, double a1, int lane) 
   v += dpp_f64<DPP_QUAD_XOR2>(v);
   v += dpp_f64<0x124>(v);      // row_ror:4
   v += dpp_f64<0x128>(v);      // row_ror:8
-  return row_pair_sum<32>(row_pair_sum<16>(v));
+  v += __shfl_xor(v, 16);
+  v += __shfl_xor(v, 32);
+  return v;
 }
 
 // Weights are read once: nontemporal loads keep them from displacing the activation in the caches.

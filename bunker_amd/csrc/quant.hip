@@ -21,11 +21,11 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const void* __restri
     else v = bf16_to_f32(((const uint16_t*)xin)[(int64_t)row * K + e]);
   }
   float amax = row16_max(fabsf(v));
-  amax = row_pair_max<16>(amax);
+  amax = fmaxf(amax, __shfl_xor(amax, 16));
   const double d = div127_f64((double)amax);
   int q = q8_1_round(v, q8_1_inv(amax), d != 0.0 ? d : 1.0);
   int sum = row16_sum_i32(q);
-  sum = row_pair_sum<16>(sum);
+  sum += __shfl_xor(sum, 16);
   q = q < -128 ? -128 : (q > 127 ? 127 : q);
   if (blk < nblk) {
     uint8_t* o = out + ((int64_t)row * nblk + blk) * 36;
