@@ -69,6 +69,8 @@ static int need(Kernel& k, const char* key) {
   if (!k.has(key)) return set_error(BK_ERR_ARG, "kernel '%s': missing parameter %s=", k.op.c_str(), key);
   return BK_OK;
 }
+// Nothing in a workspace has to start with a value: whatever a launch reads there it has written itself.  (A fill at creation would have to be
+// waited for: the library's streams are not ordered behind the null stream, and a handle may be launched on any of them.)
 static int alloc_scratch(Kernel& k, size_t bytes) {
   BK_HIP(hipMalloc(&k.scratch, bytes));
   k.scratch_bytes = bytes;
@@ -334,8 +336,8 @@ static int run_fa2_fused(Kernel& k, const uint64_t* s) {
   const int max_len = (int)k.get("MAX_LEN", 0), bt_stride = (max_len + 15) / 16, half = (int)k.get("ROT_HALF", 0);
   const int32_t* pos_dev = dev ? P<int32_t>(s[7]) : nullptr;
   const int pos = dev ? 0 : (int)(int32_t)s[7];
-  // workspace: normalised, rotated q as bf16 [batch, NH, HD]; exact=1: the same as f64 [batch, NKV, HD, 8] (written by the
-  // prep kernel, unused columns stay zero from creation); then the partials of the splits
+  // workspace: normalised, rotated q as bf16 [batch, NH, HD]; exact=1: the same as f64 [batch, NKV, HD, 8] (both written by
+  // the prep kernel, the unused columns too); then the partials of the splits
   const int exact = (int)k.get("exact", 1);
   const size_t qn_bytes = fa2_qn_bytes(batch, NH, HD), qf_bytes = exact ? attn_exact_qf_bytes(batch, NKV) : 0;
   void* qn = k.scratch;
@@ -477,7 +479,6 @@ static int build_kernel(Kernel& k) {
     BK_REQUIRE(!exact || k.get("NH", 0) / NKV <= 8, "fa2_fused: exact=1 serves at most 8 query heads per KV head (exact=0 takes 16)");
     const size_t qbytes = fa2_qn_bytes(batch, (int)k.get("NH", 0), (int)k.get("HD", 0));
     if ((rc = alloc_scratch(k, qbytes + fa2_ws_bytes(batch, NKV, splits, exact)))) return rc;
-    if (exact) BK_HIP(hipMemset(k.scratch, 0, k.scratch_bytes));        // columns of the f64 query copy past the group stay zero
     k.run = run_fa2_fused; k.nslots = 11 + (k.get("q8out", 0) ? 1 : 0);
     return BK_OK;
   }
@@ -519,7 +520,6 @@ static int build_kernel(Kernel& k) {
     const size_t qbytes = fa2_qn_bytes(T, (int)k.get("NH", 0), (int)k.get("HD", 0));
     const size_t ws_bytes = tiled ? attn_prefill_workspace_bytes(T, NHq, NKV, max_len) : rows16 ? 0 : fa2_ws_bytes(T, NKV, splits, exact);
     if ((rc = alloc_scratch(k, qbytes + ws_bytes))) return rc;
-    if (exact && !rows16) BK_HIP(hipMemset(k.scratch, 0, k.scratch_bytes));
     k.run = run_fa2_prefill; k.nslots = 12;
     return BK_OK;
   }

@@ -522,7 +522,7 @@ struct PrepArgs {
   const float *cos_t, *sin_t;      // f32 [max_len, half]
   const int32_t* pos_dev; int pos_scalar;
   uint16_t *qout, *kc, *vc;
-  uint32_t* qf;                    // optional: the query heads also widened to f64, high words [B, NKV, 256, 8], for the double-precision attention
+  uint32_t* qf;                    // optional: the query heads also widened to f64, high words [B, NKV, 256, 8], for the double-precision attention (columns past a group's heads: zeros)
   const int32_t* block_table; int bt_stride;
   int NH, NKV, half, max_len;
 };
@@ -575,8 +575,11 @@ __global__ __launch_bounds__(64) void attn_prep_kernel(PrepArgs A) {
     }
     dst[i] = o;
     if (is_q && A.qf) {
-      const int G = A.NH / A.NKV;
-      A.qf[(((int64_t)b * A.NKV + role / G) * ATT_HD + i) * 8 + role % G] = (uint32_t)(__builtin_bit_cast(uint64_t, (double)bf16_to_f32(o)) >> 32);
+      const int G = A.NH / A.NKV, c = role % G;
+      uint32_t* const qf = A.qf + (((int64_t)b * A.NKV + role / G) * ATT_HD + i) * 8;
+      qf[c] = (uint32_t)(__builtin_bit_cast(uint64_t, (double)bf16_to_f32(o)) >> 32);
+      if (c == 0)
+        for (int z = G; z < 8; z++) qf[z] = 0u;
     }
   }
 }

@@ -24,6 +24,29 @@ def test_header_symbols_are_exported():
     assert set(rt._SIGS) | {"bk_last_error"} == set(names)
 
 
+def test_everything_on_the_device_names_its_stream():
+    """The library's streams are made with hipStreamNonBlocking: a copy or a fill without a stream goes to the null stream, which they are not ordered
+    behind, and a launch right after it may run first.  No such call is linked, and every kernel launch names the library's stream."""
+    import re
+    import subprocess
+
+    _lib_or_skip()
+    used = set(re.findall(r"\bhip\w+", subprocess.run(["nm", "-D", "--undefined-only", rt.LIB_PATH], check=True, capture_output=True, text=True).stdout))
+    assert "hipMemcpyAsync" in used
+    unordered = {n for n in used if re.match(r"hipMem(cpy|set)", n) and "Async" not in n}
+    assert not unordered, unordered
+    csrc = os.path.join(os.path.dirname(rt.LIB_PATH), "csrc")
+    launches = 0
+    for f in sorted(os.listdir(csrc)):
+        if f.endswith((".hip", ".h")):
+            text = open(os.path.join(csrc, f)).read()
+            assert "<<<" not in text, f
+            for m in re.finditer(r"hipLaunchKernelGGL\(.*?;", text, flags=re.S):
+                assert re.search(r",\s*stream\(\)", m.group(0)), (f, m.group(0))
+                launches += 1
+    assert launches >= 40
+
+
 _CTYPE = {
     "int": rt.i32, "int64_t": rt.i64, "uint64_t": rt.u64,
     "const char*": C.c_char_p, "char*": C.c_char_p, "const void*": rt.vp, "void*": rt.vp,

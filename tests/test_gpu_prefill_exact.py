@@ -72,6 +72,21 @@ def test_equals_one_token_a_workgroup(orc, NH, NKV, T, pos0):
     _same(c.run(1), c.run(0))
 
 
+@pytest.mark.parametrize("NH,NKV", [(2, 2), (4, 2), (12, 2), (8, 1)])
+def test_first_launch_of_a_new_handle(orc, NH, NKV):
+    """A handle's workspace starts with what the memory held before (here NaNs of both widths) and is launched right behind its creation: one
+    to eight heads a KV head, the ones that leave columns of the query copy unused among them."""
+    c = _Case(orc, 1370 + NH, NH, NKV, 9, 40 + np.arange(9), 1024)
+    want = c.run(1)
+    for _ in range(3):
+        old = [rt.cuAlloc(n) for n in (1 << 20, 4 << 20, 16 << 20)]
+        for p, n in zip(old, (1 << 20, 4 << 20, 16 << 20)):
+            rt.cuMemset(p, 0xff, n)
+        for p in old:
+            rt.cuFree(p)
+        _same(c.run(0), want)
+
+
 @pytest.mark.parametrize("shift", [2, 4, 8])
 def test_gate_and_output_at_any_address(orc, shift):
     c = _Case(orc, 1350, 16, 2, 37, 5 + np.arange(37), 64)
