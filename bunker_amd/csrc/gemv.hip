@@ -405,22 +405,35 @@ struct XF {
   float sum_c;   // sum of the 32 activations of sub-block c (for the lane's share of the mins)
 };
 
-// Four bytes' low nibbles (SHIFT 0) or high ones (SHIFT 4) against four activations, times 2^-24: a nibble alone in 16 bits is a subnormal half, and the
-// mixed FMA reads it as it is, in either half of a register.
+// Four bytes' low nibbles (SHIFT 0) or high ones (SHIFT 4) against four activations.  LIFTED: the activations are 2^24 times what they are.  A nibble alone in
+// 16 bits is a subnormal half of 2^-24 times its value, which the mixed FMA reads as it is, in either half of a register: the products are the same numbers
+// as those of a converted nibble and the activation itself, down to the smallest.
 typedef __attribute__((ext_vector_type(2))) _Float16 half2_t;
-template <int SHIFT>
+template <int SHIFT, bool LIFTED>
 __device__ __forceinline__ float nibdot4(uint32_t q, const float* x, float acc) {
-  const half2_t n02 = __builtin_bit_cast(half2_t, (q >> SHIFT) & 0x000f000fu), n13 = __builtin_bit_cast(half2_t, (q >> (SHIFT + 8)) & 0x000f000fu);
-  acc = fmaf((float)n02[0], x[0], acc);
-  acc = fmaf((float)n13[0], x[1], acc);
-  acc = fmaf((float)n02[1], x[2], acc);
-  acc = fmaf((float)n13[1], x[3], acc);
+  if constexpr (LIFTED) {
+    const half2_t n02 = __builtin_bit_cast(half2_t, (q >> SHIFT) & 0x000f000fu), n13 = __builtin_bit_cast(half2_t, (q >> (SHIFT + 8)) & 0x000f000fu);
+    acc = fmaf((float)n02[0], x[0], acc);
+    acc = fmaf((float)n13[0], x[1], acc);
+    acc = fmaf((float)n02[1], x[2], acc);
+    acc = fmaf((float)n13[1], x[3], acc);
+  } else {
+    const uint32_t n4 = (q >> SHIFT) & 0x0f0f0f0fu;
+    acc = fmaf((float)(n4 & 0xffu), x[0], acc);
+    acc = fmaf((float)((n4 >> 8) & 0xffu), x[1], acc);
+    acc = fmaf((float)((n4 >> 16) & 0xffu), x[2], acc);
+    acc = fmaf((float)(n4 >> 24), x[3], acc);
+  }
   return acc;
 }
 
-// The lane's 32 activations of super-block blk (taken from at(i), float4 i of the row).  Lanes c and c ^ 1 hold the two halves of sub-blocks 2g and
-// 2g+1, so the sum of sub-block c is the lane's own half plus its neighbour's.  Every lane of the wave takes part in the exchange.
-template <typename AT>
+// Activations may be lifted where all are below XF_LIFT_BELOW (32 lifted ones still add up to less than 2^127).  Where all are below XF_TINY they are taken
+// times XF_TINY_LIFT as well and the result is brought back, so that a row is rounded once below the normal range and not at every step.
+constexpr float XF_LIFT = 0x1p24f, XF_LIFT_BELOW = 0x1p98f, XF_TINY = 0x1p-63f, XF_TINY_LIFT = 0x1p64f;
+
+// The lane's 32 activations of super-block blk (taken from at(i), float4 i of the row; LIFTED: as lifted ones).  Lanes c and c ^ 1 hold the two halves of
+// sub-blocks 2g and 2g+1, so the sum of sub-block c is the lane's own half plus its neighbour's.  Every lane of the wave takes part in the exchange.
+template <bool LIFTED, typename AT>
 __device__ __forceinline__ void load_xf(XF& x, AT at, int blk, int c, bool active) {
   const int g = c >> 1, half = c & 1;
   const int p0 = (active ? blk : 0) * 64 + 16 * g + 4 * half;
@@ -440,52 +453,60 @@ __device__ __forceinline__ void load_xf(XF& x, AT at, int blk, int c, bool activ
   s0 += dpp_f32<DPP_QUAD_XOR1>(s0);
   s1 += dpp_f32<DPP_QUAD_XOR1>(s1);
   x.sum_c = half ? s1 : s0;
+  if (LIFTED) x.sum_c *= 1.0f / XF_LIFT;      // (exact: what is subnormal then has few enough bits)
 }
 
-// The dots are formed 2^-24 smaller than they are (nibdot4).  Activations that are all below 2^-63 (no exponent has one of its two top bits) are taken times
-// 2^64, so that nothing is lost below the normal range; what has to be done to the result is returned.
-constexpr uint32_t XF_NOT_TINY = 0x60000000u;
-template <int NR>
-__device__ __forceinline__ float lift_tiny(XF (&x)[NR], bool tiny) {
-  if (__builtin_expect(!tiny, 1)) return 1.0f;
-#pragma unroll
-  for (int r = 0; r < NR; r++) {
-#pragma unroll
-    for (int i = 0; i < 16; i++) { x[r].lo[i] *= 0x1p64f; x[r].hi[i] *= 0x1p64f; }
-    x[r].sum_c *= 0x1p64f;
-  }
-  return 0x1p-64f;
-}
-// the same for the activations that the lanes of a wave hold between them
-template <int NR>
-__device__ __forceinline__ float lift_tiny(XF (&x)[NR]) {
-  uint32_t bits = 0;
-#pragma unroll
-  for (int r = 0; r < NR; r++)
-#pragma unroll
-    for (int i = 0; i < 16; i++) bits |= __float_as_uint(x[r].lo[i]) | __float_as_uint(x[r].hi[i]);
-  return lift_tiny(x, __ballot(bits & XF_NOT_TINY) == 0);
-}
-
+template <bool LIFTED>
 __device__ __forceinline__ float slot_dot_f32(const uint4& hdr, const uint4& q, const XF& x, const ScaleSel& sel) {
   const float d = half_to_f32((uint16_t)(hdr.x & 0xffffu));
   const float dmin = half_to_f32((uint16_t)(hdr.x >> 16));
   uint32_t sc, m;
   lane_scale_min(sel, hdr.y, hdr.z, hdr.w, sc, m);
-  const float fsc = (d * (float)sc) * 16777216.0f;
+  const float fsc = d * (float)sc;
   const float fm = (dmin * (float)m) * x.sum_c;
   float a = 0.0f, b = 0.0f;
-  a = nibdot4<0>(q.x, &x.lo[0], a);
-  b = nibdot4<4>(q.x, &x.hi[0], b);
-  a = nibdot4<0>(q.y, &x.lo[4], a);
-  b = nibdot4<4>(q.y, &x.hi[4], b);
-  a = nibdot4<0>(q.z, &x.lo[8], a);
-  b = nibdot4<4>(q.z, &x.hi[8], b);
-  a = nibdot4<0>(q.w, &x.lo[12], a);
-  b = nibdot4<4>(q.w, &x.hi[12], b);
+  a = nibdot4<0, LIFTED>(q.x, &x.lo[0], a);
+  b = nibdot4<4, LIFTED>(q.x, &x.hi[0], b);
+  a = nibdot4<0, LIFTED>(q.y, &x.lo[4], a);
+  b = nibdot4<4, LIFTED>(q.y, &x.hi[4], b);
+  a = nibdot4<0, LIFTED>(q.z, &x.lo[8], a);
+  b = nibdot4<4, LIFTED>(q.z, &x.hi[8], b);
+  a = nibdot4<0, LIFTED>(q.w, &x.lo[12], a);
+  b = nibdot4<4, LIFTED>(q.w, &x.hi[12], b);
   const float f0 = dpp_f32<DPP_PAIR_EVEN>(fsc);
   const float f1 = dpp_f32<DPP_PAIR_ODD>(fsc);
   return (f0 * a + f1 * b) - fm;
+}
+
+// One row of any length and any activations, by one wave: rounds are a run-time loop, the activation slice is re-read (from L2) in every round.
+__device__ __forceinline__ void row_dot_f32(const uint8_t* W, const float* xf, float* y, int row, int nb, int lane, const ScaleSel& sel) {
+  const uint8_t* rp = W + (int64_t)row * nb * 144;
+  const int c = lane & 7, rounds = (nb + 7) / 8;
+  float acc = 0.0f;
+#pragma unroll 1
+  for (int r = 0; r < rounds; r++) {
+    const int blk = r * 8 + (lane >> 3);
+    XF x;
+    load_xf<false>(x, [&](int i) { return ((const float4*)xf)[i]; }, blk, c, blk < nb);
+    float top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) top = fmaxf(fmaxf(top, fabsf(x.lo[i])), fabsf(x.hi[i]));
+    const int bo = (blk < nb ? blk : 0) * 144;
+    uint4 hdr = *(const uint4*)(rp + bo);
+    if (blk >= nb) hdr.x = 0;                             // past the row: d = dmin = 0
+    const uint4 q = *(const uint4*)(rp + bo + 16 + 16 * c);
+    if (__builtin_expect(__any(top >= XF_LIFT_BELOW), 0)) {
+      acc += slot_dot_f32<false>(hdr, q, x, sel);
+    } else {
+      const float up = __any(top >= XF_TINY) ? 1.0f : XF_TINY_LIFT;
+#pragma unroll
+      for (int i = 0; i < 16; i++) { x.lo[i] *= XF_LIFT * up; x.hi[i] *= XF_LIFT * up; }
+      x.sum_c *= up;
+      acc += slot_dot_f32<true>(hdr, q, x, sel) * (1.0f / up);
+    }
+  }
+  const float tot = wave_sum(acc);
+  if (lane == 0) y[row] = tot;
 }
 
 // Rows of up to 8 * NR super-blocks: the LDS staging of gemv_q4k_q8_1_lds_kernel (RPI contiguous rows per wave step,
@@ -494,14 +515,15 @@ __device__ __forceinline__ float slot_dot_f32(const uint4& hdr, const uint4& q, 
 // lanes, fold) up to a few thousand rows, then vector issue.  The workgroup reads x once and hands it to its four waves through LDS: read by every
 // wave in 16-byte pieces 64 bytes apart, x was 33 MB through the caches for a 9.4 MB matrix, and the weights were only asked for behind it.  With that and
 // the mixed FMAs (fifteen instructions for eight weights where conversions made it nineteen), us back to back on cold weights: 1024 x 1024 2.75 -> 2.6,
-// 4096 x 4096 6.1 -> 5.15 (5.46 -> 4.35 on weights in the memory-side cache), 2048 x 6144 5.85 -> 4.6, 12288 x 2048 6.85 -> 5.7, 40000 x 1024 13.4 -> 10.6,
-// 151936 x 2048 43.3 -> 38-41, 50000 x 6144 51.7 -> 42 (4.1 TB/s).
+// 4096 x 4096 6.1 -> 5.15 (5.46 -> 4.31 on weights in the memory-side cache), 2048 x 6144 5.85 -> 4.6, 12288 x 2048 6.85 -> 5.7, 40000 x 1024 13.4 -> 10.6,
+// 151936 x 2048 43.3 -> 37-41, 50000 x 6144 51.7 -> 41 (4.2 TB/s).  Activations are lifted (nibdot4) on their way into LDS; a vector with one that
+// cannot be goes row by row behind the loop (in front of it, the loop's operands took 172 registers instead of 138).
 template <int NR, int RPI>
 __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
     const uint8_t* __restrict__ W, const float* __restrict__ xf, float* __restrict__ y, int N, int nb, int nwg) {
   constexpr int LOADS = StageRegs<NR, RPI>::LOADS, TILE = StageRegs<NR, RPI>::PIECES, XLOADS = NR * 8 * 64 / (GEMV_WAVES * 64);
   __shared__ uint4 lds[GEMV_WAVES * TILE + NR * 8 * 64];
-  __shared__ int4 not_tiny;
+  __shared__ int4 range;           // per wave, of its share of x: 0 every activation tiny, 1 not, 3 one that cannot be lifted
   uint4* const xlds = lds + GEMV_WAVES * TILE;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int c = lane & 7, b = lane >> 3;
@@ -516,10 +538,13 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
   uint32_t in_row[NR];            // all ones, or zero past the row: a lane there has d = dmin = 0 and adds nothing, whatever its block holds
 #pragma unroll
   for (int r = 0; r < NR; r++) in_row[r] = r * 8 + b < nb ? ~0u : 0u;
-  // x first (all workgroups but the first ones find it in a cache), the first rows right behind it: one memory round trip for both
+  // x first (all workgroups but the first ones find it in a cache), the first rows right behind it: one memory round trip for both.  Past the
+  // row the load's range check returns zeros.
+  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)xf, 0, nb * 1024, 0x00027000);
   uint4 xp[XLOADS];
 #pragma unroll
-  for (int u = 0; u < XLOADS; u++) xp[u] = ((const uint4*)xf)[min((int)threadIdx.x + GEMV_WAVES * 64 * u, nb * 64 - 1)];
+  for (int u = 0; u < XLOADS; u++)
+    xp[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, (int)(threadIdx.x + GEMV_WAVES * 64 * u) * 16, 0, 0));
   StageRegs<NR, RPI> g;
   auto request = [&](int r0) {
     const int64_t base = (int64_t)r0 * row_pieces;
@@ -534,19 +559,33 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
   __builtin_amdgcn_sched_barrier(0);
   // piece p lies at p ^ ((p >> 4) & 3): the eight lanes of a super-block read from eight different banks
   auto at_piece = [](int p) { return p ^ ((p >> 4) & 3); };
-  uint32_t bits = 0;
+  float top = 0.0f;
 #pragma unroll
   for (int u = 0; u < XLOADS; u++) {
-    xlds[at_piece(threadIdx.x + GEMV_WAVES * 64 * u)] = xp[u];
-    bits |= xp[u].x | xp[u].y | xp[u].z | xp[u].w;
+    const float4 v = __builtin_bit_cast(float4, xp[u]);
+    top = fmaxf(fmaxf(top, fabsf(v.x)), fabsf(v.y));
+    top = fmaxf(fmaxf(top, fabsf(v.z)), fabsf(v.w));
+    xlds[at_piece(threadIdx.x + GEMV_WAVES * 64 * u)] =
+        __builtin_bit_cast(uint4, make_float4(v.x * XF_LIFT, v.y * XF_LIFT, v.z * XF_LIFT, v.w * XF_LIFT));
   }
-  ((int*)&not_tiny)[wv] = __ballot(bits & XF_NOT_TINY) != 0;
+  ((int*)&range)[wv] = __any(top >= XF_LIFT_BELOW) ? 3 : __any(top >= XF_TINY);
   __syncthreads();
+  const int4 f = range;
 #pragma unroll
-  for (int r = 0; r < NR; r++) load_xf(x[r], [&](int i) { return __builtin_bit_cast(float4, xlds[at_piece(i)]); }, r * 8 + b, c, r * 8 + b < nb);
-  const int4 f = not_tiny;
-  const float unlift = lift_tiny(x, __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w) == 0);
-  while (row0 < N) {
+  for (int r = 0; r < NR; r++) load_xf<true>(x[r], [&](int i) { return __builtin_bit_cast(float4, xlds[at_piece(i)]); }, r * 8 + b, c, true);
+  const int kind = __builtin_amdgcn_readfirstlane(f.x | f.y | f.z | f.w);
+  const int end = kind == 3 ? 0 : N;
+  float down = 1.0f;
+  if (__builtin_expect(kind == 0, 0)) {
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) { x[r].lo[i] *= XF_TINY_LIFT; x[r].hi[i] *= XF_TINY_LIFT; }
+      x[r].sum_c *= XF_TINY_LIFT;
+    }
+    down = 1.0f / XF_TINY_LIFT;
+  }
+  while (row0 < end) {
 #pragma unroll
     for (int u = 0; u < LOADS; u++)
       if (lane + 64 * u < tile_pieces) tile[lane + 64 * u] = g.v[u];
@@ -563,7 +602,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
         const int blk = i * row_pieces + min(r * 8 + b, nb - 1) * 9;       // piece index of the block header
         uint4 hdr = tile[blk];
         hdr.x &= in_row[r];
-        acc[i] += slot_dot_f32(hdr, tile[blk + 1 + c], x[r], sel);
+        acc[i] += slot_dot_f32<true>(hdr, tile[blk + 1 + c], x[r], sel);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -571,38 +610,27 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_lds_kernel(
 #pragma unroll
     for (int i = 0; i < RPI; i++) {
       const float tot = wave_sum(acc[i]);
-      if (lane == 0 && row0 + i < N) y[row0 + i] = tot * unlift;
+      if (lane == 0 && row0 + i < N) y[row0 + i] = tot * down;
     }
     row0 += step;
   }
+  if (__builtin_expect(kind == 3, 0)) {
+    int l = lane;
+    asm("" : "+v"(l));      // (seen through, what this path derives from it stays in registers across the loop above)
+    const ScaleSel sl = make_scale_sel(l & 7);
+    for (; row0 < N; row0 += step)
+      for (int i = 0; i < RPI && row0 + i < N; i++) row_dot_f32(W, xf, y, row0 + i, nb, l, sl);
+  }
 }
 
-// Longer rows: rounds are a run-time loop, the activation slice is re-read (from L2) in every round.
+// Longer rows.
 __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_f32_generic_kernel(
     const uint8_t* __restrict__ W, const float* __restrict__ xf, float* __restrict__ y, int N, int nb) {
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * GEMV_WAVES + (threadIdx.x >> 6);
   const int nwaves = gridDim.x * GEMV_WAVES;
-  const int c = lane & 7;
-  const ScaleSel sel = make_scale_sel(c);
-  const int64_t row_bytes = (int64_t)nb * 144;
-  const int rounds = (nb + 7) / 8;
-  for (int row = wave; row < N; row += nwaves) {
-    const uint8_t* rp = W + (int64_t)row * row_bytes;
-    float acc = 0.0f;
-    for (int r = 0; r < rounds; r++) {
-      const int blk = r * 8 + (lane >> 3);
-      XF x[1];
-      load_xf(x[0], [&](int i) { return ((const float4*)xf)[i]; }, blk, c, blk < nb);
-      const float unlift = lift_tiny(x);
-      const int bo = (blk < nb ? blk : 0) * 144;
-      uint4 hdr = *(const uint4*)(rp + bo);
-      if (blk >= nb) hdr.x = 0;                             // past the row: d = dmin = 0
-      acc += slot_dot_f32(hdr, *(const uint4*)(rp + bo + 16 + 16 * c), x[0], sel) * unlift;
-    }
-    const float tot = wave_sum(acc);
-    if (lane == 0) y[row] = tot;
-  }
+  const ScaleSel sel = make_scale_sel(lane & 7);
+  for (int row = wave; row < N; row += nwaves) row_dot_f32(W, xf, y, row, nb, lane, sel);
 }
 
 template <int NR, int RPI>

@@ -416,3 +416,29 @@ def test_gemv_q4k_f32_activations_of_any_magnitude(orc, dev, N, K, exponent):
     want = ys[0].astype(np.float64) * 2.0**exponent
     assert np.isfinite(ys[1]).all() and (np.abs(ys[1].astype(np.float64) - want) <= 2.0**-150 * (1 if K <= 6144 else 64 * -(-K // 2048))).all()
     _assert_rel(ys[0], orc.gemv_q4k_f32(W, x, N, K, acc64=True))
+
+
+@pytest.mark.parametrize("loud,rest", [(0, -110), (0, -118), (0, -125), (97, -100), (98, -20), (110, -125)])
+@pytest.mark.parametrize("N,K", [(5, 256), (300, 1024), (1030, 2304), (2100, 2048), (9, 6144), (7, 6400)])
+def test_gemv_q4k_f32_small_activations_beside_a_large_one(orc, dev, N, K, loud, rest):
+    """One activation of 2^loud under weights of zero (all rows but the first) among activations of about 2^rest, on both sides of the line where activations
+    are no longer lifted: the small ones keep every bit of their products.  A term meets at most 33 roundings on its way (scale, a lane's sixteen FMAs or sums,
+    the joins of its lane, rounds and wave, and three in the checker's weight) of half a unit each, 2^-24 of the sum of magnitudes, and below the normal
+    range four per sixteen weights of 2^-150."""
+    print(f"gemv f32 loud N={N} K={K} 2^{loud} 2^{rest}", flush=True)
+    g = synth.rng(31 + N + K)
+    W = synth.q4k_random(g, N, K, 1.0)
+    quiet = W.reshape(N, K // 256, 144)[1:, K // 512]
+    quiet[:, 4] &= 0xc0      # scale and min of its first sub-block
+    quiet[:, 8] &= 0xc0
+    x = ((1 + g.random(K)) * g.choice([-1.0, 1.0], K) * 2.0**rest).astype(np.float32)
+    x[K // 512 * 256 + 5] = 2.0**loud
+    dy = dev.empty(N * 4)
+    rt.gemv_q4k_f32(dev.up(W), dev.up(x), dy, N, K)
+    y = rt.from_device(dy, (N,), np.float32).astype(np.float64)
+    parts = [W.copy(), W.copy()]      # the weights without their mins, and the mins alone
+    parts[0][:, 2:4] = 0
+    parts[1][:, 0:2] = 0
+    terms = sum(np.abs(orc.gemv_q4k_f32(p, np.abs(x), N, K, acc64=True).astype(np.float64)) for p in parts)
+    worst = np.abs(y - orc.gemv_q4k_f32(W, x, N, K, acc64=True)) / (33 * 2.0**-24 * terms + K / 4 * 2.0**-150)
+    assert worst.max() <= 1.0, worst.max()
