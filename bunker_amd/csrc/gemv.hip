@@ -128,10 +128,12 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_q4k_q8_1_lds_kernel(
 // Bound by the instructions of a round (about 70 for 64 slots) and the waves that the registers allow, no longer by idle lanes: 1.5 to 2 times the
 // rounds made K = 4608 with 67527 rows 43.9 us (4.0 TB/s), here 31.4 (5.6); K = 2560, 100000 rows 34.0 -> 26.1 (5.5 TB/s).  Without the activation row
 // through LDS, with a grid of two steps a wave and all of a step's operands in registers at once (a wave a SIMD less): 38.8 and 30.2.
-// Waves a SIMD that the registers allow (what a lane keeps for the slots is ten registers a round).
-constexpr int flat_waves(int S, int RPI) { return S <= 1 ? 8 : S == 2 ? 6 : S == 3 ? 5 : S <= 5 || RPI == 2 ? 4 : 3; }
+// Waves a SIMD that the registers allow (what a lane keeps for the slots is ten registers a round).  S = 6 with two rows takes 138: held to 128, for four
+// waves, it parked a piece of the next step's weights in scratch as it arrived, and a wave waited for it before it folded the step at hand
+// (5376 x 54000 39.4 us direct, 32.5 so, 29.1 with three waves).
+constexpr int flat_waves(int S) { return S <= 1 ? 8 : S == 2 ? 6 : S == 3 ? 5 : S <= 5 ? 4 : 3; }
 template <int S, int RPI, int EPI>
-__global__ __launch_bounds__(GEMV_WAVES * 64, flat_waves(S, RPI)) void gemv_q4k_q8_1_flat_kernel(
+__global__ __launch_bounds__(GEMV_WAVES * 64, flat_waves(S)) void gemv_q4k_q8_1_flat_kernel(
     const uint8_t* __restrict__ W, const uint8_t* __restrict__ xq_all, void* __restrict__ y,
     const uint16_t* __restrict__ res, int N, int nb) {
   constexpr int NB1 = 8 * S / RPI, NB0 = 8 * (S - 1) / RPI + 1;
@@ -314,7 +316,7 @@ static void launch_q8_1_lds(dim3 block, const uint8_t* w, const uint8_t* x, void
 // As many workgroups as the chip holds at once, with the steps dealt out evenly.
 template <int S, int RPI, int EPI>
 static void launch_q8_1_flat(const uint8_t* w, const uint8_t* x, void* y, const uint16_t* r, int N, int nb, int batch) {
-  const int64_t wgs = ((int64_t)N + GEMV_WAVES * RPI - 1) / (GEMV_WAVES * RPI), room = num_cus() * flat_waves(S, RPI);
+  const int64_t wgs = ((int64_t)N + GEMV_WAVES * RPI - 1) / (GEMV_WAVES * RPI), room = num_cus() * flat_waves(S);
   const int64_t steps = g_tune_steps > 0 ? g_tune_steps : (wgs * batch + room - 1) / room;
   hipLaunchKernelGGL((gemv_q4k_q8_1_flat_kernel<S, RPI, EPI>), dim3((unsigned)((wgs + steps - 1) / steps), batch), dim3(GEMV_WAVES * 64), 0, stream(), w, x, y, r, N, nb);
 }
@@ -325,7 +327,7 @@ static void launch_q8_1_flat(const uint8_t* w, const uint8_t* x, void* y, const 
 //   K = 1536: 33000 8.7 -> 8.9, 54000 11.5 -> 11.3, 100000 18.6 -> 16.9 (1792 saves no round and stays);  2304: 8000 6.5 -> 6.5, 13000 8.5 -> 7.9, 33000 14.6 -> 11.4, 100000 32.7 -> 25.1;
 //   K = 3072: 8000 6.9 -> 6.9, 10000 7.7 -> 7.9, 13000 9.1 -> 8.4, 54000 22.3 -> 18.7;  3584: 8000 7.3 -> 7.4, 10000 8.0 -> 8.7, 13000 9.8 -> 9.2, 86820 38.1 -> 31.4;
 //   K = 3840: 17000 11.7 -> 12.6, 26000 15.2 -> 16.2, 33000 17.9 -> 16.7, 81032 36.6 -> 31.3;  4608: 4000 7.3 -> 6.1, 8000 8.7 -> 8.7, 13000 12.1 -> 10.9, 67527 43.9 -> 31.4;
-//   K = 5120: 13000 12.6 -> 11.1, 60774 40.2 -> 30.3;  5888: 4000 8.1 -> 7.05, 8000 9.0 -> 9.85, 13000 13.5 -> 12.6, 54000 40.3 -> 31.2.
+//   K = 5120: 13000 12.6 -> 11.1, 60774 40.2 -> 30.3;  5888: 1500 7.0 -> 4.95, 4000 8.25 -> 6.9, 8000 9.45 -> 8.9, 13000 13.35 -> 12.8, 54000 41.3 -> 31.0.
 static int gemv_flat_rounds(int nb, int N, int batch) {
   if (nb % 8 == 0 || nb == 7 || nb > 23) return 0;
   const int rpi = nb < 16 ? 4 : 2, S = (rpi * nb + 7) / 8;
@@ -334,7 +336,7 @@ static int gemv_flat_rounds(int nb, int N, int batch) {
   if (S == 1) pays = wgs > 5 * cus;
   else if (S == 2) pays = wgs > 6 * cus;
   else if (S == 3) pays = wgs > 15 * cus;
-  else if (S == 6) pays = wgs <= 2 * cus || wgs > flat_waves(S, rpi) * cus;
+  else if (S == 6 && rpi == 4) pays = wgs <= 2 * cus || wgs > flat_waves(S) * cus;
   else if (S == 7) pays = wgs > 3 * cus;
   else if (S == 8) pays = wgs > 7 * cus;
   return pays || g_tune_gemv_impl == 3 ? 10 * S + rpi : 0;

@@ -237,3 +237,15 @@ def test_results_of_the_tiles_matmul_are_first_read_where_the_compiler_sees_it(t
                     break
                 assert not (writes and _registers(x[1]) & results), (name, first, x)
         assert checked >= 2 * 32, (name, checked)
+
+
+def test_the_numbered_rows_gemv_fits_the_registers_of_its_waves(tmp_path_factory):
+    """gemv.hip: every form of the flat kernel and of the f32 kernel without scratch.  A spilled piece of the next step's weights is waited for before
+    the step at hand is folded."""
+    asm = _compile_to_asm(tmp_path_factory, "gemv.hip")
+    names = [n for n in _kernels(asm) if "gemv_q4k_q8_1_flat_kernel" in n or "gemv_q4k_f32_lds_kernel" in n]
+    assert len(names) == 9 * 3 + 4
+    for name in names:
+        meta = re.search(r"\.name:\s+%s\n(.*?)\.wavefront_size" % re.escape(name), asm, flags=re.S).group(1)
+        assert int(re.search(r"\.vgpr_spill_count:\s+(\d+)", meta).group(1)) == 0, name
+        assert int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", meta).group(1)) == 0, name
