@@ -28,7 +28,8 @@ def _activations(orc, g, B, K):
 
 
 @pytest.mark.parametrize("form", ["plain", "large", "shifted", "gap", "mixed", "negative", "infinite"])
-@pytest.mark.parametrize("N,K,B", [(1, 256, 8), (33, 768, 33), (64, 512, 64), (97, 256, 65), (31, 1280, 31), (130, 512, 130)])
+@pytest.mark.parametrize("N,K,B", [(1, 256, 8), (33, 768, 33), (64, 512, 64), (97, 256, 65), (31, 1280, 31), (130, 512, 130),
+                                   (163, 2048, 131), (33, 4096, 70), (97, 6144, 65)])
 def test_outputs_equal_the_host_loop(orc, N, K, B, form):
     print(f"matmul tiles {form} N={N} K={K} B={B}", flush=True)
     g = synth.rng(4200 + N + K + B)
@@ -102,7 +103,7 @@ def test_four_matrices_in_one_launch_with_every_epilogue(orc, B):
             assert v.any() and np.array_equal(u, v)
 
 
-@pytest.mark.parametrize("N,K,B,offset", [(32, 256, 9, 0), (96, 512, 33, 2), (160, 1024, 70, 0), (64, 768, 64, 8), (32, 512, 129, 0)])
+@pytest.mark.parametrize("N,K,B,offset", [(32, 256, 9, 0), (96, 512, 33, 2), (160, 1024, 70, 0), (64, 768, 64, 8), (32, 512, 129, 0), (160, 2048, 131, 0), (64, 6144, 33, 2)])
 def test_swiglu_blocks(orc, N, K, B, offset):
     print(f"swiglu tiles N={N} K={K} B={B} offset={offset}", flush=True)
     g = synth.rng(500 + N + B)
@@ -126,7 +127,7 @@ def test_swiglu_blocks(orc, N, K, B, offset):
         assert np.array_equal(gq[b], orc.pack_q8_1((ref.astype(np.uint32) << 16).view(np.float32))), b
 
 
-@pytest.mark.parametrize("N,K,B", [(3072, 512, 1024), (8240, 256, 1000)])
+@pytest.mark.parametrize("N,K,B", [(3072, 512, 1024), (8240, 256, 1000), (4063, 6144, 1000), (6113, 2048, 1023)])
 def test_large_launches_choose_it_and_return_the_same_bits(orc, N, K, B):
     print(f"matmul tiles by shape N={N} K={K} B={B}", flush=True)
     g = synth.rng(N + B)
