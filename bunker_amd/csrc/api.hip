@@ -566,7 +566,7 @@ using namespace bk;
 
 extern "C" {
 
-// Tuning hooks for measurements: "gemv_impl" (0 direct loads, 2 rows through LDS), "gemv_rpi" (rows per wave step),
+// Tuning hooks for measurements: "gemv_impl" (0 direct loads, 2 from the shape, 3 rows numbered through where that form exists), "gemv_rpi" (rows per wave step),
 // "gemv_cap" (workgroups per CU), "gemm_nw" (waves per MFMA tile), "memread_*" (calibration read kernel).
 int bk_tune_set(const char* key, int value) {
   BK_REQUIRE(key, "bk_tune_set: null key");

@@ -257,8 +257,8 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 || TR < 32 ? 1 
     // sum in two halves (rounded once): below 128 (values below 16256) d8_j * 2^24 still fits 31 bits, above that the fold
     // takes d8_j * 2^(24 - s) as long as these are whole numbers, which scales of 2^(s - 14) and more are.  What is left (non-finite
     // scales, and one of 2^(7 + s) beside one below 2^(s - 14)) is folded in double, one sub-block after the other.  us for
-    // 77 rows x 12288 x 2048 and for gate + up of 1024 x 6144 x 2048, every unit of a kind: scales below 4 24.0 and 171, up to 128 24.9
-    // and 172, above 26.1 and 179, non-finite 30.4 and 221; everything in double, pipelined over the sub-blocks: 25.3 and 184.  (That
+    // 77 rows x 12288 x 2048 and for gate + up of 1024 x 6144 x 2048, every unit of a kind: scales below 4 24.0 and 154, up to 128 24.9
+    // and 163, above 26.1 and 179, non-finite 30.4 and 217; everything in double, pipelined over the sub-blocks: 25.3 and 184.  (That
     // form beside this one takes more than the 256 registers of two waves a SIMD.)
     double S1[RF];
     auto fold = [&](auto small_scales, const unsigned char* mW, const unsigned char* mX, const unsigned char* mS, int s) __attribute__((always_inline)) {
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(64 * NW * (SWIGLU ? 2 : 1), NW == 1 || TR < 32 ? 1 
     // Prompts: a thread takes eight consecutive weight rows of one batch row, four neighbouring lanes a Q8_1 block, so that the
     // block's maximum, scale and sum are formed once per eight values and the lanes' eight sigmoids are independent.  (With a
     // value per lane and the block across 32 lanes, every value paid for them: this step was 27 of 169 us at 1024 rows x
-    // 2 x 6144 x 2048.)  With this form 155 us.
+    // 2 x 6144 x 2048.)  With this form 154 us.
     const int g8 = lane & 3, b = 16 * wave + (lane >> 2);
     float f[8];
     uint32_t a2[4];

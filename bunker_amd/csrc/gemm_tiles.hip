@@ -10,12 +10,12 @@
 // One set of accumulators: the tile is four 16 x 16 products.  v_mfma_i32_16x16x32_i8 leaves row 4 q + v of its tile in register v of lanes 16 q..,
 // v_mfma_f64_16x16x4_f64 row 4 v + q; the weight rows of the first are handed over in the order (4 (i % 4) + i / 4) that makes the two agree, and
 // the min term is added to the sums of the fold where they are.  (The 32 x 32 form takes half the matrix time, but its rows
-// cannot be made to agree.  With it, 227 registers and two waves a SIMD: 1024 rows x 12288 x 2048 137 us, this 123; the lone waves of gemm_mfma.hip 149.)
+// cannot be made to agree.  With it, 227 registers and two waves a SIMD: 1024 rows x 12288 x 2048 137 us where this took 123.)
 //
 // What bounds it: vector issue and the matrix unit together.  A unit (32 x 32 x 256) is 1900 cycles of vector instructions (1024 of them the fold: a
 // multiply and a 64-bit multiply-add per dot), 512 of the f64 matrix instruction, which runs on the vector unit, and 512 of the int8 one,
 // of which about 300 hide behind the others: 2600 of the 2900 that pass.  us, gemm_mfma.hip -> here, 1024 rows:
-//   12288 x 2048: 142 -> 122; 6144 x 2048: 74.2 -> 63.8; 2048 x 6144: 74.0 -> 73.1; gate + up 2 x 6144 x 2048 with SwiGLU: 155 -> 125.
+//   12288 x 2048: 139 -> 120; 6144 x 2048: 73.1 -> 64.2; 4096 x 6144: 135 -> 127; gate + up 2 x 6144 x 2048 with SwiGLU: 154 -> 126.
 #include "ops.h"
 #include <algorithm>
 #include <type_traits>
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256, 3) void gemm_q4k_q8_1_tiles_kernel(TileArgs A)
 #define GT_SB __builtin_amdgcn_sched_barrier(0)
 
   // One super-block from LDS.  The fold, its ranges of scales and its forms for large ones are those of gemm_mfma.hip.  us for gate + up of 1024 x 6144 x 2048,
-  // every unit of a kind: scales below 4 141 (there 174), up to 128 146 (182), above 174 (182), non-finite 204 (220).
+  // every unit of a kind: scales below 4 126 (there 154), up to 128 132 (163), above 174 (179), non-finite 201 (217).
   auto compute = [&]() __attribute__((always_inline)) {
     const int4 fl = *(const int4*)(lds + GT_FLAG);
     f64x4_t S1[2][2];
@@ -388,11 +388,14 @@ int g_tune_gemm_tiles = -1;      // 0: never, 1: always, -1: from the shape
 
 // Where this kernel is the faster one.  Its time goes by the workgroups per CU, rounded up (three run at a time); that of gemm_mfma.hip by tiles per CU,
 // finer by four (by two with SwiGLU).  us at K = 1024 / 2048 / 6144, gemm_mfma.hip -> here, by workgroups per CU with every tile in use:
-//   one (1024 x 1024 rows): 11.3 -> 12.1, 16.9 -> 19.6, 40.5 -> 51.8; two (2048): 18.2 -> 16.5, 29.1 -> 27.2, 74.0 -> 73.1;
-//   three (3072): 24.9 -> 21.4, 41.1 -> 36.0, 107 -> 95.7; four (4096): 30.8 -> 26.7, 52.1 -> 46.3, 138 -> 126; six (6144): 44.2 -> 36.5, 74.2 -> 63.8, 201 -> 178;
+//   one (1024 x 1024 rows): 11.3 -> 12.1, 16.9 -> 19.6, 40.5 -> 51.8; two (2048): 17.4 -> 16.0, 28.2 -> 27.4, 71.0 -> 72.3 (K = 3072 43.2 -> 43.0, 4096 53.8 -> 54.1);
+//   three (3072): 24.9 -> 21.4, 41.1 -> 36.0, 107 -> 95.7; four (4096): 30.8 -> 26.7, 52.1 -> 46.3, 135 -> 127; six (6144): 44.2 -> 36.5, 73.1 -> 64.2, 201 -> 178;
 // in microseconds at K = 2048, 3.0 per tile and CU + 5 there against 9.3 per workgroup + 8.5 here: tiles left over from an odd
 // number of either side (12288 at 160 rows: 8 tiles, 3 workgroups a CU: 29.4 -> 34.6) must leave 4 tiles > 13 workgroups + 4.
-// SwiGLU, pairs of tiles: two (1024): 19.6 -> 17.5, 30.4 -> 28.4, 75.7 -> 74.8; three (1536): 33.0 -> 22.8, 48.8 -> 37.6, 116 -> 99.0; four (2048): 36.3 -> 28.9, 60.6 -> 48.6, 161 -> 128;
+// (Long rows on two workgroups, and on seven with 24 tiles (5952 at 1056 rows, K = 2048 / 4096 / 6144: 83.6 -> 82.3, 146 -> 148, 210 -> 215), are 1 to 3 % slower
+// here by themselves.  In prompts, whose chunks overlap on two streams, it goes either way: with two workgroups left to gemm_mfma.hip above K = 4096, 2999 tokens in
+// the forms for throughput take 5.54 ms instead of 5.48, 2048 tokens in the default ones 24.9 instead of 25.2.)
+// SwiGLU, pairs of tiles: two (1024): 18.6 -> 16.9, 29.4 -> 28.5, 71.8 -> 73.3 (K = 4096 51.1 -> 51.1); three (1536): 33.0 -> 22.8, 48.8 -> 37.6, 116 -> 99.0; four (2048): 36.3 -> 28.9, 60.6 -> 48.6, 161 -> 128;
 // seven (3584): 58.1 -> 44.1, 97.5 -> 77.6, 256 -> 209; three pairs on two workgroups 18.5 -> 17.3, 28.6 -> 28.0, 60.4 -> 71.3 (left to gemm_mfma.hip),
 // four on three (6144 at 160 rows) 20.2 -> 22.4, 31.0 -> 36.9, 74.5 -> 93.5, seven on four (3584 at 512) 34.8 -> 29.3, 54.9 -> 48.0, 139 -> 127.
 bool gemm_tiles_pay(int tiles, int batch, int nb, bool swiglu) {

@@ -80,7 +80,7 @@ BK_API int bk_prof_report(char* buf, int cap);       /* profGpuReport, src/ttir.
  * crashes (LOG.md:710-738); here the graph lives behind scalar handles.
  * Between begin and end only launches are legal: alloc, free, memset, copies,
  * sync, event waits, a stream switch, a graph launch, bk_kernel_create and
- * bk_kernel_destroy (they allocate, clear and free a handle's workspace) return
+ * bk_kernel_destroy (they allocate and free a handle's workspace) return
  * an error (state -3, "not legal between bk_capture_begin and bk_capture_end")
  * and leave the capture open. */
 BK_API int bk_capture_begin(void);
@@ -94,7 +94,7 @@ BK_API int bk_graph_node_count(uint64_t graph, int* count);
 /* Launch-shape knobs for experiments and tests; the defaults (0, or -1 = chosen from the shape) are the tuned values:
  * "gemv_rpi", "gemv_cap", "gemv_steps", "gemv_impl", "fused_cap" (GEMV rows per wave step, workgroups per CU up to
  * which a wave takes one step, row steps per wave, kernel variant: 0 = direct loads, 2 = from the shape, 3 = several rows'
- * super-blocks numbered through wherever K is no multiple of 2048),
+ * super-blocks numbered through for every K below 6144 that is no multiple of 2048, 1792 aside),
  * "gemm_tiles" (workgroups of 64 x 64 outputs: 1 = always, 0 = never, -1 = from the shape; "gemm_nw" comes first), "gemm_nw" (waves per matmul tile: 1, 2, 4, 8), "gemm_r16" (narrow matmul tiles: 1 = 16 weight rows, 2 = 8), "small_rows" (0: the two 16-row
  * matrices of a batched projection group stay in the matmul instead of the norm's launch), "rows" (products of 2 to 7
  * sequences in one pass over the weights: 0 = never, 1 = where it is the faster form, the default, 2 = wherever there is a
