@@ -480,32 +480,31 @@ __device__ __forceinline__ float slot_dot_f32(const uint4& hdr, const uint4& q, 
   return (f0 * a + f1 * b) - fm;
 }
 
-// One row of any length and any activations, by one wave: rounds are a run-time loop, the activation slice is re-read (from L2) in every round.
+// One row of any length and any activations, by one wave: rounds are a run-time loop, the activation slice is re-read (from L2) in every round, so that
+// lifting it (32 multiplications for one use) costs more than converting the nibbles (16 instructions): 4096 x 8192 11.4 -> 11.15 us, 2048 x 12288 9.75 -> 9.35.
 __device__ __forceinline__ void row_dot_f32(const uint8_t* W, const float* xf, float* y, int row, int nb, int lane, const ScaleSel& sel) {
   const uint8_t* rp = W + (int64_t)row * nb * 144;
   const int c = lane & 7, rounds = (nb + 7) / 8;
   float acc = 0.0f;
-#pragma unroll 1
   for (int r = 0; r < rounds; r++) {
     const int blk = r * 8 + (lane >> 3);
     XF x;
     load_xf<false>(x, [&](int i) { return ((const float4*)xf)[i]; }, blk, c, blk < nb);
+    const int bo = (blk < nb ? blk : 0) * 144;
+    uint4 hdr = *(const uint4*)(rp + bo);
+    const uint4 q = *(const uint4*)(rp + bo + 16 + 16 * c);
+    if (blk >= nb) hdr.x = 0;                             // past the row: d = dmin = 0
     float top = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; i++) top = fmaxf(fmaxf(top, fabsf(x.lo[i])), fabsf(x.hi[i]));
-    const int bo = (blk < nb ? blk : 0) * 144;
-    uint4 hdr = *(const uint4*)(rp + bo);
-    if (blk >= nb) hdr.x = 0;                             // past the row: d = dmin = 0
-    const uint4 q = *(const uint4*)(rp + bo + 16 + 16 * c);
-    if (__builtin_expect(__any(top >= XF_LIFT_BELOW), 0)) {
-      acc += slot_dot_f32<false>(hdr, q, x, sel);
-    } else {
-      const float up = __any(top >= XF_TINY) ? 1.0f : XF_TINY_LIFT;
+    float down = 1.0f;
+    if (__builtin_expect(!__any(top >= XF_TINY), 0)) {
 #pragma unroll
-      for (int i = 0; i < 16; i++) { x.lo[i] *= XF_LIFT * up; x.hi[i] *= XF_LIFT * up; }
-      x.sum_c *= up;
-      acc += slot_dot_f32<true>(hdr, q, x, sel) * (1.0f / up);
+      for (int i = 0; i < 16; i++) { x.lo[i] *= XF_TINY_LIFT; x.hi[i] *= XF_TINY_LIFT; }
+      x.sum_c *= XF_TINY_LIFT;
+      down = 1.0f / XF_TINY_LIFT;
     }
+    acc += slot_dot_f32<false>(hdr, q, x, sel) * down;
   }
   const float tot = wave_sum(acc);
   if (lane == 0) y[row] = tot;
